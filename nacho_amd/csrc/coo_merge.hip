@@ -668,7 +668,8 @@ int coo2_rows(const nacho_coo *a, const nacho_coo *b, nacho_coo *z, void *stream
     const csr::LevelOperand B{pb, b->dim_j_indices, b->values, nnz_b, nullptr};
     const csr::LevelResult Z{pz, zj, zv, nullptr, nullptr, zi};
     long long nnz = 0;
-    NACHO_TRY(csr::merge_level(call, OP == Op::Intersect, true, false, rows, A, B, Z, &nnz, name));
+    NACHO_TRY(csr::merge_level(call, OP == Op::Intersect, true, false, rows,
+                               csr::extent_bits(a->dim_j_size), A, B, Z, &nnz, name));
     if (nnz > cap) return NACHO_ERR_MALFORMED_INPUT;
     if (nnz == 0) {
         call.drop_result(zi);
@@ -789,7 +790,8 @@ int coo3_rows(const nacho_coo3 *a, const nacho_coo3 *b, nacho_coo3 *z, void *str
     const csr::LevelOperand B{pb, kb, b->values, nnz_b, nullptr};
     const csr::LevelResult Z{pz, zj, zv, nullptr, nullptr, zi, zk, kbits};
     long long nnz = 0;
-    NACHO_TRY(csr::merge_level(call, false, true, false, rows, A, B, Z, &nnz, name));
+    NACHO_TRY(csr::merge_level(call, false, true, false, rows,
+                               bits_for_extent(a->dim_j_size) + kbits, A, B, Z, &nnz, name));
     if (nnz > cap) return NACHO_ERR_MALFORMED_INPUT;
     if (nnz == 0) {
         call.drop_result(zi);
@@ -874,7 +876,8 @@ int coo_csr_add(const nacho_csr *a, const nacho_coo *b, nacho_csr *z, int32_t nb
     const csr::LevelOperand B{pb, b->dim_j_indices, b->values, b->nnz, nullptr};
     const csr::LevelResult Z{pc, cc, vc, nullptr, nullptr};
     long long nnz = 0;
-    NACHO_TRY(csr::merge_level(call, false, true, false, rows, A, B, Z, &nnz, "coo_csr_add"));
+    NACHO_TRY(csr::merge_level(call, false, true, false, rows, csr::extent_bits(a->dim_j_size), A, B,
+                               Z, &nnz, "coo_csr_add"));
     if (nnz > cap) return NACHO_ERR_MALFORMED_INPUT;
     if (nnz == 0) {
         call.drop_result(cc);
@@ -953,7 +956,8 @@ int coo3_inner_prod(const nacho_coo3 *a, const nacho_coo3 *b, nacho_scalar *z, i
         csr::LevelResult Z{nullptr, nullptr, nullptr, nullptr, nullptr};
         Z.dot = value;
         long long unused = 0;
-        NACHO_TRY(csr::merge_level(call, true, true, false, rows, A, B, Z, &unused,
+        NACHO_TRY(csr::merge_level(call, true, true, false, rows,
+                                   bits_for_extent(a->dim_j_size) + kbits, A, B, Z, &unused,
                                    "inner_prod_coo"));
         z->values = value;
         z->nnz = 1;

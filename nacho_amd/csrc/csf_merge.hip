@@ -88,7 +88,8 @@ int csf_add(const nacho_csf3 *a, const nacho_csf3 *b, nacho_csf3 *z, int32_t num
         const csr::LevelOperand B{root + 2, b->dim_i_indices, nullptr, b->dim_i_length,
                                   b->dim_j_offsets};
         const csr::LevelResult Z{root_out, crd_i, nullptr, ci_a, ci_b};
-        NACHO_TRY(csr::merge_level(call, false, false, true, 1, A, B, Z, &ni, "csf_add"));
+        NACHO_TRY(csr::merge_level(call, false, false, true, 1,
+                                   csr::extent_bits(a->dim_i_size), A, B, Z, &ni, "csf_add"));
     }
 
     // j level: rows = output i fibres
@@ -102,7 +103,8 @@ int csf_add(const nacho_csf3 *a, const nacho_csf3 *b, nacho_csf3 *z, int32_t num
         const csr::LevelOperand A{ci_a, a->dim_j_indices, nullptr, a->dim_j_length, a->dim_k_offsets};
         const csr::LevelOperand B{ci_b, b->dim_j_indices, nullptr, b->dim_j_length, b->dim_k_offsets};
         const csr::LevelResult Z{pos_j, crd_j, nullptr, cj_a, cj_b};
-        NACHO_TRY(csr::merge_level(call, false, false, true, static_cast<int>(ni), A, B, Z, &nj,
+        NACHO_TRY(csr::merge_level(call, false, false, true, static_cast<int>(ni),
+                                   csr::extent_bits(a->dim_j_size), A, B, Z, &nj,
                                    "csf_add"));
     }
 
@@ -117,7 +119,8 @@ int csf_add(const nacho_csf3 *a, const nacho_csf3 *b, nacho_csf3 *z, int32_t num
         const csr::LevelOperand A{cj_a, a->dim_k_indices, a->values, a->dim_k_length, nullptr};
         const csr::LevelOperand B{cj_b, b->dim_k_indices, b->values, b->dim_k_length, nullptr};
         const csr::LevelResult Z{pos_k, crd_k, val, nullptr, nullptr};
-        NACHO_TRY(csr::merge_level(call, false, true, false, static_cast<int>(nj), A, B, Z, &nk,
+        NACHO_TRY(csr::merge_level(call, false, true, false, static_cast<int>(nj),
+                                   csr::extent_bits(a->dim_k_size), A, B, Z, &nk,
                                    "csf_add"));
     }
     if (ni > cap_i || nj > cap_j || nk > cap_k) return NACHO_ERR_MALFORMED_INPUT;
@@ -337,7 +340,8 @@ int csf_inner_prod(const nacho_csf3 *a, const nacho_csf3 *b, nacho_scalar *z, in
         csr::LevelResult Z{nullptr, nullptr, nullptr, nullptr, nullptr};
         Z.dot = value;
         long long unused = 0;
-        NACHO_TRY(csr::merge_level(call, true, true, false, rows, A, B, Z, &unused,
+        NACHO_TRY(csr::merge_level(call, true, true, false, rows,
+                                   std::max(extent_bits(a->dim_j_size) + kbits, 1), A, B, Z, &unused,
                                    "inner_prod"));
         z->values = value;
         z->nnz = 1;
@@ -360,7 +364,8 @@ int csf_inner_prod(const nacho_csf3 *a, const nacho_csf3 *b, nacho_scalar *z, in
         const csr::LevelOperand B{root + 2, b->dim_i_indices, nullptr, b->dim_i_length,
                                   b->dim_j_offsets};
         const csr::LevelResult Z{root_out, crd_i, nullptr, ci_a, ci_b};
-        NACHO_TRY(csr::merge_level(call, false, false, true, 1, A, B, Z, &ni, "inner_prod"));
+        NACHO_TRY(csr::merge_level(call, false, false, true, 1,
+                                   csr::extent_bits(a->dim_i_size), A, B, Z, &ni, "inner_prod"));
     }
     if (ni > cap_i) return NACHO_ERR_MALFORMED_INPUT;
 
@@ -375,7 +380,8 @@ int csf_inner_prod(const nacho_csf3 *a, const nacho_csf3 *b, nacho_scalar *z, in
         const csr::LevelOperand A{ci_a, a->dim_j_indices, nullptr, a->dim_j_length, a->dim_k_offsets};
         const csr::LevelOperand B{ci_b, b->dim_j_indices, nullptr, b->dim_j_length, b->dim_k_offsets};
         const csr::LevelResult Z{pos_j, crd_j, nullptr, cj_a, cj_b};
-        NACHO_TRY(csr::merge_level(call, false, false, true, static_cast<int>(ni), A, B, Z, &nj,
+        NACHO_TRY(csr::merge_level(call, false, false, true, static_cast<int>(ni),
+                                   csr::extent_bits(a->dim_j_size), A, B, Z, &nj,
                                    "inner_prod"));
     }
     if (nj > cap_j) return NACHO_ERR_MALFORMED_INPUT;
@@ -387,7 +393,8 @@ int csf_inner_prod(const nacho_csf3 *a, const nacho_csf3 *b, nacho_scalar *z, in
         csr::LevelResult Z{nullptr, nullptr, nullptr, nullptr, nullptr};
         Z.dot = value;
         long long unused = 0;
-        NACHO_TRY(csr::merge_level(call, true, true, false, static_cast<int>(nj), A, B, Z,
+        NACHO_TRY(csr::merge_level(call, true, true, false, static_cast<int>(nj),
+                                   csr::extent_bits(a->dim_k_size), A, B, Z,
                                    &unused, "inner_prod"));
     }
     z->values = value;

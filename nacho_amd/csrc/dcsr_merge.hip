@@ -138,7 +138,8 @@ int dcsr_binary(bool intersect, const nacho_dcsr *a, const nacho_dcsr *b, nacho_
         const csr::LevelOperand B{root + 2, b->dim_i_indices, nullptr, b->dim_i_length,
                                   intersect ? nullptr : b->dim_j_offsets};
         const csr::LevelResult Z{root_out, crd_u, nullptr, ci_a, ci_b};
-        NACHO_TRY(csr::merge_level(call, false, false, true, 1, A, B, Z, &nu, name));
+        NACHO_TRY(csr::merge_level(call, false, false, true, 1,
+                                   csr::extent_bits(a->dim_i_size), A, B, Z, &nu, name));
     }
     if (nu > cap_i) return NACHO_ERR_MALFORMED_INPUT;
 
@@ -188,8 +189,8 @@ int dcsr_binary(bool intersect, const nacho_dcsr *a, const nacho_dcsr *b, nacho_
         const csr::LevelOperand A{ja, a->dim_j_indices, a->values, a->dim_j_length, nullptr};
         const csr::LevelOperand B{jb, b->dim_j_indices, b->values, b->dim_j_length, nullptr};
         const csr::LevelResult Z{pos_u, crd_j, val, nullptr, nullptr};
-        NACHO_TRY(csr::merge_level(call, intersect, true, false, static_cast<int>(nu), A, B, Z,
-                                   &nj, name, csr::UnionCount::kAuto,
+        NACHO_TRY(csr::merge_level(call, intersect, true, false, static_cast<int>(nu),
+                                   csr::extent_bits(a->dim_j_size), A, B, Z, &nj, name,
                                    intersect ? &nj_pending : nullptr));
     }
 

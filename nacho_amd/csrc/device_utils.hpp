@@ -43,6 +43,19 @@ __device__ __forceinline__ int wave_inclusive_max_dpp(int v) {
     return v;
 }
 
+// The same running maximum for unsigned values: 0 is the identity of the unsigned maximum, so
+// each step is one DPP instruction.
+__device__ __forceinline__ unsigned wave_inclusive_umax_dpp(unsigned v) {
+    auto step = [](unsigned x, int y) { return max(x, static_cast<unsigned>(y)); };
+    v = step(v, __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x111, 0xf, 0xf, true));
+    v = step(v, __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x112, 0xf, 0xf, true));
+    v = step(v, __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x114, 0xf, 0xf, true));
+    v = step(v, __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x118, 0xf, 0xf, true));
+    v = step(v, __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xa, 0xf, false));
+    v = step(v, __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xc, 0xf, false));
+    return v;
+}
+
 // Inclusive prefix sum over the 64 lanes of a wavefront (DPP for 32-bit integers, lane
 // shuffles otherwise).
 template <typename T>

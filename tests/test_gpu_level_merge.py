@@ -1,0 +1,110 @@
+"""The level merge at its limits: tile and wavefront boundaries, 32- and 64-bit merge keys,
+sparse tiles (searched) beside dense ones (sorted), empty operands.
+
+Bar: pos / i, crd and values bit-exact against the numpy closed forms, for csr_add / csr_mul
+and, through the same levels with output rows, coo_add / coo_mul.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle
+from tests.helpers import assert_csr_equal, csr_from_rows
+
+pytestmark = pytest.mark.gpu
+
+
+def _distinct(rng, n, cols):
+    """n distinct sorted columns below cols, the last column always among them."""
+    c = np.unique(rng.integers(0, cols, size=2 * n + 8))
+    c = rng.permutation(c)[: max(n - 1, 0)]
+    return np.unique(np.append(c, cols - 1))[-n:] if n else c[:0]
+
+
+def _partner(rng, c, n, cols):
+    """n columns, about half of them out of c."""
+    kept = rng.permutation(c)[: n // 2]
+    return np.unique(np.append(kept, _distinct(rng, n - len(kept), cols)))
+
+
+def _case(name):
+    rng = np.random.default_rng(7)
+    kind, _, arg = name.partition(":")
+    if kind == "edge":  # one long row of about half a tile's entries per operand
+        n = int(arg)
+        c = np.arange(2 * n)
+        return 2 * n, [c[::2], c[:0]], [_partner(rng, c[::2], n, 2 * n), c[:3]]
+    if kind == "identical":  # pairs across every wavefront boundary, at both parities
+        n = int(arg)
+        c = np.arange(n)
+        return n, [c[:1], c], [c[:0], c]
+    if kind == "cols":  # many nearly empty rows beside a long one: the key's row bits
+        cols = int(arg)
+        a = [_distinct(rng, int(rng.integers(0, 2)), cols) for _ in range(3000)]
+        b = [_partner(rng, x, int(rng.integers(0, 2)), cols) for x in a]
+        a[1500], b[1500] = _distinct(rng, 900, cols), _distinct(rng, 1100, cols)
+        return cols, a, b
+    if kind == "few":  # long rows of one operand, `arg` entries of the other in each
+        n, cols = int(arg), 1 << 20
+        long = [_distinct(rng, 2000, cols) for _ in range(6)]
+        short = [_partner(rng, x, n, cols) for x in long]
+        a = [long[0], short[1], long[2], [], short[4], long[5]]
+        b = [short[0], long[1], short[2], long[3], long[4], []]
+        return cols, a, b
+    if kind == "gap":  # a tile with more rows than the sparse path takes
+        cols, n = 5000, int(arg)
+        a = [_distinct(rng, 2500, cols)] + [[]] * n + [_distinct(rng, 2500, cols)]
+        b = [[7]] + [[]] * n + [_distinct(rng, 3, cols)]
+        return cols, a, b
+    raise AssertionError(name)
+
+
+CASES = (["edge:%d" % n for n in (1, 2015, 2016, 2017, 4031, 4033)] +
+         ["identical:%d" % n for n in (1024, 1025, 4031, 9000)] +
+         ["cols:%d" % n for n in (1 << 19, (1 << 19) + 1, 1 << 20, 2**31 - 1)] +
+         ["few:%d" % n for n in (1, 60, 127, 128, 129, 300)] +
+         ["gap:%d" % n for n in (500, 511, 4100)])
+
+
+@pytest.mark.parametrize("name", CASES)
+@pytest.mark.parametrize("op", ["add", "mul"])
+def test_level_limits(gpu, op, name):
+    import nacho_amd
+
+    cols, ra, rb = _case(name)
+    rows = len(ra)
+    a, b = csr_from_rows(rows, cols, ra), csr_from_rows(rows, cols, rb)
+    print(f"[gpu] level merge {op} {name} rows={rows} cols={cols}", flush=True)
+    shape = torch.tensor([rows, cols], dtype=torch.int32)
+
+    def dev(x):
+        return torch.from_numpy(np.ascontiguousarray(x)).to(gpu)
+
+    want = oracle.closed_csr_binary(op, rows, cols, *a, *b)
+    z = getattr(nacho_amd, f"gpu_csr_{op}_f32")(
+        *(nacho_amd.CSR_gpu(*(dev(x) for x in t), shape) for t in (a, b)))
+    got = tuple(x.cpu().numpy() for x in (z.dim_j_offsets, z.dim_j_indices, z.values))
+    assert_csr_equal(got, want, name)
+    row_of = [np.repeat(np.arange(rows, dtype=np.int32), np.diff(t[0])) for t in (a, b, want)]
+    z = getattr(nacho_amd, f"gpu_coo_{op}_f32")(
+        *(nacho_amd.COO_gpu(dev(i), dev(t[1]), dev(t[2]), shape)
+          for i, t in zip(row_of, (a, b))))
+    assert np.array_equal(z.dim_i_indices.cpu().numpy(), row_of[2])
+    assert np.array_equal(z.dim_j_indices.cpu().numpy(), want[1])
+    assert np.array_equal(z.values.cpu().numpy().view(np.uint32), want[2].view(np.uint32))
+
+
+@pytest.mark.parametrize("op", ["add", "mul"])
+@pytest.mark.parametrize("empty", ["a", "b", "both"])
+def test_empty_operand(gpu, op, empty):
+    import nacho_amd
+
+    c = np.arange(5000)
+    full, none = csr_from_rows(2, 5000, [c, c[::3]]), csr_from_rows(2, 5000, [[], []])
+    a, b = (none if empty in ("a", "both") else full), (none if empty in ("b", "both") else full)
+    shape = torch.tensor([2, 5000], dtype=torch.int32)
+    z = getattr(nacho_amd, f"gpu_csr_{op}_f32")(
+        *(nacho_amd.CSR_gpu(*(torch.from_numpy(x).to(gpu) for x in t), shape) for t in (a, b)))
+    got = tuple(x.cpu().numpy() for x in (z.dim_j_offsets, z.dim_j_indices, z.values))
+    assert_csr_equal(got, oracle.closed_csr_binary(op, 2, 5000, *a, *b), empty)
