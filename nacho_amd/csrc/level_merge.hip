@@ -61,6 +61,10 @@ static_assert(kWords == dev::kWave, "one order word per lane");
 // Tiles per pair total: a wavefront of the emit kernel sums the chunks before its tile's and
 // the tiles before it in its own chunk (at most 2^31 / kTile / kChunk + kChunk loads).
 constexpr int kChunk = 256;
+// Levels of at most this many tiles take one launch (fused_kernel): one per CU.  Per call, one
+// launch against three: 4 tiles 28.7 / 30.6 us, 42 tiles 29.0 / 34.0, 253 tiles 30.8 / 35.3, but
+// 421 tiles 34.9 / 34.0 (csr_add, 8 entries per row and operand).
+constexpr int kFusedTiles = 256;
 // 32-bit words between the totals: atomics are serialised per cache line.
 constexpr int kChunkStride = 32;
 
@@ -522,60 +526,17 @@ __device__ __forceinline__ unsigned load_at(const int *base, int bytes) {
                                                static_cast<unsigned>(bytes));
 }
 
-// One tile per workgroup.  side / dup: kBlock 16-bit masks per tile; tile_pairs[t] gets the
-// tile's pairs, which are also added into chunk_pairs[t / kChunk] (zeroed by the partition
-// kernel).  The last workgroup stores the result length: the pairs (intersection), or
-// `items` (the operands' entries) less the pairs.  WIDE: the level's coordinates may need
-// 64-bit keys.  SPARSE: split_sparse_kernel ran; state[t] holds the pairs of a tile that it
-// wrote, or kDense.
-template <bool WIDE, bool SPARSE>
-__global__ __launch_bounds__(kBlock, WIDE ? 4 : 6) void order_kernel(
-    const int *__restrict__ pa, const int *__restrict__ ca, const int *__restrict__ pb,
-    const int *__restrict__ cb, const int *__restrict__ split_r, const int *__restrict__ split_a,
-    const int *__restrict__ split_b, int bits, unsigned short *__restrict__ side_out,
-    unsigned short *__restrict__ dup_out, const unsigned *__restrict__ state,
-    unsigned *__restrict__ tile_pairs, unsigned *__restrict__ chunk_pairs,
-    unsigned long long *__restrict__ done,
-    int64_t *__restrict__ length_out, int intersect, long long items) {
-    __shared__ __align__(16) OrderLds sh;
-    const int tid = threadIdx.x;
+// The merge order of the tile `sp`: lane tid's 16 slots as bit masks `side` and `dup`, and the
+// tile's pairs, the same in every lane.  `some`: any readable word.  Ends without a barrier.
+template <bool WIDE>
+__device__ __forceinline__ unsigned order_tile(OrderLds &sh, const TileSplit &sp,
+                                               const int *__restrict__ pa,
+                                               const int *__restrict__ ca,
+                                               const int *__restrict__ pb,
+                                               const int *__restrict__ cb, const int *some,
+                                               int bits, int tid, unsigned &side, unsigned &dup) {
     const int l = tid % dev::kWave;
     const int w = __builtin_amdgcn_readfirstlane(tid / dev::kWave);
-    const int t = blockIdx.x;
-    const int c = t / kChunk;
-    // The tile's pairs, or those of a chunk's written tiles, `tickets` of the chunk's (one
-    // thread).
-    auto total = [&](unsigned pairs, int tickets) {
-        if (pairs) atomicAdd(&chunk_pairs[c * kChunkStride], pairs);
-        const int64_t all = SPARSE ? ticket_total(pairs, tickets, c, gridDim.x, done)
-                                   : dev::two_level_total(pairs, done);
-        if (all >= 0) dev::store_system(length_out, intersect ? all : items - all);
-    };
-    if (SPARSE) {
-        if (t % kChunk == 0) {  // uniform: the chunk's tiles whose order is written
-            const int at = t + tid;
-            const unsigned v = at < static_cast<int>(gridDim.x) ? state[at] : 0u;
-            const unsigned long long dense = __ballot(v == kDense);
-            const int sum = dev::wave_inclusive_sum_dpp(v == kDense ? 0 : static_cast<int>(v));
-            if (l == dev::kWave - 1) {
-                sh.pairs[w] = static_cast<unsigned>(sum);
-                sh.sides[w] = static_cast<unsigned>(__popcll(dense));
-            }
-            __syncthreads();
-            if (tid == 0) {
-                unsigned pairs = 0, left = 0;
-#pragma unroll
-                for (int i = 0; i < kWaves; ++i) {
-                    pairs += sh.pairs[i];
-                    left += sh.sides[i];
-                }
-                total(pairs, kChunkTickets - static_cast<int>(left));
-            }
-            __syncthreads();
-        }
-        if (state[t] != kDense) return;  // uniform
-    }
-    const TileSplit sp = load_split(split_r, split_a, split_b, t);
     const int na = sp.a1 - sp.a0, nb = sp.b1 - sp.b0, nr = sp.r1 - sp.r0 + 1;
 
     // Slot tid + 256 j is A's entry of that index, or B's entry kSlots - 1 - slot.  The
@@ -588,7 +549,7 @@ __global__ __launch_bounds__(kBlock, WIDE ? 4 : 6) void order_kernel(
         const int first = kBlock * j + dev::kWave * w;  // the wavefront's slots
         const int base = kSlots - kBlock * (j + 1);     // B's entry of tid == kBlock - 1
         const bool in_a = first < na, in_b = first + dev::kWave > kSlots - nb;
-        const int *from = in_a ? ca + sp.a0 + kBlock * j : in_b ? cb + sp.b0 + base : split_r;
+        const int *from = in_a ? ca + sp.a0 + kBlock * j : in_b ? cb + sp.b0 + base  : some;
         const int last = in_a ? na - 1 - kBlock * j : in_b ? nb - 1 - base : 0;
         x[j] = load_at(from, min(in_a ? 4 * tid : 4 * (kBlock - 1 - tid), 4 * last));
     }
@@ -650,7 +611,6 @@ __global__ __launch_bounds__(kBlock, WIDE ? 4 : 6) void order_kernel(
     }
     __syncthreads();  // (the keys replace the marks)
 
-    unsigned side, dup;
     // (bits of nr, not of nr - 1: the padding's row, all ones, is no row of the tile)
     const int row_bits = 32 - __builtin_clz(static_cast<unsigned>(nr));
     const bool wide = WIDE && row_bits + bits + 1 > 32;
@@ -689,6 +649,66 @@ __global__ __launch_bounds__(kBlock, WIDE ? 4 : 6) void order_kernel(
         dup = 0;
         pairs = 0;
     }
+    return pairs;
+}
+
+// One tile per workgroup.  side / dup: kBlock 16-bit masks per tile; tile_pairs[t] gets the
+// tile's pairs, which are also added into chunk_pairs[t / kChunk] (zeroed by the partition
+// kernel).  The last workgroup stores the result length: the pairs (intersection), or
+// `items` (the operands' entries) less the pairs.  WIDE: the level's coordinates may need
+// 64-bit keys.  SPARSE: split_sparse_kernel ran; state[t] holds the pairs of a tile that it
+// wrote, or kDense.
+template <bool WIDE, bool SPARSE>
+__global__ __launch_bounds__(kBlock, WIDE ? 4 : 6) void order_kernel(
+    const int *__restrict__ pa, const int *__restrict__ ca, const int *__restrict__ pb,
+    const int *__restrict__ cb, const int *__restrict__ split_r, const int *__restrict__ split_a,
+    const int *__restrict__ split_b, int bits, unsigned short *__restrict__ side_out,
+    unsigned short *__restrict__ dup_out, const unsigned *__restrict__ state,
+    unsigned *__restrict__ tile_pairs, unsigned *__restrict__ chunk_pairs,
+    unsigned long long *__restrict__ done,
+    int64_t *__restrict__ length_out, int intersect, long long items) {
+    __shared__ __align__(16) OrderLds sh;
+    const int tid = threadIdx.x;
+    const int l = tid % dev::kWave;
+    const int w = __builtin_amdgcn_readfirstlane(tid / dev::kWave);
+    const int t = blockIdx.x;
+    const int c = t / kChunk;
+    // The tile's pairs, or those of a chunk's written tiles, `tickets` of the chunk's (one
+    // thread).
+    auto total = [&](unsigned pairs, int tickets) {
+        if (pairs) atomicAdd(&chunk_pairs[c * kChunkStride], pairs);
+        const int64_t all = SPARSE ? ticket_total(pairs, tickets, c, gridDim.x, done)
+                                   : dev::two_level_total(pairs, done);
+        if (all >= 0) dev::store_system(length_out, intersect ? all : items - all);
+    };
+    if (SPARSE) {
+        if (t % kChunk == 0) {  // uniform: the chunk's tiles whose order is written
+            const int at = t + tid;
+            const unsigned v = at < static_cast<int>(gridDim.x) ? state[at] : 0u;
+            const unsigned long long dense = __ballot(v == kDense);
+            const int sum = dev::wave_inclusive_sum_dpp(v == kDense ? 0 : static_cast<int>(v));
+            if (l == dev::kWave - 1) {
+                sh.pairs[w] = static_cast<unsigned>(sum);
+                sh.sides[w] = static_cast<unsigned>(__popcll(dense));
+            }
+            __syncthreads();
+            if (tid == 0) {
+                unsigned pairs = 0, left = 0;
+#pragma unroll
+                for (int i = 0; i < kWaves; ++i) {
+                    pairs += sh.pairs[i];
+                    left += sh.sides[i];
+                }
+                total(pairs, kChunkTickets - static_cast<int>(left));
+            }
+            __syncthreads();
+        }
+        if (state[t] != kDense) return;  // uniform
+    }
+    const TileSplit sp = load_split(split_r, split_a, split_b, t);
+    unsigned side, dup;
+    const unsigned pairs =
+        order_tile<WIDE>(sh, sp, pa, ca, pb, cb, split_r, bits, tid, side, dup);
     side_out[static_cast<size_t>(t) * kBlock + tid] = static_cast<unsigned short>(side);
     dup_out[static_cast<size_t>(t) * kBlock + tid] = static_cast<unsigned short>(dup);
     if (tid == 0) {
@@ -739,10 +759,17 @@ __device__ __forceinline__ int pairs_before(const EmitArgs &g, int t, int l) {
     return __builtin_amdgcn_readlane(dev::wave_inclusive_sum_dpp(sum), dev::kWave - 1);
 }
 
-// One tile per workgroup (DOT: tiles strided over the grid), a quarter of its slots and of
-// its row ends per wavefront; nothing is shared between wavefronts (but for the row marks of
-// ROWS).  Lane l of every wavefront holds order word l of the tile and the running counts of
-// B entries and pairs before it.  A wavefront's 16 words are loaded kGroup at a time before
+// LDS of a tile's output rows (ROWS).
+template <bool ROWS>
+struct RowLds {
+    alignas(16) unsigned short mark[ROWS ? kSlots : 8];
+    int carry[kWaves];
+};
+
+// Writes one tile's outputs, a quarter of its slots and of its row ends per wavefront; nothing
+// is shared between wavefronts (but for the row marks of ROWS).  Lane l of every wavefront
+// holds order word l of the tile (side_w, dup_w) and the running counts of B entries and pairs
+// before it; `pairs` is the pairs of the tiles before.  A wavefront's 16 words are loaded kGroup at a time before
 // any of them is stored: the loads in flight are what the memory's latency is hidden by.
 // C2's 547 MB take 105 us (5.2 TB/s; a copy reaches 5.5); with 4 words at a time and a
 // resident grid walking chunks of tiles it took 127 us.
@@ -752,192 +779,201 @@ __device__ __forceinline__ int pairs_before(const EmitArgs &g, int t, int l) {
 // [child[o], child[o + 1]) is the operand's child range under o, empty when absent (null
 // next: the position itself).  ROWS: rc receives each output's row.  ck (optional, with
 // ROWS): outputs stored split, c >> kbits to cc and the low kbits to ck.  DOT
-// (intersection): the workgroup's products summed in binary64 to partial[w] instead.
+// (intersection): the products are added to acc instead.
 //
 // The operands' arrays are never null (the host passes some valid array for an empty one):
 // every load is unconditional, at an entry of the operand.
 template <Op OP, bool VALUES, bool CHILD, bool ROWS, bool DOT>
-__global__ __launch_bounds__(kBlock) void emit_kernel(EmitArgs g) {
+__device__ __forceinline__ void emit_tile(const EmitArgs &g, const TileSplit &sp, int t,
+                                          unsigned long long side_w, unsigned long long dup_w,
+                                          int pairs, int tid, RowLds<ROWS> &lds, double &acc) {
     static_assert(!(VALUES && CHILD) && (VALUES || !ROWS), "a level carries one kind of payload");
     static_assert(!DOT || (OP == Op::Intersect && VALUES), "the inner product: intersection");
     constexpr int kGroup = OP == Op::Union && VALUES ? 16 : 8;  // words loaded together
     constexpr int kWordsPerWave = kWords / kWaves;
-    __shared__ __align__(16) unsigned short s_mark[ROWS ? kSlots : 8];
-    __shared__ int s_carry[kWaves];
+    const int l = tid % dev::kWave;
+    const int w = __builtin_amdgcn_readfirstlane(tid / dev::kWave);
+    const int n = sp.a1 - sp.a0 + sp.b1 - sp.b0;
+    const int ends = sp.r1 - sp.r0;  // rows r0 .. r0 + ends - 1 end in the tile
+    const int side_n = __popcll(side_w), dup_n = __popcll(dup_w);
+    const int side_before = dev::wave_inclusive_sum_dpp(side_n) - side_n;
+    const int dup_incl = dev::wave_inclusive_sum_dpp(dup_n);
+    const int dup_before = dup_incl - dup_n;
+    const int tile_pairs = __builtin_amdgcn_readlane(dup_incl, dev::kWave - 1);
+    const int out0 = OP == Op::Union ? sp.a0 + sp.b0 - pairs : pairs;  // first output
+
+    if (ROWS) {  // row marks by slot, as in the order kernel but in merged order
+        uint4 *clear = reinterpret_cast<uint4 *>(lds.mark);
+        clear[tid] = uint4{0, 0, 0, 0};
+        clear[tid + kBlock] = uint4{0, 0, 0, 0};
+        if (tid < kWaves) lds.carry[tid] = 0;
+        __syncthreads();
+        for (int k = tid; k <= ends; k += kBlock) {
+            const int s = k == 0 ? 0 : g.pa[sp.r0 + k] - sp.a0 + g.pb[sp.r0 + k] - sp.b0;
+            const int e = k == ends ? n
+                                    : g.pa[sp.r0 + k + 1] - sp.a0 + g.pb[sp.r0 + k + 1] - sp.b0;
+            if (e > s) {
+                lds.mark[s] = static_cast<unsigned short>(k);
+                atomicMax(&lds.carry[s / (kSlots / kWaves)], k);
+            }
+        }
+        __syncthreads();
+    }
+    int row_carry = 0;  // last row started before the wavefront's next word (tile-local)
+    if (ROWS) {
+        for (int i = 0; i < w; ++i) row_carry = max(row_carry, lds.carry[i]);
+        row_carry = __builtin_amdgcn_readfirstlane(row_carry);
+    }
+
+    for (int i0 = w * kWordsPerWave; i0 < (w + 1) * kWordsPerWave; i0 += kGroup) {
+        if (i0 * 64 >= n) break;  // uniform
+        if (OP == Op::Intersect && !ROWS) {  // words without pairs: next (uniform)
+            const unsigned long long any = __ballot(dup_w != 0);
+            // (a pair's A slot may be the last one before its B slot's word; with ROWS,
+            // every word carries its last row to the next)
+            if (((any >> i0) & ((2ull << kGroup) - 1ull)) == 0) continue;
+        }
+        int c[kGroup], ra[CHILD ? kGroup : 1], rb[CHILD ? kGroup : 1];
+        float v[kGroup], v2[OP == Op::Intersect ? kGroup : 1];
+        // slots of word i that hold an entry
+        auto valid_of = [&](int i) {
+            const int left = n - i * 64;
+            return left >= 64 ? ~0ull : left <= 0 ? 0ull : (1ull << left) - 1ull;
+        };
+        // A entries of pairs in word i: the slot after them is a pair's B entry
+        auto pairs_of = [&](int i, unsigned long long dup) {
+            const unsigned long long next =
+                i + 1 < kWords ? readlane64(dup_w, min(i + 1, kWords - 1)) : 0ull;
+            return (dup >> 1) | (next << 63);
+        };
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) {
+            const int i = i0 + u;
+            const unsigned long long side = readlane64(side_w, i);
+            const int sb = __builtin_amdgcn_readlane(side_before, i);
+            const int below = bits_below(side);
+            const int ib = sp.b0 + sb + below;                 // B position reached
+            const int ia = sp.a0 + i * 64 - sb + (l - below);  // A position reached
+            if (OP == Op::Union) {
+                const bool is_b = __builtin_amdgcn_inverse_ballot_w64(side);
+                const bool in = __builtin_amdgcn_inverse_ballot_w64(valid_of(i));
+                const int at = in ? (is_b ? ib : ia) : 0;
+                c[u] = (is_b ? g.cb : g.ca)[at];
+                if (VALUES) v[u] = (is_b ? g.vb : g.va)[at];
+                if (CHILD) {
+                    const int xa = in ? ia : 0, xb = in ? ib : 0;
+                    ra[u] = g.next_a ? g.next_a[xa] : xa;
+                    rb[u] = g.next_b ? g.next_b[xb] : xb;
+                }
+            } else {
+                // Lanes without a pair load too: no branch between the loads.  The
+                // result's: the entries reached, whose lines its neighbours need; the
+                // inner product's, where pairs are few: entry 0.
+                const bool in = !DOT || __builtin_amdgcn_inverse_ballot_w64(
+                                            pairs_of(i, readlane64(dup_w, i)));
+                const int xa = in ? min(ia, max(g.nnz_a - 1, 0)) : 0;
+                const int xb = in ? min(ib, max(g.nnz_b - 1, 0)) : 0;
+                if (!DOT) c[u] = g.ca[xa];
+                v[u] = g.va[xa];
+                v2[u] = g.vb[xb];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) {
+            const int i = i0 + u;
+            const unsigned long long dup = readlane64(dup_w, i);
+            const unsigned long long pair_a = pairs_of(i, dup);
+            const unsigned long long emit = OP == Op::Union ? valid_of(i) & ~dup : pair_a;
+            float val = v[u];
+            if (OP == Op::Intersect) {
+                val = v[u] * v2[u];
+            } else if (VALUES && pair_a != 0) {  // uniform
+                // the pair's B value was loaded by the next slot (wave_shl:1)
+                float other = __int_as_float(__builtin_amdgcn_update_dpp(
+                    0, __float_as_int(v[u]), 0x130, 0xf, 0xf, true));
+                if (pair_a >> 63) {  // the next word's first slot
+                    float next = 0.0f;
+                    if (u + 1 < kGroup) {
+                        next = __int_as_float(__builtin_amdgcn_readlane(
+                            __float_as_int(v[(u + 1) % kGroup]), 0));
+                    } else {
+                        const unsigned long long side = readlane64(side_w, i);
+                        next = g.vb[sp.b0 + __builtin_amdgcn_readlane(side_before, i) +
+                                    __popcll(side)];
+                    }
+                    if (l == dev::kWave - 1) other = next;
+                }
+                if (__builtin_amdgcn_inverse_ballot_w64(pair_a)) val = v[u] + other;
+            }
+            if (DOT) {
+                if (__builtin_amdgcn_inverse_ballot_w64(emit)) acc += static_cast<double>(val);
+                continue;
+            }
+            int row = 0;
+            if (ROWS) {
+                const int m = dev::wave_inclusive_max_dpp(lds.mark[i * 64 + l]);
+                row = max(m, row_carry);
+                row_carry = max(row_carry, __builtin_amdgcn_readlane(m, dev::kWave - 1));
+            }
+            const int db = __builtin_amdgcn_readlane(dup_before, i);
+            const int first = OP == Op::Union ? out0 + i * 64 - db : out0 + db;
+            const int o = first + (OP == Op::Union ? l - bits_below(dup) : bits_below(dup));
+            if (__builtin_amdgcn_inverse_ballot_w64(emit)) {
+                if (ROWS && g.ck) {
+                    g.cc[o] = c[u] >> g.kbits;
+                    g.ck[o] = static_cast<int>(static_cast<unsigned>(c[u]) &
+                                               ((1u << g.kbits) - 1u));
+                } else {
+                    g.cc[o] = c[u];
+                }
+                if (VALUES) g.vc[o] = val;
+                if (CHILD) {
+                    g.child_a[o] = ra[u];
+                    g.child_b[o] = rb[u];
+                }
+                if (ROWS) g.rc[o] = sp.r0 + row;
+            }
+        }
+    }
+
+    if (!DOT) {  // row ends: row r0 + k ends before slot s of the tile
+        for (int k0 = w * dev::kWave; k0 < ends; k0 += kBlock) {  // uniform in the wave
+            const int k = min(k0 + l, ends - 1);
+            const int s = g.pa[sp.r0 + k + 1] - sp.a0 + g.pb[sp.r0 + k + 1] - sp.b0;
+            int d = 0;
+            if (tile_pairs != 0) {  // pairs whose B slot lies before s
+                const int at = min(s >> 6, kWords - 1);
+                const unsigned long long word = __shfl(dup_w, at, dev::kWave);
+                const int used = s - (at << 6);  // 0 .. 64
+                const unsigned long long low = used >= 64 ? ~0ull : (1ull << used) - 1ull;
+                d = __shfl(dup_before, at, dev::kWave) + __popcll(word & low);
+            }
+            if (k0 + l < ends) g.pc[sp.r0 + k + 1] = out0 + (OP == Op::Union ? s - d : d);
+        }
+        if (t == 0 && tid == 0) g.pc[0] = 0;
+    }
+    if (CHILD && t == g.num_tiles - 1 && tid == 0) {
+        const int end = out0 + n - tile_pairs;
+        g.child_a[end] = g.next_a ? g.next_a[g.nnz_a] : g.nnz_a;
+        g.child_b[end] = g.next_b ? g.next_b[g.nnz_b] : g.nnz_b;
+    }
+}
+
+// One tile per workgroup (DOT: tiles strided over the grid, the workgroup's products summed
+// to partial[w]).
+template <Op OP, bool VALUES, bool CHILD, bool ROWS, bool DOT>
+__global__ __launch_bounds__(kBlock) void emit_kernel(EmitArgs g) {
+    __shared__ RowLds<ROWS> lds;
     __shared__ double s_dot[DOT ? kBlock : 1];
     const int tid = threadIdx.x;
     const int l = tid % dev::kWave;
-    const int w = __builtin_amdgcn_readfirstlane(tid / dev::kWave);
     double acc = 0.0;
     for (int t = blockIdx.x; t < g.num_tiles; t += gridDim.x) {  // (once but for DOT)
         const unsigned long long side_w = g.side[static_cast<size_t>(t) * kWords + l];
         const unsigned long long dup_w = g.dup[static_cast<size_t>(t) * kWords + l];
         const TileSplit sp = load_split(g.split_r, g.split_a, g.split_b, t);
-        const int n = sp.a1 - sp.a0 + sp.b1 - sp.b0;
-        const int ends = sp.r1 - sp.r0;  // rows r0 .. r0 + ends - 1 end in the tile
-        const int pairs = DOT ? 0 : pairs_before(g, t, l);
-        const int side_n = __popcll(side_w), dup_n = __popcll(dup_w);
-        const int side_before = dev::wave_inclusive_sum_dpp(side_n) - side_n;
-        const int dup_incl = dev::wave_inclusive_sum_dpp(dup_n);
-        const int dup_before = dup_incl - dup_n;
-        const int tile_pairs = __builtin_amdgcn_readlane(dup_incl, dev::kWave - 1);
-        const int out0 = OP == Op::Union ? sp.a0 + sp.b0 - pairs : pairs;  // first output
-
-        if (ROWS) {  // row marks by slot, as in the order kernel but in merged order
-            uint4 *clear = reinterpret_cast<uint4 *>(s_mark);
-            clear[tid] = uint4{0, 0, 0, 0};
-            clear[tid + kBlock] = uint4{0, 0, 0, 0};
-            if (tid < kWaves) s_carry[tid] = 0;
-            __syncthreads();
-            for (int k = tid; k <= ends; k += kBlock) {
-                const int s = k == 0 ? 0 : g.pa[sp.r0 + k] - sp.a0 + g.pb[sp.r0 + k] - sp.b0;
-                const int e = k == ends ? n
-                                        : g.pa[sp.r0 + k + 1] - sp.a0 + g.pb[sp.r0 + k + 1] - sp.b0;
-                if (e > s) {
-                    s_mark[s] = static_cast<unsigned short>(k);
-                    atomicMax(&s_carry[s / (kSlots / kWaves)], k);
-                }
-            }
-            __syncthreads();
-        }
-        int row_carry = 0;  // last row started before the wavefront's next word (tile-local)
-        if (ROWS) {
-            for (int i = 0; i < w; ++i) row_carry = max(row_carry, s_carry[i]);
-            row_carry = __builtin_amdgcn_readfirstlane(row_carry);
-        }
-
-        for (int i0 = w * kWordsPerWave; i0 < (w + 1) * kWordsPerWave; i0 += kGroup) {
-            if (i0 * 64 >= n) break;  // uniform
-            if (OP == Op::Intersect && !ROWS) {  // words without pairs: next (uniform)
-                const unsigned long long any = __ballot(dup_w != 0);
-                // (a pair's A slot may be the last one before its B slot's word; with ROWS,
-                // every word carries its last row to the next)
-                if (((any >> i0) & ((2ull << kGroup) - 1ull)) == 0) continue;
-            }
-            int c[kGroup], ra[CHILD ? kGroup : 1], rb[CHILD ? kGroup : 1];
-            float v[kGroup], v2[OP == Op::Intersect ? kGroup : 1];
-            // slots of word i that hold an entry
-            auto valid_of = [&](int i) {
-                const int left = n - i * 64;
-                return left >= 64 ? ~0ull : left <= 0 ? 0ull : (1ull << left) - 1ull;
-            };
-            // A entries of pairs in word i: the slot after them is a pair's B entry
-            auto pairs_of = [&](int i, unsigned long long dup) {
-                const unsigned long long next =
-                    i + 1 < kWords ? readlane64(dup_w, min(i + 1, kWords - 1)) : 0ull;
-                return (dup >> 1) | (next << 63);
-            };
-#pragma unroll
-            for (int u = 0; u < kGroup; ++u) {
-                const int i = i0 + u;
-                const unsigned long long side = readlane64(side_w, i);
-                const int sb = __builtin_amdgcn_readlane(side_before, i);
-                const int below = bits_below(side);
-                const int ib = sp.b0 + sb + below;                 // B position reached
-                const int ia = sp.a0 + i * 64 - sb + (l - below);  // A position reached
-                if (OP == Op::Union) {
-                    const bool is_b = __builtin_amdgcn_inverse_ballot_w64(side);
-                    const bool in = __builtin_amdgcn_inverse_ballot_w64(valid_of(i));
-                    const int at = in ? (is_b ? ib : ia) : 0;
-                    c[u] = (is_b ? g.cb : g.ca)[at];
-                    if (VALUES) v[u] = (is_b ? g.vb : g.va)[at];
-                    if (CHILD) {
-                        const int xa = in ? ia : 0, xb = in ? ib : 0;
-                        ra[u] = g.next_a ? g.next_a[xa] : xa;
-                        rb[u] = g.next_b ? g.next_b[xb] : xb;
-                    }
-                } else {
-                    // Lanes without a pair load too: no branch between the loads.  The
-                    // result's: the entries reached, whose lines its neighbours need; the
-                    // inner product's, where pairs are few: entry 0.
-                    const bool in = !DOT || __builtin_amdgcn_inverse_ballot_w64(
-                                                pairs_of(i, readlane64(dup_w, i)));
-                    const int xa = in ? min(ia, max(g.nnz_a - 1, 0)) : 0;
-                    const int xb = in ? min(ib, max(g.nnz_b - 1, 0)) : 0;
-                    if (!DOT) c[u] = g.ca[xa];
-                    v[u] = g.va[xa];
-                    v2[u] = g.vb[xb];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kGroup; ++u) {
-                const int i = i0 + u;
-                const unsigned long long dup = readlane64(dup_w, i);
-                const unsigned long long pair_a = pairs_of(i, dup);
-                const unsigned long long emit = OP == Op::Union ? valid_of(i) & ~dup : pair_a;
-                float val = v[u];
-                if (OP == Op::Intersect) {
-                    val = v[u] * v2[u];
-                } else if (VALUES && pair_a != 0) {  // uniform
-                    // the pair's B value was loaded by the next slot (wave_shl:1)
-                    float other = __int_as_float(__builtin_amdgcn_update_dpp(
-                        0, __float_as_int(v[u]), 0x130, 0xf, 0xf, true));
-                    if (pair_a >> 63) {  // the next word's first slot
-                        float next = 0.0f;
-                        if (u + 1 < kGroup) {
-                            next = __int_as_float(__builtin_amdgcn_readlane(
-                                __float_as_int(v[(u + 1) % kGroup]), 0));
-                        } else {
-                            const unsigned long long side = readlane64(side_w, i);
-                            next = g.vb[sp.b0 + __builtin_amdgcn_readlane(side_before, i) +
-                                        __popcll(side)];
-                        }
-                        if (l == dev::kWave - 1) other = next;
-                    }
-                    if (__builtin_amdgcn_inverse_ballot_w64(pair_a)) val = v[u] + other;
-                }
-                if (DOT) {
-                    if (__builtin_amdgcn_inverse_ballot_w64(emit)) acc += static_cast<double>(val);
-                    continue;
-                }
-                int row = 0;
-                if (ROWS) {
-                    const int m = dev::wave_inclusive_max_dpp(s_mark[i * 64 + l]);
-                    row = max(m, row_carry);
-                    row_carry = max(row_carry, __builtin_amdgcn_readlane(m, dev::kWave - 1));
-                }
-                const int db = __builtin_amdgcn_readlane(dup_before, i);
-                const int first = OP == Op::Union ? out0 + i * 64 - db : out0 + db;
-                const int o = first + (OP == Op::Union ? l - bits_below(dup) : bits_below(dup));
-                if (__builtin_amdgcn_inverse_ballot_w64(emit)) {
-                    if (ROWS && g.ck) {
-                        g.cc[o] = c[u] >> g.kbits;
-                        g.ck[o] = static_cast<int>(static_cast<unsigned>(c[u]) &
-                                                   ((1u << g.kbits) - 1u));
-                    } else {
-                        g.cc[o] = c[u];
-                    }
-                    if (VALUES) g.vc[o] = val;
-                    if (CHILD) {
-                        g.child_a[o] = ra[u];
-                        g.child_b[o] = rb[u];
-                    }
-                    if (ROWS) g.rc[o] = sp.r0 + row;
-                }
-            }
-        }
-
-        if (!DOT) {  // row ends: row r0 + k ends before slot s of the tile
-            for (int k0 = w * dev::kWave; k0 < ends; k0 += kBlock) {  // uniform in the wave
-                const int k = min(k0 + l, ends - 1);
-                const int s = g.pa[sp.r0 + k + 1] - sp.a0 + g.pb[sp.r0 + k + 1] - sp.b0;
-                int d = 0;
-                if (tile_pairs != 0) {  // pairs whose B slot lies before s
-                    const int at = min(s >> 6, kWords - 1);
-                    const unsigned long long word = __shfl(dup_w, at, dev::kWave);
-                    const int used = s - (at << 6);  // 0 .. 64
-                    const unsigned long long low = used >= 64 ? ~0ull : (1ull << used) - 1ull;
-                    d = __shfl(dup_before, at, dev::kWave) + __popcll(word & low);
-                }
-                if (k0 + l < ends) g.pc[sp.r0 + k + 1] = out0 + (OP == Op::Union ? s - d : d);
-            }
-            if (t == 0 && tid == 0) g.pc[0] = 0;
-        }
-        if (CHILD && t == g.num_tiles - 1 && tid == 0) {
-            const int end = out0 + n - tile_pairs;
-            g.child_a[end] = g.next_a ? g.next_a[g.nnz_a] : g.nnz_a;
-            g.child_b[end] = g.next_b ? g.next_b[g.nnz_b] : g.nnz_b;
-        }
+        emit_tile<OP, VALUES, CHILD, ROWS, DOT>(g, sp, t, side_w, dup_w,
+                                                DOT ? 0 : pairs_before(g, t, l), tid, lds, acc);
     }
     if (DOT) {
         s_dot[tid] = acc;
@@ -948,6 +984,103 @@ __global__ __launch_bounds__(kBlock) void emit_kernel(EmitArgs g) {
         }
         if (tid == 0) g.partial[blockIdx.x] = s_dot[0];
     }
+}
+
+// ---- small levels ----------------------------------------------------------------------
+//
+// A level of few tiles in one launch: a workgroup finds its tile's boundaries, orders it,
+// publishes its pairs, waits for those of the tiles before it and writes its outputs.  Tiles
+// are dealt by a ticket, so a workgroup only waits for workgroups that have started; with few
+// tiles they all run at once and the wait is the spread of their starts.  (With thousands, the
+// first tile's output would wait for nothing while the memory is idle: three launches are
+// better.)
+//
+// `sync` is a block of words that only these kernels write: a ticket counter that keeps
+// counting from launch to launch (this launch's tickets start at `base`) and, per tile, the
+// pairs tagged with the launch's epoch, so that it is never cleared.
+constexpr int kSyncTiles = 16;  // word of tile 0
+constexpr int kMaxPolls = 1 << 22;  // seconds
+constexpr size_t kSyncBytes = (kSyncTiles + kFusedTiles) * sizeof(unsigned long long);
+
+template <Op OP, bool VALUES, bool CHILD, bool ROWS, bool WIDE>
+__global__ __launch_bounds__(kBlock) void fused_kernel(EmitArgs g, int rows, int total, int bits,
+                                                       unsigned long long *__restrict__ sync,
+                                                       unsigned epoch, unsigned base,
+                                                       int64_t *__restrict__ length_out,
+                                                       long long items) {
+    __shared__ __align__(16) OrderLds sh;
+    __shared__ __align__(8) unsigned short s_side[kBlock], s_dup[kBlock];
+    __shared__ RowLds<ROWS> lds;
+    __shared__ int s_split[6];
+    __shared__ int s_ticket, s_wave[kWaves];
+    const int tid = threadIdx.x;
+    const int l = tid % dev::kWave;
+    const int w = __builtin_amdgcn_readfirstlane(tid / dev::kWave);
+    int t = 0;
+    if (g.num_tiles > 1) {  // uniform
+        if (tid == 0) s_ticket = static_cast<int>(atomicAdd(reinterpret_cast<unsigned *>(sync), 1u) - base);
+        __syncthreads();
+        t = __builtin_amdgcn_readfirstlane(s_ticket);
+        if (t < 0 || t >= g.num_tiles) return;  // (as above)
+    }
+    if (w < 2) {  // boundary t + w
+        const int b = t + w;
+        int r = 0, x = 0, y = 0;
+        if (b == g.num_tiles) {
+            r = rows;
+            x = g.pa[rows];
+            y = g.pb[rows];
+        } else if (b > 0) {
+            find_split<dev::kWave>(g.pa, g.ca, g.pb, g.cb, rows,
+                                   static_cast<int>(min(static_cast<long long>(b) * kTile,
+                                                        static_cast<long long>(total))),
+                                   r, x, y);
+        }
+        if (l == 0) {
+            s_split[3 * w] = r;
+            s_split[3 * w + 1] = x;
+            s_split[3 * w + 2] = y;
+        }
+    }
+    __syncthreads();
+    auto u = [&](int i) { return __builtin_amdgcn_readfirstlane(s_split[i]); };
+    const TileSplit sp{u(0), u(1), u(2), u(3), u(4), u(5)};
+    unsigned side, dup;
+    const unsigned own = order_tile<WIDE>(sh, sp, g.pa, g.ca, g.pb, g.cb, g.pa, bits, tid, side, dup);
+    if (tid == 0 && t + 1 < g.num_tiles) {
+        __hip_atomic_store(&sync[kSyncTiles + t],
+                           (static_cast<unsigned long long>(epoch) << 32) | own,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    s_side[tid] = static_cast<unsigned short>(side);
+    s_dup[tid] = static_cast<unsigned short>(dup);
+    // (The waits end: the workgroups of the tiles before have started and wait for earlier
+    // ones only.  The bound is for a block whose counts are not what the host believes: the
+    // length is then never stored, which the host reports.)
+    int before = 0;
+    bool found = true;
+    for (int i = tid; i < t && found; i += kBlock) {
+        unsigned long long v = 0;
+        int polls = 0;
+        do {
+            v = __hip_atomic_load(&sync[kSyncTiles + i], __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+        } while ((v >> 32) != epoch && ++polls < kMaxPolls);
+        found = (v >> 32) == epoch;
+        if (found) before += static_cast<int>(v & 0xffffffffull);
+    }
+    int pairs = 0;
+    (void)dev::block_exclusive_sum<kBlock>(before, s_wave, pairs);
+    pairs = __builtin_amdgcn_readfirstlane(pairs);
+    if (__syncthreads_or(!found)) return;
+    if (tid == 0 && t == g.num_tiles - 1) {
+        const int64_t all = static_cast<int64_t>(pairs) + own;
+        dev::store_system(length_out, OP == Op::Union ? items - all : all);
+    }
+    const unsigned long long side_w = reinterpret_cast<const unsigned long long *>(s_side)[l];
+    const unsigned long long dup_w = reinterpret_cast<const unsigned long long *>(s_dup)[l];
+    double acc = 0.0;
+    emit_tile<OP, VALUES, CHILD, ROWS, false>(g, sp, t, side_w, dup_w, pairs, tid, lds, acc);
 }
 
 // ---- fixed-order sums ------------------------------------------------------------------
@@ -1039,6 +1172,52 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
     }
     const int chunks = (num_tiles + kChunk - 1) / kChunk;
 
+    const hipStream_t s = call.stream();
+    const long long items = static_cast<long long>(A.len) + B.len;
+    // 32-bit keys hold any tile's rows (12 bits) beside coordinates of up to 19 bits.
+    const bool wide = crd_bits + 13 > 32;
+    // (an empty operand's arrays may be null: A's offsets stand in, never used as values)
+    const int *ca = A.len > 0 ? A.crd : A.pos, *cb = B.len > 0 ? B.crd : A.pos;
+    const float *va = A.len > 0 && values ? A.val : reinterpret_cast<const float *>(A.pos);
+    const float *vb = B.len > 0 && values ? B.val : reinterpret_cast<const float *>(A.pos);
+    EmitArgs args{A.pos, ca, va, B.pos, cb, vb, nullptr, nullptr, nullptr, nullptr, nullptr,
+                  nullptr, nullptr, num_tiles, Z.pos, Z.crd, Z.val, A.next, B.next, Z.child_a,
+                  Z.child_b, A.len, B.len, Z.row, Z.crd_low, Z.low_bits, nullptr};
+    SyncBlock sync{};
+    if (num_tiles <= kFusedTiles && !Z.dot) {
+        // (one tile takes no ticket)
+        NACHO_TRY(call.sync_block(kSyncBytes, num_tiles > 1 ? num_tiles : 0, &sync));
+    }
+    if (sync.words) {
+        void (*fused)(EmitArgs, int, int, int, unsigned long long *, unsigned, unsigned,
+                      int64_t *, long long) =
+#define NACHO_FUSED(OP, VAL, CHD, ROWS) \
+    (wide ? fused_kernel<OP, VAL, CHD, ROWS, true> : fused_kernel<OP, VAL, CHD, ROWS, false>)
+            child       ? NACHO_FUSED(Op::Union, false, true, false)
+            : intersect ? (Z.row ? NACHO_FUSED(Op::Intersect, true, false, true)
+                                 : NACHO_FUSED(Op::Intersect, true, false, false))
+            : Z.row     ? NACHO_FUSED(Op::Union, true, false, true)
+                        : NACHO_FUSED(Op::Union, true, false, false);
+#undef NACHO_FUSED
+        int64_t *length_out = nullptr;
+        NACHO_TRY(call.length_word(&length_out));
+        NACHO_TRY(call.timer_start(kernel_name));
+        fused<<<num_tiles, kBlock, 0, s>>>(args, rows, static_cast<int>(total), crd_bits,
+                                           sync.words, sync.epoch, sync.base, length_out, items);
+        NACHO_TRY_HIP(hipGetLastError());
+        call.sync_launched();
+        NACHO_TRY(call.mark_length());
+        NACHO_TRY(call.timer_stop());
+        if (length_pending) {
+            *length_pending = true;
+            return NACHO_OK;
+        }
+        int64_t len = 0;
+        NACHO_TRY(call.wait_length(&len));
+        *out_len = len;
+        return NACHO_OK;
+    }
+
     int *splits = nullptr;
     unsigned *counts = nullptr;
     unsigned short *order = nullptr;
@@ -1066,8 +1245,6 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
         NACHO_TRY(call.length_word(&length_out));
     }
 
-    const hipStream_t s = call.stream();
-    const long long items = static_cast<long long>(A.len) + B.len;
     NACHO_TRY(call.timer_start(kernel_name));  // the whole device pipeline of this level
     unsigned long long *side64 = reinterpret_cast<unsigned long long *>(side);
     unsigned long long *dup64 = reinterpret_cast<unsigned long long *>(dup);
@@ -1084,8 +1261,6 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
             split_a, split_b, done, counts, chunks, kChunkStride);
     }
     NACHO_TRY_HIP(hipGetLastError());
-    // 32-bit keys hold any tile's rows (12 bits) beside coordinates of up to 19 bits.
-    const bool wide = crd_bits + 13 > 32;
     auto order_fn = sparse ? (wide ? order_kernel<true, true> : order_kernel<false, true>)
                            : (wide ? order_kernel<true, false> : order_kernel<false, false>);
     order_fn<<<num_tiles, kBlock, 0, s>>>(A.pos, A.crd, B.pos, B.crd, split_r, split_a, split_b,
@@ -1093,13 +1268,14 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
                                           length_out, intersect ? 1 : 0, items);
     NACHO_TRY_HIP(hipGetLastError());
     if (!Z.dot) NACHO_TRY(call.mark_length());
-    // (an empty operand's arrays may be null: the splits stand in, never used as values)
-    const int *ca = A.len > 0 ? A.crd : splits, *cb = B.len > 0 ? B.crd : splits;
-    const float *va = A.len > 0 && values ? A.val : reinterpret_cast<const float *>(splits);
-    const float *vb = B.len > 0 && values ? B.val : reinterpret_cast<const float *>(splits);
-    const EmitArgs args{A.pos, ca, va, B.pos, cb, vb, split_r, split_a, split_b,
-                        side64, dup64, tile_pairs, counts, num_tiles, Z.pos, Z.crd, Z.val, A.next, B.next, Z.child_a, Z.child_b,
-                        A.len, B.len, Z.row, Z.crd_low, Z.low_bits, partial};
+    args.split_r = split_r;
+    args.split_a = split_a;
+    args.split_b = split_b;
+    args.side = side64;
+    args.dup = dup64;
+    args.tile_pairs = tile_pairs;
+    args.chunk_pairs = counts;
+    args.partial = partial;
     emit<<<grid, kBlock, 0, s>>>(args);
     NACHO_TRY_HIP(hipGetLastError());
     if (Z.dot) {

@@ -9,6 +9,8 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <thread>
+#include <tuple>
 #include <unordered_map>
 #include <utility>
 #include <vector>
@@ -95,6 +97,8 @@ void drop_shared_locked(SharedEvent *s) {
     }
 }
 
+void free_sync_blocks_locked();
+
 size_t size_class(size_t bytes) {
     if (bytes <= 512) return 512;
     size_t p = 1;
@@ -115,6 +119,7 @@ void release_cached_blocks_locked() {
     }
     g_free.clear();
     g_free_bytes = 0;
+    free_sync_blocks_locked();
     for (hipEvent_t e : g_event_pool) (void)hipEventDestroy(e);
     g_event_pool.clear();
 }
@@ -250,6 +255,93 @@ int record_stream(void *ptr, hipStream_t stream) {
     return NACHO_OK;
 }
 
+// ---- sync blocks -----------------------------------------------------------------------
+// One block per (device, stream, host thread): a thread's launches on one stream run in the
+// order it made them, which is the order of the epochs and tickets it took.  A block in use by
+// a call is not freed; the others (a few KB each) go back to the driver with the cache
+// (nacho_release_cached_memory) and when they outnumber kMaxSyncBlocks.
+struct SyncEntry {
+    unsigned long long *words;
+    size_t bytes;
+    unsigned epoch;
+    unsigned tickets;
+    bool busy;
+};
+using SyncKey = std::tuple<int, hipStream_t, std::thread::id>;
+constexpr size_t kMaxSyncBlocks = 64;
+std::map<SyncKey, SyncEntry> g_sync;
+
+__global__ void clear_words_kernel(unsigned long long *words, size_t n) {
+    for (size_t i = threadIdx.x; i < n; i += blockDim.x) words[i] = 0ull;
+}
+
+// Frees every block that no call holds (their launches may still run: the device is
+// synchronised first).  Caller holds g_cache_mutex.
+void free_sync_blocks_locked() {
+    (void)hipDeviceSynchronize();
+    for (auto it = g_sync.begin(); it != g_sync.end();) {
+        if (it->second.busy) {
+            ++it;
+        } else {
+            (void)hipFree(it->second.words);
+            it = g_sync.erase(it);
+        }
+    }
+}
+
+// A use of the caller's block, which stays busy until give_sync_block.
+int take_sync_block(size_t bytes, unsigned tickets, hipStream_t stream, SyncKey *key,
+                    SyncBlock *out) {
+    int device = 0;
+    NACHO_TRY_HIP(hipGetDevice(&device));
+    *key = SyncKey{device, stream, std::this_thread::get_id()};
+    std::lock_guard<std::mutex> lock(g_cache_mutex);
+    auto it = g_sync.find(*key);
+    if (it != g_sync.end() && (it->second.bytes < bytes || it->second.epoch == UINT_MAX)) {
+        (void)hipDeviceSynchronize();
+        (void)hipFree(it->second.words);
+        g_sync.erase(it);
+        it = g_sync.end();
+    }
+    if (it == g_sync.end()) {
+        if (g_sync.size() >= kMaxSyncBlocks) free_sync_blocks_locked();
+        void *p = nullptr;
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return NACHO_OK;  // none to take
+        }
+        unsigned long long *words = static_cast<unsigned long long *>(p);
+        clear_words_kernel<<<1, 256, 0, stream>>>(words, bytes / sizeof(unsigned long long));
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) {
+            (void)hipFree(p);
+            return static_cast<int>(e);
+        }
+        it = g_sync.insert({*key, SyncEntry{words, bytes, 0u, 0u, false}}).first;
+    }
+    SyncEntry &b = it->second;
+    b.busy = true;
+    out->words = b.words;
+    out->epoch = ++b.epoch;
+    out->base = b.tickets;
+    b.tickets += tickets;
+    return NACHO_OK;
+}
+
+// The call that took the block ends; `sound`: every launch it was taken for was made (the
+// block's counts are otherwise unknown, so it is dropped).
+void give_sync_block(const SyncKey &key, bool sound) {
+    std::lock_guard<std::mutex> lock(g_cache_mutex);
+    auto it = g_sync.find(key);
+    if (it == g_sync.end()) return;
+    it->second.busy = false;
+    if (!sound) {
+        (void)hipDeviceSynchronize();
+        (void)hipFree(it->second.words);
+        g_sync.erase(it);
+    }
+}
+
 // Kernel timing state (per host thread).
 std::atomic<int> g_timing_enabled{0};
 thread_local hipEvent_t t_ev_start = nullptr;
@@ -282,6 +374,11 @@ Call::Call(void *stream, void *arena, size_t arena_bytes)
 
 Call::~Call() {
     if (arena_) return;  // nothing was allocated
+    if (sync_held_) {
+        int device = 0;
+        (void)hipGetDevice(&device);
+        give_sync_block(SyncKey{device, stream_, std::this_thread::get_id()}, sync_sound_);
+    }
     if (timed_) t_last_ms = timed_ms_;
     if (!committed_) scratch_.insert(scratch_.end(), results_.begin(), results_.end());
     if (alloc_) {
@@ -331,6 +428,18 @@ int Call::result(size_t bytes, void **out) {
     results_.push_back(p);
     *out = p;
     return NACHO_OK;
+}
+
+int Call::sync_block(size_t bytes, unsigned tickets, SyncBlock *out) {
+    *out = SyncBlock{};
+    if (arena_ || alloc_) return NACHO_OK;
+    SyncKey key;
+    const int rc = take_sync_block(bytes, tickets, stream_, &key, out);
+    if (out->words) {
+        sync_held_ = true;
+        sync_sound_ = false;  // until the launch is made
+    }
+    return rc;
 }
 
 void Call::drop_result(void *ptr) {

@@ -34,6 +34,16 @@ namespace nacho {
         if (nacho_rc_ != NACHO_OK) return nacho_rc_;                                         \
     } while (0)
 
+// A block of 64-bit device words that only one family of kernels writes, kept between calls
+// and never cleared: `epoch` (>= 1, new for every use of the block; words start as zero) tags
+// what a launch stores, and `base` is the count the block's first word, a ticket counter
+// advanced by every use, starts from.
+struct SyncBlock {
+    unsigned long long *words;
+    unsigned epoch;
+    unsigned base;
+};
+
 // One call's execution context: its stream and allocator, and every buffer it allocated.
 // Scratch buffers are released when the call ends; result buffers are released only if the
 // call fails (commit() hands them to the caller).
@@ -64,6 +74,14 @@ class Call {
     int result_n(size_t count, T **out) {
         return result(count * sizeof(T), reinterpret_cast<void **>(out));
     }
+
+    // A sync block of at least `bytes` whose counter this call's next launch advances by
+    // `tickets`; kept for this stream's later calls.  words stays null where there is none to
+    // take (an arena call, or a caller's allocator, which the library keeps no memory of).
+    // sync_launched says that the launch was made: without it the block is dropped when the
+    // call ends.
+    int sync_block(size_t bytes, unsigned tickets, SyncBlock *out);
+    void sync_launched() { sync_sound_ = true; }
 
     // Release one result buffer early (e.g. an over-allocated array that turned out empty).
     void drop_result(void *ptr);
@@ -115,6 +133,7 @@ class Call {
     int64_t *arena_len_ = nullptr;
     int64_t *arena_side_ = nullptr;
     bool timed_ = false;
+    bool sync_held_ = false, sync_sound_ = true;
     bool len_marked_ = false;  // mark_length: this call launched the kernel storing its length
     float timed_ms_ = 0.0f;  // sum of this call's bracketed intervals
 };

@@ -108,3 +108,69 @@ def test_empty_operand(gpu, op, empty):
         *(nacho_amd.CSR_gpu(*(torch.from_numpy(x).to(gpu) for x in t), shape) for t in (a, b)))
     got = tuple(x.cpu().numpy() for x in (z.dim_j_offsets, z.dim_j_indices, z.values))
     assert_csr_equal(got, oracle.closed_csr_binary(op, 2, 5000, *a, *b), empty)
+
+
+@pytest.mark.parametrize("rows", [1, 230, 245, 500, 60_000, 62_500])
+def test_one_launch_limits(gpu, rows):
+    """One tile, two, and both sides of the tile count up to which a level is one launch."""
+    import nacho_amd
+
+    rng = np.random.default_rng(rows)
+    cols = 300_000
+    t = []
+    for _ in range(2):
+        keys = np.unique(rng.integers(0, rows * cols, size=8 * rows))
+        pos = np.zeros(rows + 1, np.int32)
+        pos[1:] = np.cumsum(np.bincount(keys // cols, minlength=rows))
+        t.append((pos, (keys % cols).astype(np.int32),
+                  rng.uniform(-1, 1, len(keys)).astype(np.float32)))
+    shape = torch.tensor([rows, cols], dtype=torch.int32)
+    ops = [nacho_amd.CSR_gpu(*(torch.from_numpy(x).to(gpu) for x in o), shape) for o in t]
+    for op in ("add", "mul", "add"):  # (the sync block is reused from call to call)
+        z = getattr(nacho_amd, f"gpu_csr_{op}_f32")(*ops)
+        got = tuple(x.cpu().numpy() for x in (z.dim_j_offsets, z.dim_j_indices, z.values))
+        assert_csr_equal(got, oracle.closed_csr_binary(op, rows, cols, *t[0], *t[1]), op)
+
+
+def test_one_launch_threads_and_streams(gpu):
+    """Threads on one stream and on streams of their own, with the cache given back between."""
+    import threading
+
+    import nacho_amd
+
+    rng = np.random.default_rng(3)
+    rows = cols = 4000
+    t = []
+    for _ in range(2):
+        keys = np.unique(rng.integers(0, rows * cols, size=40_000))
+        pos = np.zeros(rows + 1, np.int32)
+        pos[1:] = np.cumsum(np.bincount(keys // cols, minlength=rows))
+        t.append((pos, (keys % cols).astype(np.int32),
+                  rng.uniform(-1, 1, len(keys)).astype(np.float32)))
+    shape = torch.tensor([rows, cols], dtype=torch.int32)
+    ops = [nacho_amd.CSR_gpu(*(torch.from_numpy(x).to(gpu) for x in o), shape) for o in t]
+    torch.cuda.synchronize()
+    want = oracle.closed_csr_binary("add", rows, cols, *t[0], *t[1])
+    failures = []
+
+    def work(own_stream):
+        try:
+            stream = torch.cuda.Stream() if own_stream else torch.cuda.default_stream()
+            with torch.cuda.stream(stream):
+                for i in range(30):
+                    z = nacho_amd.gpu_csr_add_f32(*ops)
+                    if i % 10 == 9:
+                        stream.synchronize()
+                        got = tuple(x.cpu().numpy()
+                                    for x in (z.dim_j_offsets, z.dim_j_indices, z.values))
+                        assert_csr_equal(got, want, f"call {i}")
+                        nacho_amd.release_cached_memory()
+        except BaseException as e:  # noqa: BLE001
+            failures.append(e)
+
+    threads = [threading.Thread(target=work, args=(k % 2 == 1,)) for k in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not failures, failures[0]
