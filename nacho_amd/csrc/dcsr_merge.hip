@@ -78,12 +78,6 @@ __global__ void compact_rows_kernel(const int64_t *__restrict__ keep_off,
     }
 }
 
-// *dst = *src (a count computed on the device, into the call's side word, which the host
-// reads from pinned memory while the stream runs on).
-__global__ void store_count_kernel(const int64_t *__restrict__ src, int64_t *__restrict__ dst) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) dev::store_system(dst, *src);
-}
-
 static unsigned grid_for(long long n) {
     return static_cast<unsigned>((n + kBlock - 1) / kBlock > 0 ? (n + kBlock - 1) / kBlock : 1);
 }
@@ -164,9 +158,7 @@ int dcsr_binary(bool intersect, const nacho_dcsr *a, const nacho_dcsr *b, nacho_
                                                                  keep);
             NACHO_TRY_HIP(hipGetLastError());
         }
-        NACHO_TRY(scan::exclusive_scan_i64(call, keep, nu, keep_off));
-        store_count_kernel<<<1, 64, 0, s>>>(keep_off + nu, kept_dev);
-        NACHO_TRY_HIP(hipGetLastError());
+        NACHO_TRY(scan::exclusive_scan_i64(call, keep, nu, keep_off, kept_dev));
         NACHO_TRY(call.timer_stop());
         NACHO_TRY(call.collect_timer());  // (kernel timing only) before the j level's interval
         ja = ra;

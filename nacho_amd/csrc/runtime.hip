@@ -353,8 +353,8 @@ thread_local const char *t_last_name = "";
 // Pinned host word for length readbacks, one per host thread.
 thread_local void *t_pinned = nullptr;
 
-// Coherent pinned words that kernels store a length and a side count into (early readback)
-// and their device address; one pair per host thread.
+// Coherent pinned words that kernels store a length, a side count and Call::kValueWords values
+// into (early readback) and their device address; one block per host thread.
 thread_local volatile int64_t *t_len_host = nullptr;
 thread_local int64_t *t_len_dev = nullptr;
 
@@ -557,6 +557,19 @@ int Call::side_value(int64_t *v) {
         NACHO_TRY(spin_for_word(t_len_host + 1, stream_, v));
     }
     return *v < 0 ? NACHO_ERR_INTERNAL : NACHO_OK;
+}
+
+int Call::value_word(int i, int64_t **dev) {
+    if (arena_ || i < 0 || i >= kValueWords) return NACHO_ERR_INVALID_ARGUMENT;
+    NACHO_TRY(ensure_len_words());
+    t_len_host[2 + i] = -1;
+    *dev = t_len_dev + 2 + i;
+    return NACHO_OK;
+}
+
+int Call::value(int i, int64_t *v) {
+    if (arena_ || i < 0 || i >= kValueWords) return NACHO_ERR_INVALID_ARGUMENT;
+    return spin_for_word(t_len_host + 2 + i, stream_, v);
 }
 
 int Call::mark_length() {

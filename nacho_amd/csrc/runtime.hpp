@@ -108,6 +108,15 @@ class Call {
     int side_word(int64_t **dev);
     int side_value(int64_t *v);
 
+    // Further pinned words, for counts that size later steps: value_word(i) gives word i's
+    // device address (0 <= i < kValueWords) with the word reading "not stored", a queued
+    // kernel stores a value >= 0 to it (system scope), and value(i) waits for it as
+    // wait_length does.  A blocking copy of a count took about 15 us, this wait about 3.  Not
+    // for arena calls.
+    static constexpr int kValueWords = 6;
+    int value_word(int i, int64_t **dev);
+    int value(int i, int64_t *v);
+
     // Kernel timing hook (see nacho_set_kernel_timing): intervals between timer_start and
     // timer_stop are summed over the call and reported when the call ends.  An interval is
     // collected at the next read_back (which synchronises the stream).

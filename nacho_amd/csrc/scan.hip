@@ -1,7 +1,14 @@
-// Device-wide exclusive prefix sum of int64 counts (reduce, scan of block sums, scan) — the
-// 64-bit replacement for the CUB DeviceScan::InclusiveSum calls of the reference's generated
-// code (stitch_and_generate_gpu.cpp:412-446, 717-740), whose int32 counters overflow on the
+// Device-wide exclusive prefix sums of int64 counts — the 64-bit replacement for the CUB
+// DeviceScan::InclusiveSum calls of the reference's generated code
+// (stitch_and_generate_gpu.cpp:412-446, 717-740), whose int32 counters overflow on the
 // SpGEMM configuration (6.0e9 products).
+//
+// Two launches: every chunk's sum, then every chunk's scan, whose workgroup adds up the sums
+// of the chunks before its own (at most a few thousand words, read from L2) instead of waiting
+// for a launch that scans them, and whose last chunk stores the total.  Inputs of up to
+// kDirectChunks chunks need the second launch only: its workgroups add up the entries before
+// their own.  Against four launches (sums, their scan, chunks, total), or one of a single
+// workgroup up to 32,768 entries (10.8 us), 8 to 10 us less per scan on MI355X.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -15,13 +22,33 @@ namespace scan {
 constexpr int kBlock = 256;
 constexpr int kPerThread = 16;
 constexpr int kChunk = kBlock * kPerThread;
-constexpr int64_t kSmall = 8 * kChunk;  // scanned by one workgroup in one launch
+constexpr unsigned kDirectChunks = 4;  // a launch costs about as much as reading 3 chunks
 
-__global__ __launch_bounds__(kBlock) void block_sums_kernel(const int64_t *__restrict__ in,
-                                                            int64_t n,
+struct Jobs {
+    const int64_t *in[kMaxJobs];
+    int64_t *out[kMaxJobs];
+    int64_t *total[kMaxJobs];
+    int64_t n[kMaxJobs];
+    unsigned first[kMaxJobs + 1];  // first chunk of each job; [count] = all chunks
+    int count;
+};
+
+// The job of chunk `b`, and the chunk's number in it.
+__device__ __forceinline__ int job_of(const Jobs &jobs, unsigned b, unsigned &chunk) {
+    int j = 0;
+    while (j + 1 < jobs.count && b >= jobs.first[j + 1]) ++j;
+    chunk = b - jobs.first[j];
+    return j;
+}
+
+__global__ __launch_bounds__(kBlock) void chunk_sums_kernel(Jobs jobs,
                                                             int64_t *__restrict__ sums) {
     __shared__ int64_t s_wave[kBlock / dev::kWave];
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * kChunk;
+    unsigned chunk;
+    const int job = job_of(jobs, blockIdx.x, chunk);
+    const int64_t *__restrict__ in = jobs.in[job];
+    const int64_t n = jobs.n[job];
+    const int64_t base = static_cast<int64_t>(chunk) * kChunk;
     int64_t v = 0;
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j) {
@@ -33,55 +60,16 @@ __global__ __launch_bounds__(kBlock) void block_sums_kernel(const int64_t *__res
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-// One workgroup: exclusive scan of in[0, n) into out (in == out allowed), chunk by chunk with
-// a running carry; the total goes to *grand.
-template <int BLOCK>
-__device__ __forceinline__ void scan_one_workgroup(const int64_t *in, int64_t n, int64_t *out,
-                                                   int64_t *grand) {
-    constexpr int kStep = BLOCK * kPerThread;
-    __shared__ int64_t s_wave[BLOCK / dev::kWave];
-    int64_t carry = 0;
-    for (int64_t start = 0; start < n; start += kStep) {
-        int64_t v[kPerThread];
-        int64_t mine = 0;
-#pragma unroll
-        for (int j = 0; j < kPerThread; ++j) {
-            const int64_t i = start + static_cast<int64_t>(threadIdx.x) * kPerThread + j;
-            v[j] = i < n ? in[i] : 0;
-            mine += v[j];
-        }
-        int64_t total = 0;
-        int64_t run = carry + dev::block_exclusive_sum<BLOCK>(mine, s_wave, total);
-#pragma unroll
-        for (int j = 0; j < kPerThread; ++j) {
-            const int64_t i = start + static_cast<int64_t>(threadIdx.x) * kPerThread + j;
-            if (i < n) out[i] = run;
-            run += v[j];
-        }
-        carry += total;
-    }
-    if (threadIdx.x == 0) *grand = carry;
-}
-
-// Exclusive scan of the block sums in place; total to *grand.
-__global__ __launch_bounds__(kBlock) void scan_sums_kernel(int64_t *sums, int64_t nb,
-                                                           int64_t *__restrict__ grand) {
-    scan_one_workgroup<kBlock>(sums, nb, sums, grand);
-}
-
-// Short inputs in one launch of one wide workgroup: out[0, n) and out[n] = total.
-constexpr int kSmallBlock = 1024;
-__global__ __launch_bounds__(kSmallBlock) void scan_small_kernel(const int64_t *in, int64_t n,
-                                                                 int64_t *out) {
-    scan_one_workgroup<kSmallBlock>(in, n, out, out + n);
-}
-
-__global__ __launch_bounds__(kBlock) void scan_blocks_kernel(const int64_t *__restrict__ in,
-                                                             int64_t n,
-                                                             const int64_t *__restrict__ sums,
-                                                             int64_t *__restrict__ out) {
+// sums: the chunks' sums, or null (few chunks).
+__global__ __launch_bounds__(kBlock) void scan_chunks_kernel(Jobs jobs,
+                                                             const int64_t *__restrict__ sums) {
     __shared__ int64_t s_wave[kBlock / dev::kWave];
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * kChunk;
+    unsigned chunk;
+    const int job = job_of(jobs, blockIdx.x, chunk);
+    const int64_t *__restrict__ in = jobs.in[job];
+    int64_t *__restrict__ out = jobs.out[job];
+    const int64_t n = jobs.n[job];
+    const int64_t base = static_cast<int64_t>(chunk) * kChunk;
     // blocked arrangement: thread t owns elements [t*kPerThread, (t+1)*kPerThread)
     int64_t v[kPerThread];
     int64_t mine = 0;
@@ -91,44 +79,65 @@ __global__ __launch_bounds__(kBlock) void scan_blocks_kernel(const int64_t *__re
         v[j] = i < n ? in[i] : 0;
         mine += v[j];
     }
+    int64_t before = 0, carry = 0;
+    if (chunk > 0) {  // uniform
+        if (!sums) {
+#pragma unroll 8
+            for (int64_t i = threadIdx.x; i < base; i += kBlock) before += in[i];
+        } else {
+            for (unsigned c = threadIdx.x; c < chunk; c += kBlock) {
+                before += sums[jobs.first[job] + c];
+            }
+        }
+        (void)dev::block_exclusive_sum<kBlock>(before, s_wave, carry);
+    }
     int64_t total = 0;
-    int64_t run = sums[blockIdx.x] + dev::block_exclusive_sum<kBlock>(mine, s_wave, total);
+    int64_t run = carry + dev::block_exclusive_sum<kBlock>(mine, s_wave, total);
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j) {
         const int64_t i = base + static_cast<int64_t>(threadIdx.x) * kPerThread + j;
         if (i < n) out[i] = run;
         run += v[j];
     }
+    if (blockIdx.x + 1 == jobs.first[job + 1] && threadIdx.x == 0) {
+        out[n] = carry + total;
+        if (jobs.total[job]) dev::store_system(jobs.total[job], carry + total);
+    }
 }
 
-__global__ void copy_total_kernel(const int64_t *__restrict__ grand, int64_t *__restrict__ dst) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *dst = *grand;
-}
-
-int exclusive_scan_i64(Call &call, const int64_t *in, int64_t n, int64_t *out) {
+int exclusive_scans(Call &call, const Job *jobs, int count) {
+    if (count < 1 || count > kMaxJobs) return NACHO_ERR_INVALID_ARGUMENT;
+    Jobs j{};
+    j.count = count;
+    bool direct = true;  // every input is a few chunks
+    int64_t chunks = 0;
+    for (int k = 0; k < count; ++k) {
+        j.in[k] = jobs[k].in;
+        j.out[k] = jobs[k].out;
+        j.total[k] = jobs[k].total;
+        j.n[k] = jobs[k].n;
+        j.first[k] = static_cast<unsigned>(chunks);
+        const int64_t c = jobs[k].n > 0 ? (jobs[k].n + kChunk - 1) / kChunk : 1;
+        direct = direct && c <= kDirectChunks;
+        chunks += c;
+        if (chunks > INT32_MAX) return NACHO_ERR_INDEX_OVERFLOW;
+    }
+    j.first[count] = static_cast<unsigned>(chunks);
     const hipStream_t s = call.stream();
-    if (n <= kSmall) {  // one workgroup, one launch: launch latency dominates short scans
-        scan_small_kernel<<<1, kSmallBlock, 0, s>>>(in, n, out);
-        NACHO_TRY_HIP(hipGetLastError());
-        return NACHO_OK;
-    }
-    const int64_t nb = n > 0 ? (n + kChunk - 1) / kChunk : 0;
     int64_t *sums = nullptr;
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(nb) + 2, &sums));
-    int64_t *grand = sums + nb;
-    if (nb > 0) {
-        block_sums_kernel<<<static_cast<unsigned>(nb), kBlock, 0, s>>>(in, n, sums);
+    if (!direct) {
+        NACHO_TRY(call.scratch_n(static_cast<size_t>(chunks), &sums));
+        chunk_sums_kernel<<<static_cast<unsigned>(chunks), kBlock, 0, s>>>(j, sums);
         NACHO_TRY_HIP(hipGetLastError());
     }
-    scan_sums_kernel<<<1, kBlock, 0, s>>>(sums, nb, grand);
-    NACHO_TRY_HIP(hipGetLastError());
-    if (nb > 0) {
-        scan_blocks_kernel<<<static_cast<unsigned>(nb), kBlock, 0, s>>>(in, n, sums, out);
-        NACHO_TRY_HIP(hipGetLastError());
-    }
-    copy_total_kernel<<<1, 64, 0, s>>>(grand, out + n);
+    scan_chunks_kernel<<<static_cast<unsigned>(chunks), kBlock, 0, s>>>(j, sums);
     NACHO_TRY_HIP(hipGetLastError());
     return NACHO_OK;
+}
+
+int exclusive_scan_i64(Call &call, const int64_t *in, int64_t n, int64_t *out, int64_t *total) {
+    const Job job{in, n, out, total};
+    return exclusive_scans(call, &job, 1);
 }
 
 }  // namespace scan

@@ -9,8 +9,11 @@
 // count in int32, which the R-MAT scale-20 square (6.0e9 products, 3.6e9 results) overflows.
 //
 // Pipeline (every count and offset is int64):
-//   1. sizes: len[p] = |row crdA[p] of B| per A entry; exclusive scan -> off[p], P = off[nnzA];
-//      row i's products are [row_off[i], row_off[i+1]) in natural (j, k) order.
+//   1. sizes: a row's products are the lengths of its A entries' B rows; exclusive scan ->
+//      row_off, P: row i's products are [row_off[i], row_off[i+1]) in natural (j, k) order.
+//      (Small products are bound by launches and waits for counts: the scans of one step run
+//      together, counts reach the host through pinned words, and steps of long rows are
+//      skipped where there are none; 2^8 vertices 251 -> 129 us, 2^13 412 -> 316 us.)
 //   2. segments: a row with at most kShort products is one segment.  A longer row is split by
 //      column into nb buckets of 2^shift columns (one device-wide radix digit, k >> shift);
 //      each bucket is a segment.  Segments are numbered row-major, bucket-minor, so their
@@ -102,34 +105,70 @@ using dev::last_le;
 
 // ---- 1-2: sizes and segments -----------------------------------------------------------
 
-__global__ void lengths_kernel(const int *__restrict__ crd_a, int64_t nnz_a,
-                               const int *__restrict__ pos_b, int64_t *__restrict__ len) {
-    for (int64_t p = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; p < nnz_a;
-         p += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const int j = crd_a[p];
-        len[p] = static_cast<int64_t>(pos_b[j + 1] - pos_b[j]);
+// Per row of A: its products, the A entries whose B row is not empty, its segments (1, or nb
+// for a long row) and, for a long row, its work blocks of kBlock A entries.  Eight lanes per
+// row; a row of more than kWave entries (a hub) is taken by its whole wavefront.
+constexpr int kRowLanes = 8;
+__global__ __launch_bounds__(kBlock) void row_products_kernel(
+    const int *__restrict__ pos_a, const int *__restrict__ crd_a, int rows,
+    const int *__restrict__ pos_b, int nb, int64_t *__restrict__ products,
+    int *__restrict__ entries, int64_t *__restrict__ seg_count, int64_t *__restrict__ nblk) {
+    const int l = dev::lane();
+    const int64_t i = (blockIdx.x * static_cast<int64_t>(kBlock) + threadIdx.x) / kRowLanes;
+    const bool lead = l % kRowLanes == 0;
+    int s = 0, e = 0;
+    if (i < rows) {
+        s = pos_a[i];
+        e = pos_a[i + 1];
     }
-}
-
-// row_off[i] = off[posA[i]]; seg_count[i] = segments of row i (1, or nb for a long row).
-__global__ void rows_kernel(const int *__restrict__ pos_a, int rows,
-                            const int64_t *__restrict__ off, int nb,
-                            int64_t *__restrict__ row_off, int64_t *__restrict__ seg_count) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i <= rows; i += gridDim.x * blockDim.x) {
-        row_off[i] = off[pos_a[i]];
-        if (i < rows) {
-            const int64_t prod = off[pos_a[i + 1]] - off[pos_a[i]];
-            seg_count[i] = prod > kShort ? nb : 1;
-        }
+    auto add = [&](int p, int64_t &sum, int &some) {
+        const int j = crd_a[p];
+        const int len = pos_b[j + 1] - pos_b[j];
+        sum += len;
+        some += len > 0 ? 1 : 0;
+    };
+    auto store = [&](int64_t row, int first, int last, int64_t sum, int some) {
+        products[row] = sum;
+        entries[row] = some;
+        seg_count[row] = sum > kShort ? nb : 1;
+        nblk[row] = sum > kShort ? (last - first + kBlock - 1) / kBlock : 0;
+    };
+    const bool hub = e - s > dev::kWave;
+    int64_t sum = 0;
+    int some = 0;
+    if (!hub) {
+#pragma unroll 4
+        for (int p = s + l % kRowLanes; p < e; p += kRowLanes) add(p, sum, some);
+    }
+#pragma unroll
+    for (int d = kRowLanes / 2; d > 0; d >>= 1) {
+        sum += __shfl_xor(sum, d, dev::kWave);
+        some += __shfl_xor(some, d, dev::kWave);
+    }
+    if (lead && i < rows && !hub) store(i, s, e, sum, some);
+    unsigned long long hubs = __ballot(hub && lead);
+    while (hubs) {  // uniform
+        const int src = __ffsll(static_cast<long long>(hubs)) - 1;
+        hubs &= hubs - 1;
+        const int hs = __shfl(s, src, dev::kWave), he = __shfl(e, src, dev::kWave);
+        int64_t hsum = 0;
+        int hsome = 0;
+#pragma unroll 4
+        for (int p = hs + l; p < he; p += dev::kWave) add(p, hsum, hsome);
+        hsum = dev::wave_sum(hsum);
+        hsome = dev::wave_sum(hsome);
+        if (l == src) store(i, hs, he, hsum, hsome);
     }
 }
 
 // Segment table: row of each segment, product and run counts (short rows known now: one run
 // per A entry whose B row is not empty; long rows counted by the histogram pass) and the
-// zeroed fill counters of the long rows' run emission.
+// zeroed fill counters of the long rows' run emission.  blk_row[b] = the row of work block b
+// (kBlock consecutive A entries of one long row; blocks numbered by the scan blk_off).
 __global__ void segments_kernel(const int64_t *__restrict__ row_off,
                                 const int64_t *__restrict__ seg_prefix, int rows,
-                                const int *__restrict__ pos_a, const int64_t *__restrict__ len,
+                                const int *__restrict__ entries,
+                                const int64_t *__restrict__ blk_off, int *__restrict__ blk_row,
                                 int *__restrict__ seg_row, int64_t *__restrict__ seg_len,
                                 int64_t *__restrict__ seg_runs, int64_t *__restrict__ seg_fill) {
     // One row per lane; a long row's segments (one per column bucket) are then written by
@@ -144,9 +183,8 @@ __global__ void segments_kernel(const int64_t *__restrict__ row_off,
             s0 = seg_prefix[i];
             s1 = seg_prefix[i + 1];
             prod = row_off[i + 1] - row_off[i];
-            if (prod > 0 && prod <= kShort) {
-                for (int p = pos_a[i]; p < pos_a[i + 1]; ++p) runs += len[p] > 0 ? 1 : 0;
-            }
+            if (prod <= kShort) runs = entries[i];
+            for (int64_t b = blk_off[i]; b < blk_off[i + 1]; ++b) blk_row[b] = i;
             if (s1 - s0 == 1) {  // a short row's single segment
                 seg_row[s0] = i;
                 seg_len[s0] = prod > kShort ? 0 : prod;
@@ -180,13 +218,17 @@ __global__ void segments_kernel(const int64_t *__restrict__ row_off,
 // lengths.  At C4 (R-MAT 2^20, 128 buckets) this is 4.3e8 run visits instead of 5.9e9
 // products.
 
-// flag[p] = 1 where B entry p starts a run: its bucket differs from entry p - 1's.  Row
-// starts are flagged by run_row_starts_kernel, launched after this one.
-__global__ void run_flags_kernel(const int *__restrict__ crd_b, int64_t nnz_b, int shift,
-                                 int64_t *__restrict__ flag) {
+// B's columns and value bits as one array of pairs, read by the reduce units' gathers, and
+// (flag not null) flag[p] = 1 where B entry p starts a run: its bucket differs from entry
+// p - 1's.  Row starts are flagged by run_row_starts_kernel, launched after this one.
+__global__ void pairs_flags_kernel(const int *__restrict__ crd_b, const float *__restrict__ val_b,
+                                   int64_t nnz_b, int shift, int2 *__restrict__ cv_b,
+                                   int64_t *__restrict__ flag) {
     for (int64_t p = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; p < nnz_b;
          p += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        flag[p] = (p == 0 || (crd_b[p] >> shift) != (crd_b[p - 1] >> shift)) ? 1 : 0;
+        const int c = crd_b[p];
+        cv_b[p] = make_int2(c, __float_as_int(val_b[p]));
+        if (flag) flag[p] = (p == 0 || (c >> shift) != (crd_b[p - 1] >> shift)) ? 1 : 0;
     }
 }
 
@@ -221,25 +263,6 @@ __global__ void run_lengths_kernel(const int64_t *__restrict__ run_idx, int64_t 
     for (int64_t q = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; q < n_runs;
          q += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         run[q].y = run_start[q + 1] - run_start[q];
-    }
-}
-
-// Work blocks of the histogram: kBlock consecutive A entries of one long row.
-// nblk[i] = blocks of row i (0 for a short row).
-__global__ void hist_blocks_kernel(const int *__restrict__ pos_a, int rows,
-                                   const int64_t *__restrict__ row_off,
-                                   int64_t *__restrict__ nblk) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += gridDim.x * blockDim.x) {
-        const int len = pos_a[i + 1] - pos_a[i];
-        nblk[i] = row_off[i + 1] - row_off[i] > kShort ? (len + kBlock - 1) / kBlock : 0;
-    }
-}
-
-// blk_row[b] = the row of work block b (blocks numbered by the scan blk_off of nblk).
-__global__ void hist_rows_kernel(const int64_t *__restrict__ blk_off, int rows,
-                                 int *__restrict__ blk_row) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += gridDim.x * blockDim.x) {
-        for (int64_t b = blk_off[i]; b < blk_off[i + 1]; ++b) blk_row[b] = i;
     }
 }
 
@@ -351,15 +374,6 @@ __global__ __launch_bounds__(kBlock) void long_hist_kernel(
             }
         }
         __syncthreads();  // the histograms are read before the next block clears them
-    }
-}
-
-// B's columns and value bits as one array of pairs, read by the reduce units' gathers.
-__global__ void interleave_kernel(const int *__restrict__ crd_b, const float *__restrict__ val_b,
-                                  int64_t nnz_b, int2 *__restrict__ cv_b) {
-    for (int64_t p = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; p < nnz_b;
-         p += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        cv_b[p] = make_int2(crd_b[p], __float_as_int(val_b[p]));
     }
 }
 
@@ -633,14 +647,21 @@ __global__ void unit_map_kernel(const int64_t *__restrict__ seg_units,
 // cost (clearing and scanning its bitmap), so units of many small buckets are sorted
 // instead: at most kMaxBitmapBuckets nonempty buckets.  At C4 (units of about 2000
 // products) the limits 16 / 32 / 64 / 256 gave a call of 99.6 / 96.6 / 96.9 / 98.0 ms.
+// *units of the `bound` entries are units; the others' flags are cleared.
 __global__ void unit_bitmap_kernel(const int *__restrict__ unit_seg,
-                                   const int64_t *__restrict__ unit_dense, int64_t n_units,
+                                   int64_t *__restrict__ unit_dense,
+                                   const int64_t *__restrict__ units, int64_t bound,
                                    int64_t n_seg, const int64_t *__restrict__ seg_len,
                                    const int *__restrict__ seg_row,
                                    const int64_t *__restrict__ row_off, bool narrow_buckets,
                                    int64_t *__restrict__ unit_bitmap) {
-    for (int64_t u = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; u < n_units;
+    const int64_t n_units = *units;
+    for (int64_t u = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; u < bound;
          u += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+        if (u >= n_units) {
+            unit_dense[u] = unit_bitmap[u] = 0;
+            continue;
+        }
         const int64_t s0 = unit_seg[u];
         const int64_t s1 = u + 1 < n_units ? unit_seg[u + 1] : n_seg;
         bool ok = narrow_buckets && !unit_dense[u] && s1 - s0 <= kMaxBitmapSegs;
@@ -1675,6 +1696,16 @@ int col_bits(int cols) {
     return b;
 }
 
+// Workgroups of the long rows' kernels, which stride over their work blocks.
+unsigned long_grid(int64_t blocks) {
+    return static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(blocks, kHistGrid)));
+}
+
+// At most this many products (64 MB of run descriptors) or segments are taken as the bound of
+// the runs or units; more are counted, which costs a wait of the host for the device.
+constexpr int64_t kBoundRuns = int64_t{1} << 22;
+constexpr int64_t kBoundUnits = int64_t{1} << 18;
+
 // How the result is sized.  Staged: the reduce units write their distinct entries at their
 // units' product offsets in a staging buffer of 8 bytes per product, and a copy moves them
 // into the result once every unit's count is known.  Symbolic: the symbolic pass counts
@@ -1692,6 +1723,7 @@ Output output_mode(int64_t products, bool symbolic_fits) {
     if (v != nullptr && std::strcmp(v, "staged") == 0) return Output::Staged;
     if (!symbolic_fits) return Output::Staged;
     if (v != nullptr && std::strcmp(v, "symbolic") == 0) return Output::Symbolic;
+    if (products <= kBoundRuns) return Output::Staged;  // 32 MB: not worth asking
     size_t free_bytes = 0, total_bytes = 0;
     if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) return Output::Symbolic;
     const double room = (static_cast<double>(free_bytes) + static_cast<double>(nacho_cached_bytes())) / 2;
@@ -1713,7 +1745,6 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
     const hipStream_t st = call.stream();
     const int rows = a->dim_i_size;
     const int cols = b->dim_j_size;
-    const int64_t nnz_a = a->dim_j_length;
     const int cb = col_bits(cols);
     // one radix digit over the columns: buckets of 2^shift columns, at most kMaxBuckets
     const int shift = std::max(std::min(kDenseBits, cb), cb - kMaxBucketBits);
@@ -1722,29 +1753,43 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
     const char *name = "spgemm: runs+reduce+output";
     NACHO_TRY(call.timer_start(name));
 
-    // 1-2. products per A entry, per row; segments per row
-    int64_t *len = nullptr, *off = nullptr, *row_off = nullptr, *seg_count = nullptr;
-    int64_t *seg_prefix = nullptr;
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_a) + 1, &len));
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_a) + 1, &off));
+    // 1-2. products, segments and long-row work blocks per row
+    int64_t *per_row = nullptr, *row_off = nullptr, *seg_prefix = nullptr, *blk_off = nullptr;
+    int *entries = nullptr;
+    NACHO_TRY(call.scratch_n(3 * (static_cast<size_t>(rows) + 1), &per_row));
+    NACHO_TRY(call.scratch_n(static_cast<size_t>(rows) + 1, &entries));
     NACHO_TRY(call.scratch_n(static_cast<size_t>(rows) + 1, &row_off));
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(rows) + 1, &seg_count));
     NACHO_TRY(call.scratch_n(static_cast<size_t>(rows) + 1, &seg_prefix));
-    if (nnz_a > 0) {
-        lengths_kernel<<<grid_for(nnz_a, 256), 256, 0, st>>>(a->dim_j_indices, nnz_a,
-                                                             b->dim_j_offsets, len);
+    NACHO_TRY(call.scratch_n(static_cast<size_t>(rows) + 1, &blk_off));
+    int64_t *products = per_row, *seg_count = per_row + (rows + 1),
+            *nblk = per_row + 2 * (static_cast<size_t>(rows) + 1);
+    if (rows > 0) {
+        const int64_t blocks = (static_cast<int64_t>(rows) * kRowLanes + kBlock - 1) / kBlock;
+        row_products_kernel<<<static_cast<unsigned>(blocks), kBlock, 0, st>>>(
+            a->dim_j_offsets, a->dim_j_indices, rows, b->dim_j_offsets, nb, products, entries,
+            seg_count, nblk);
         NACHO_TRY_HIP(hipGetLastError());
     }
-    NACHO_TRY(scan::exclusive_scan_i64(call, len, nnz_a, off));
-    rows_kernel<<<grid_for(static_cast<int64_t>(rows) + 1, 256), 256, 0, st>>>(
-        a->dim_j_offsets, rows, off, nb, row_off, seg_count);
-    NACHO_TRY_HIP(hipGetLastError());
-    NACHO_TRY(scan::exclusive_scan_i64(call, seg_count, rows, seg_prefix));
-    int64_t P = 0, n_seg = 0;
-    NACHO_TRY(call.timer_stop());
-    NACHO_TRY(call.read_back(&P, row_off + rows, sizeof(P)));
-    NACHO_TRY(call.read_back(&n_seg, seg_prefix + rows, sizeof(n_seg)));
-    NACHO_TRY(call.timer_start(name));
+    int64_t *word[3] = {nullptr, nullptr, nullptr};  // counts read back on the way
+    auto words = [&](int n) {
+        for (int i = 0; i < n; ++i) NACHO_TRY(call.value_word(i, &word[i]));
+        return static_cast<int>(NACHO_OK);
+    };
+    // The n words' values, once the kernels queued so far have stored them.
+    auto values = [&](int n, int64_t *v) {
+        NACHO_TRY(call.timer_stop());
+        for (int i = 0; i < n; ++i) NACHO_TRY(call.value(i, v + i));
+        NACHO_TRY(call.collect_timer());
+        return call.timer_start(name);
+    };
+    NACHO_TRY(words(3));
+    const scan::Job row_jobs[3] = {{products, rows, row_off, word[0]},
+                                   {seg_count, rows, seg_prefix, word[1]},
+                                   {nblk, rows, blk_off, word[2]}};
+    NACHO_TRY(scan::exclusive_scans(call, row_jobs, 3));
+    int64_t counts3[3] = {0, 0, 0};
+    NACHO_TRY(values(3, counts3));
+    const int64_t P = counts3[0], n_seg = counts3[1], n_blk = counts3[2];
     if (n_seg >= INT_MAX) return NACHO_ERR_INDEX_OVERFLOW;  // segment ids are int32
     const bool symbolic =
         P > 0 && output_mode(P, cb <= kSymColBits &&
@@ -1768,9 +1813,11 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
         NACHO_TRY(call.scratch_n(static_cast<size_t>(n_seg), &seg_fill));
         NACHO_TRY(call.scratch_n(static_cast<size_t>(n_seg) + 1, &seg_runs));
         NACHO_TRY(call.scratch_n(static_cast<size_t>(n_seg) + 1, &seg_roff));
-        segments_kernel<<<grid_for(rows, 256), 256, 0, st>>>(row_off, seg_prefix, rows,
-                                                            a->dim_j_offsets, len, seg_row,
-                                                            seg_len, seg_runs, seg_fill);
+        int *blk_row = nullptr;
+        NACHO_TRY(call.scratch_n(static_cast<size_t>(n_blk) + 1, &blk_row));
+        segments_kernel<<<grid_for(rows, 256), 256, 0, st>>>(row_off, seg_prefix, rows, entries,
+                                                            blk_off, blk_row, seg_row, seg_len,
+                                                            seg_runs, seg_fill);
         NACHO_TRY_HIP(hipGetLastError());
 
         // symbolic pass: distinct columns per segment, scanned into result offsets
@@ -1820,56 +1867,50 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
         // long rows' bucket counts from B's runs (P > 0, so B has entries)
         const int64_t nnz_b = b->dim_j_length;
         const int rows_b = b->dim_i_size;
+        int2 *cv_b = nullptr;
+        NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b), &cv_b));
         int64_t *flag = nullptr, *run_idx = nullptr;
         int2 *run = nullptr;
         int *run_start = nullptr;
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b) + 1, &flag));
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b) + 1, &run_idx));
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b), &run));
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b) + 1, &run_start));
-        run_flags_kernel<<<grid_for(nnz_b, 256), 256, 0, st>>>(b->dim_j_indices, nnz_b, shift,
-                                                               flag);
+        if (n_blk > 0) {
+            NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b) + 1, &flag));
+            NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b) + 1, &run_idx));
+            NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b), &run));
+            NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b) + 1, &run_start));
+        }
+        pairs_flags_kernel<<<grid_for(nnz_b, 256), 256, 0, st>>>(b->dim_j_indices, b->values,
+                                                                 nnz_b, shift, cv_b, flag);
         NACHO_TRY_HIP(hipGetLastError());
-        if (rows_b > 0) {
+        const BRuns br{run_idx, run, run_start};
+        if (n_blk > 0) {
             run_row_starts_kernel<<<grid_for(rows_b, 256), 256, 0, st>>>(b->dim_j_offsets,
                                                                           rows_b, flag);
             NACHO_TRY_HIP(hipGetLastError());
+            NACHO_TRY(scan::exclusive_scan_i64(call, flag, nnz_b, run_idx));
+            runs_kernel<<<grid_for(nnz_b, 256), 256, 0, st>>>(b->dim_j_indices, nnz_b, shift,
+                                                              flag, run_idx, run, run_start);
+            NACHO_TRY_HIP(hipGetLastError());
+            run_lengths_kernel<<<grid_for(nnz_b, 256), 256, 0, st>>>(run_idx, nnz_b, run_start,
+                                                                     run);
+            NACHO_TRY_HIP(hipGetLastError());
+            long_hist_kernel<<<long_grid(n_blk), kBlock, 0, st>>>(
+                a->dim_j_offsets, a->dim_j_indices, blk_off, blk_row, rows, b->dim_j_offsets, br,
+                nb, seg_prefix, seg_len, seg_runs);
+            NACHO_TRY_HIP(hipGetLastError());
         }
-        NACHO_TRY(scan::exclusive_scan_i64(call, flag, nnz_b, run_idx));
-        runs_kernel<<<grid_for(nnz_b, 256), 256, 0, st>>>(b->dim_j_indices, nnz_b, shift, flag,
-                                                          run_idx, run, run_start);
-        NACHO_TRY_HIP(hipGetLastError());
-        run_lengths_kernel<<<grid_for(nnz_b, 256), 256, 0, st>>>(run_idx, nnz_b, run_start, run);
-        NACHO_TRY_HIP(hipGetLastError());
-        int2 *cv_b = nullptr;
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b), &cv_b));
-        interleave_kernel<<<grid_for(nnz_b, 256), 256, 0, st>>>(b->dim_j_indices, b->values,
-                                                                nnz_b, cv_b);
-        NACHO_TRY_HIP(hipGetLastError());
-        int64_t *nblk = nullptr, *blk_off = nullptr;
-        int *blk_row = nullptr;
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(rows) + 1, &nblk));
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(rows) + 1, &blk_off));
-        // at most one block per kBlock entries of A, plus one per row
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_a / kBlock + rows + 1), &blk_row));
-        hist_blocks_kernel<<<grid_for(rows, 256), 256, 0, st>>>(a->dim_j_offsets, rows, row_off,
-                                                               nblk);
-        NACHO_TRY_HIP(hipGetLastError());
-        NACHO_TRY(scan::exclusive_scan_i64(call, nblk, rows, blk_off));
-        hist_rows_kernel<<<grid_for(rows, 256), 256, 0, st>>>(blk_off, rows, blk_row);
-        NACHO_TRY_HIP(hipGetLastError());
-        const BRuns br{run_idx, run, run_start};
-        long_hist_kernel<<<kHistGrid, kBlock, 0, st>>>(
-            a->dim_j_offsets, a->dim_j_indices, blk_off, blk_row, rows, b->dim_j_offsets, br,
-            nb, seg_prefix, seg_len, seg_runs);
-        NACHO_TRY_HIP(hipGetLastError());
-        NACHO_TRY(scan::exclusive_scan_i64(call, seg_len, n_seg, seg_off));
-        NACHO_TRY(scan::exclusive_scan_i64(call, seg_runs, n_seg, seg_roff));
-        int64_t n_runs = 0, nnz_sym = 0;
-        NACHO_TRY(call.timer_stop());
-        NACHO_TRY(call.read_back(&n_runs, seg_roff + n_seg, sizeof(n_runs)));
+        // A product lies in one run: few products bound the runs without waiting for their
+        // count.
+        int64_t n_runs = P, nnz_sym = 0;
+        const bool count_runs = P > kBoundRuns;
+        NACHO_TRY(words(1));
+        const scan::Job seg_jobs[2] = {{seg_len, n_seg, seg_off},
+                                       {seg_runs, n_seg, seg_roff, count_runs ? word[0] : nullptr}};
+        NACHO_TRY(scan::exclusive_scans(call, seg_jobs, 2));
+        if (count_runs) NACHO_TRY(values(1, &n_runs));
         if (symbolic) {
+            NACHO_TRY(call.timer_stop());
             NACHO_TRY(call.read_back(&nnz_sym, seg_out + n_seg, sizeof(nnz_sym)));
+            NACHO_TRY(call.timer_start(name));
             if (sizeof(PosT) == sizeof(int32_t) && nnz_sym > INT_MAX) {
                 return NACHO_ERR_INDEX_OVERFLOW;
             }
@@ -1878,13 +1919,14 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
             ukey = z->crd;
             uval = z->val;
         }
-        NACHO_TRY(call.timer_start(name));
         int4 *desc = nullptr;
         NACHO_TRY(call.scratch_n(static_cast<size_t>(std::max<int64_t>(n_runs, 1)), &desc));
-        long_runs_kernel<<<kHistGrid, kBlock, 0, st>>>(
-            a->dim_j_offsets, a->dim_j_indices, a->values, blk_off, blk_row, rows,
-            b->dim_j_offsets, br, nb, seg_prefix, seg_roff, seg_fill, desc);
-        NACHO_TRY_HIP(hipGetLastError());
+        if (n_blk > 0) {
+            long_runs_kernel<<<long_grid(n_blk), kBlock, 0, st>>>(
+                a->dim_j_offsets, a->dim_j_indices, a->values, blk_off, blk_row, rows,
+                b->dim_j_offsets, br, nb, seg_prefix, seg_roff, seg_fill, desc);
+            NACHO_TRY_HIP(hipGetLastError());
+        }
         short_runs_kernel<<<grid_for(rows, 256), 256, 0, st>>>(
             a->dim_j_offsets, a->dim_j_indices, a->values, rows, row_off, seg_prefix, seg_roff,
             b->dim_j_offsets, desc);
@@ -1897,42 +1939,46 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
         unit_count_kernel<<<grid_for(n_seg, 256), 256, 0, st>>>(
             seg_len, seg_off, n_seg, seg_row, row_off, dense_min, seg_units);
         NACHO_TRY_HIP(hipGetLastError());
-        NACHO_TRY(scan::exclusive_scan_i64(call, seg_units, n_seg, unit_prefix));
-        NACHO_TRY(call.timer_stop());
-        NACHO_TRY(call.read_back(&n_units, unit_prefix + n_seg, sizeof(n_units)));
-        NACHO_TRY(call.timer_start(name));
-        if (n_units > INT_MAX) return NACHO_ERR_INDEX_OVERFLOW;
+        NACHO_TRY(words(3));
+        NACHO_TRY(scan::exclusive_scan_i64(call, seg_units, n_seg, unit_prefix, word[0]));
+        // (a unit starts at a segment: few segments bound the units without waiting)
+        int64_t bound = n_seg;
+        const bool count_units = n_seg > kBoundUnits;
+        if (count_units) {
+            NACHO_TRY(values(1, &bound));
+            if (bound > INT_MAX) return NACHO_ERR_INDEX_OVERFLOW;
+        }
         int *unit_seg = nullptr;
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(n_units), &unit_seg));
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(n_units) + 1, &unit_start));
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(n_units) + 1, &unit_nnz));
-        NACHO_TRY(call.scratch_n(static_cast<size_t>(n_units) + 1, &unit_out));
+        NACHO_TRY(call.scratch_n(static_cast<size_t>(bound), &unit_seg));
+        NACHO_TRY(call.scratch_n(static_cast<size_t>(bound) + 1, &unit_start));
+        NACHO_TRY(call.scratch_n(static_cast<size_t>(bound) + 1, &unit_nnz));
+        NACHO_TRY(call.scratch_n(static_cast<size_t>(bound) + 1, &unit_out));
         int *lists = nullptr;  // dense list, bitmap list, sort list
         int64_t *kinds = nullptr;  // dense flags, their ranks, bitmap flags, their ranks
-        NACHO_TRY(call.scratch_n(3 * static_cast<size_t>(n_units), &lists));
-        NACHO_TRY(call.scratch_n(4 * (static_cast<size_t>(n_units) + 1), &kinds));
-        int64_t *unit_dense = kinds, *dense_rank = kinds + (n_units + 1);
-        int64_t *unit_bitmap = kinds + 2 * (n_units + 1), *bitmap_rank = kinds + 3 * (n_units + 1);
-        int *dense_list = lists, *bitmap_list = lists + n_units, *sort_list = lists + 2 * n_units;
+        NACHO_TRY(call.scratch_n(3 * static_cast<size_t>(bound), &lists));
+        NACHO_TRY(call.scratch_n(4 * (static_cast<size_t>(bound) + 1), &kinds));
+        int64_t *unit_dense = kinds, *dense_rank = kinds + (bound + 1);
+        int64_t *unit_bitmap = kinds + 2 * (bound + 1), *bitmap_rank = kinds + 3 * (bound + 1);
+        int *dense_list = lists, *bitmap_list = lists + bound, *sort_list = lists + 2 * bound;
         unit_map_kernel<<<grid_for(n_seg + 1, 256), 256, 0, st>>>(
             seg_units, unit_prefix, seg_off, seg_len, seg_row, row_off, dense_min, n_seg, P,
             unit_seg, unit_start, unit_dense);
         NACHO_TRY_HIP(hipGetLastError());
-        unit_bitmap_kernel<<<grid_for(n_units, 256), 256, 0, st>>>(
-            unit_seg, unit_dense, n_units, n_seg, seg_len, seg_row, row_off, shift <= kDenseBits,
-            unit_bitmap);
+        unit_bitmap_kernel<<<grid_for(bound, 256), 256, 0, st>>>(
+            unit_seg, unit_dense, unit_prefix + n_seg, bound, n_seg, seg_len, seg_row, row_off,
+            shift <= kDenseBits, unit_bitmap);
         NACHO_TRY_HIP(hipGetLastError());
-        NACHO_TRY(scan::exclusive_scan_i64(call, unit_dense, n_units, dense_rank));
-        NACHO_TRY(scan::exclusive_scan_i64(call, unit_bitmap, n_units, bitmap_rank));
+        const scan::Job kind_jobs[2] = {{unit_dense, bound, dense_rank, word[1]},
+                                        {unit_bitmap, bound, bitmap_rank, word[2]}};
+        NACHO_TRY(scan::exclusive_scans(call, kind_jobs, 2));
+        int64_t kinds3[3] = {0, 0, 0};
+        NACHO_TRY(values(3, kinds3));
+        n_units = kinds3[0];
+        const int64_t n_dense = kinds3[1], n_bitmap = kinds3[2];
         unit_lists_kernel<<<grid_for(n_units, 256), 256, 0, st>>>(
             unit_dense, dense_rank, unit_bitmap, bitmap_rank, n_units, dense_list, bitmap_list,
             sort_list);
         NACHO_TRY_HIP(hipGetLastError());
-        int64_t n_dense = 0, n_bitmap = 0;
-        NACHO_TRY(call.timer_stop());
-        NACHO_TRY(call.read_back(&n_dense, dense_rank + n_units, sizeof(n_dense)));
-        NACHO_TRY(call.read_back(&n_bitmap, bitmap_rank + n_units, sizeof(n_bitmap)));
-        NACHO_TRY(call.timer_start(name));
         const int n_kind[3] = {static_cast<int>(n_dense),
                                static_cast<int>(n_units - n_dense - n_bitmap),
                                static_cast<int>(n_bitmap)};
@@ -1967,12 +2013,11 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
         if (symbolic) {
             z->nnz = nnz_sym;  // the units wrote straight into the result
         } else {
-            NACHO_TRY(scan::exclusive_scan_i64(call, unit_nnz, n_units, unit_out));
+            NACHO_TRY(words(1));
+            NACHO_TRY(scan::exclusive_scan_i64(call, unit_nnz, n_units, unit_out, word[0]));
             int64_t nnz = 0;
-            NACHO_TRY(call.timer_stop());
-            NACHO_TRY(call.read_back(&nnz, unit_out + n_units, sizeof(nnz)));
+            NACHO_TRY(values(1, &nnz));
             if (sizeof(PosT) == sizeof(int32_t) && nnz > INT_MAX) return NACHO_ERR_INDEX_OVERFLOW;
-            NACHO_TRY(call.timer_start(name));
 
             // 6. output
             NACHO_TRY(call.result_n(static_cast<size_t>(nnz), &z->crd));

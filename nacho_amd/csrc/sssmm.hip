@@ -106,17 +106,12 @@ __global__ void fill_kernel(uint64_t *__restrict__ p, int64_t n, uint64_t v) {
     }
 }
 
-__global__ void zero_kernel(int64_t *__restrict__ p, int64_t n) {
+// The mask entries' sums and hit flags, zeroed.
+__global__ void zero_sums_kernel(double *__restrict__ acc, int *__restrict__ hit, int64_t n) {
     for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
          i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        p[i] = 0;
-    }
-}
-
-__global__ void zero_int_kernel(int *__restrict__ p, int64_t n) {
-    for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        p[i] = 0;
+        acc[i] = 0.0;
+        hit[i] = 0;
     }
 }
 
@@ -158,14 +153,14 @@ __device__ __forceinline__ int64_t table_size(int64_t len) {
     return s;
 }
 
-// size[x] for the n lists; lengths from an offsets array (pos, n + 1 entries, int32) or from
-// counts (int64).
-__global__ void table_sizes_kernel(const int *__restrict__ pos, const int64_t *__restrict__ count,
-                                   int n, int64_t *__restrict__ size) {
-    for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < n; x += gridDim.x * blockDim.x) {
-        const int64_t len = pos ? static_cast<int64_t>(pos[x + 1] - pos[x]) : count[x];
-        size[x] = table_size(len);
-    }
+// Table sizes of B's columns (lengths `count`) and of A's rows (offsets `pos`).
+__global__ void table_sizes_kernel(const int64_t *__restrict__ count, int cols,
+                                   int64_t *__restrict__ size_b, const int *__restrict__ pos,
+                                   int rows, int64_t *__restrict__ size_a) {
+    const int stride = gridDim.x * blockDim.x;
+    const int first = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int x = first; x < cols; x += stride) size_b[x] = table_size(count[x]);
+    for (int x = first; x < rows; x += stride) size_a[x] = table_size(pos[x + 1] - pos[x]);
 }
 
 // Workgroup b takes entries [lo, hi) = [b*kSpan, (b+1)*kSpan) of a list split by the offsets
@@ -484,31 +479,35 @@ int multiply(const nacho_csr *a, const nacho_csr *b, const nacho_csr *c, nacho_c
     // columns of B and the table sizes
     int64_t *col_count = nullptr, *col_off = nullptr, *col_fill = nullptr;
     int64_t *tsize_b = nullptr, *toff_b = nullptr, *tsize_a = nullptr, *toff_a = nullptr;
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(cols) + 1, &col_count));
+    NACHO_TRY(call.scratch_n(2 * (static_cast<size_t>(cols) + 1), &col_count));
     NACHO_TRY(call.scratch_n(static_cast<size_t>(cols) + 1, &col_off));
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(cols) + 1, &col_fill));
+    col_fill = col_count + cols + 1;
     NACHO_TRY(call.scratch_n(static_cast<size_t>(cols) + 1, &tsize_b));
     NACHO_TRY(call.scratch_n(static_cast<size_t>(cols) + 1, &toff_b));
     NACHO_TRY(call.scratch_n(static_cast<size_t>(rows) + 1, &tsize_a));
     NACHO_TRY(call.scratch_n(static_cast<size_t>(rows) + 1, &toff_a));
-    zero_kernel<<<grid_for(cols), kBlock, 0, st>>>(col_count, cols);
-    zero_kernel<<<grid_for(cols), kBlock, 0, st>>>(col_fill, cols);
+    fill_kernel<<<grid_for(2 * (static_cast<int64_t>(cols) + 1)), kBlock, 0, st>>>(
+        reinterpret_cast<uint64_t *>(col_count), 2 * (static_cast<int64_t>(cols) + 1), 0ull);
     const unsigned span_grid =
         static_cast<unsigned>(std::max<int64_t>(1, (nnz_b + kSpan - 1) / kSpan));
     count_cols_kernel<<<span_grid, kBlock, 0, st>>>(
         b->dim_j_indices, nnz_b, cols, reinterpret_cast<unsigned long long *>(col_count));
     NACHO_TRY_HIP(hipGetLastError());
-    NACHO_TRY(scan::exclusive_scan_i64(call, col_count, cols, col_off));
-    table_sizes_kernel<<<grid_for(cols), kBlock, 0, st>>>(nullptr, col_count, cols, tsize_b);
-    table_sizes_kernel<<<grid_for(rows), kBlock, 0, st>>>(a->dim_j_offsets, nullptr, rows,
-                                                          tsize_a);
+    table_sizes_kernel<<<grid_for(std::max(cols, rows)), kBlock, 0, st>>>(
+        col_count, cols, tsize_b, a->dim_j_offsets, rows, tsize_a);
     NACHO_TRY_HIP(hipGetLastError());
-    NACHO_TRY(scan::exclusive_scan_i64(call, tsize_b, cols, toff_b));
-    NACHO_TRY(scan::exclusive_scan_i64(call, tsize_a, rows, toff_a));
+    int64_t *word[2] = {nullptr, nullptr};
+    NACHO_TRY(call.value_word(0, &word[0]));
+    NACHO_TRY(call.value_word(1, &word[1]));
+    const scan::Job size_jobs[3] = {{tsize_b, cols, toff_b, word[0]},
+                                    {tsize_a, rows, toff_a, word[1]},
+                                    {col_count, cols, col_off}};
+    NACHO_TRY(scan::exclusive_scans(call, size_jobs, 3));
     NACHO_TRY(call.timer_stop());
     int64_t sizes[2] = {0, 0};
-    NACHO_TRY(call.read_back(&sizes[0], toff_b + cols, sizeof(int64_t)));
-    NACHO_TRY(call.read_back(&sizes[1], toff_a + rows, sizeof(int64_t)));
+    NACHO_TRY(call.value(0, &sizes[0]));
+    NACHO_TRY(call.value(1, &sizes[1]));
+    NACHO_TRY(call.collect_timer());
     // A table's mask is kept in 31 bits (bit 31 flags the walked side), so no table may
     // exceed 2^31 slots.  Table sizes are powers of two, so a larger one (2^32 slots or
     // more, for a row or column of more than 2^30 entries) would make its side's total at
@@ -522,12 +521,12 @@ int multiply(const nacho_csr *a, const nacho_csr *b, const nacho_csr *c, nacho_c
     uint64_t *tab_b = nullptr, *tab_a = nullptr;
     int *csc_row = nullptr;
     float *csc_val = nullptr;
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(sizes[0]), &tab_b));
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(sizes[1]), &tab_a));
+    NACHO_TRY(call.scratch_n(static_cast<size_t>(sizes[0] + sizes[1]), &tab_b));
+    tab_a = tab_b + sizes[0];
     NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b), &csc_row));
     NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b), &csc_val));
-    fill_kernel<<<grid_for(sizes[0]), kBlock, 0, st>>>(tab_b, sizes[0], kEmptySlot);
-    fill_kernel<<<grid_for(sizes[1]), kBlock, 0, st>>>(tab_a, sizes[1], kEmptySlot);
+    fill_kernel<<<grid_for(sizes[0] + sizes[1]), kBlock, 0, st>>>(tab_b, sizes[0] + sizes[1],
+                                                                  kEmptySlot);
     transpose_kernel<<<span_grid, kBlock, 0, st>>>(
         b->dim_j_offsets, inner, b->dim_j_indices, b->values, nnz_b, col_off,
         reinterpret_cast<unsigned long long *>(col_fill), toff_b, csc_row, csc_val, tab_b);
@@ -549,22 +548,24 @@ int multiply(const nacho_csr *a, const nacho_csr *b, const nacho_csr *c, nacho_c
         reinterpret_cast<const unsigned long long *>(col_count), col_off, toff_a, toff_b, work,
         walk_base, probe_base, probe_mask);
     NACHO_TRY_HIP(hipGetLastError());
-    NACHO_TRY(scan::exclusive_scan_i64(call, work, nnz_c, woff));
+    NACHO_TRY(call.value_word(0, &word[0]));
+    NACHO_TRY(scan::exclusive_scan_i64(call, work, nnz_c, woff, word[0]));
+    // (queued ahead of the wait for the probes' number)
+    double *acc = nullptr;
+    int *hit = nullptr;
+    NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_c), &acc));
+    NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_c), &hit));
+    zero_sums_kernel<<<grid_for(nnz_c), kBlock, 0, st>>>(acc, hit, nnz_c);
+    NACHO_TRY_HIP(hipGetLastError());
     NACHO_TRY(call.timer_stop());
     int64_t total = 0;
-    NACHO_TRY(call.read_back(&total, woff + nnz_c, sizeof(total)));
+    NACHO_TRY(call.value(0, &total));
+    NACHO_TRY(call.collect_timer());
     NACHO_TRY(call.timer_start(name));
     const int64_t chunks = (total + kChunk - 1) / kChunk;
     if (chunks > INT_MAX) return NACHO_ERR_INDEX_OVERFLOW;
 
     // probes
-    double *acc = nullptr;
-    int *hit = nullptr;
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_c), &acc));
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_c), &hit));
-    fill_kernel<<<grid_for(nnz_c), kBlock, 0, st>>>(reinterpret_cast<uint64_t *>(acc), nnz_c, 0ull);
-    zero_int_kernel<<<grid_for(nnz_c), kBlock, 0, st>>>(hit, nnz_c);
-    NACHO_TRY_HIP(hipGetLastError());
     if (chunks > 0) {
         int64_t *bounds = nullptr;
         NACHO_TRY(call.scratch_n(2 * static_cast<size_t>(chunks), &bounds));
@@ -580,10 +581,12 @@ int multiply(const nacho_csr *a, const nacho_csr *b, const nacho_csr *c, nacho_c
     int64_t *keep = work, *koff = woff;  // the work counts are spent
     keep_kernel<<<grid_for(nnz_c), kBlock, 0, st>>>(hit, nnz_c, keep);
     NACHO_TRY_HIP(hipGetLastError());
-    NACHO_TRY(scan::exclusive_scan_i64(call, keep, nnz_c, koff));
+    NACHO_TRY(call.value_word(0, &word[0]));
+    NACHO_TRY(scan::exclusive_scan_i64(call, keep, nnz_c, koff, word[0]));
     NACHO_TRY(call.timer_stop());
     int64_t nnz = 0;
-    NACHO_TRY(call.read_back(&nnz, koff + nnz_c, sizeof(nnz)));
+    NACHO_TRY(call.value(0, &nnz));
+    NACHO_TRY(call.collect_timer());
     NACHO_TRY(call.timer_start(name));
     int *cz = nullptr;
     float *vz = nullptr;
