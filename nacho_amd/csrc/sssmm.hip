@@ -24,14 +24,14 @@
 //   chunk_bounds_kernel              first / last mask entry of every 4096-probe chunk
 //   probe_kernel                     one chunk per workgroup: load-balanced decode of probes
 //                                    to mask entries (max-scan of entry start marks in LDS),
-//                                    walk + probe, (a * b) * c per hit in float32 as written,
-//                                    segmented wavefront sums in float64, one atomic add per
-//                                    entry and wavefront
+//                                    walk, filter, probe, (a * b) * c per hit in float32 as
+//                                    written, summed per entry in float64 in LDS, one atomic
+//                                    add per entry and chunk
 //   keep_kernel, scan, output_kernel the entries that some product reached, in C's order
 //
 // Values: each term is rounded as the reference writes it, ((a * b) * c) in float32, and the
 // terms of an entry are summed in float64 and rounded once.  The order of the float64 sums
-// across wavefronts and chunks follows atomic arrival, so values are reproducible within
+// follows atomic arrival, so values are reproducible within
 // one float32 rounding; the structure is exact.
 #include <hip/hip_runtime.h>
 
@@ -49,7 +49,7 @@ namespace sssmm {
 constexpr int kBlock = 256;
 constexpr int kChunk = 4096;       // probes per workgroup
 constexpr int kPer = kChunk / kBlock;
-constexpr int kBatch = 2;  // probe rounds whose loads are issued together
+constexpr int kBatch = 4;  // probe rounds whose loads are issued together
 constexpr uint32_t kEmptyKey = 0xffffffffu;
 constexpr uint64_t kEmptySlot = 0x00000000ffffffffull;  // value bits 0, key empty
 constexpr uint32_t kWalkB = 0x80000000u;  // entry flag: walk B's column, probe A's row table
@@ -69,32 +69,22 @@ __device__ __forceinline__ uint32_t mix(uint32_t x) {
     return x;
 }
 
-__device__ __forceinline__ void table_insert(uint64_t *table, int64_t base, uint32_t mask,
-                                             uint32_t key, float value) {
+// The filter's bit of a key in its home slot's byte.
+__device__ __forceinline__ uint32_t filter_bit(uint32_t hash) { return hash >> 29; }
+
+__device__ __forceinline__ void table_insert(uint64_t *table, unsigned *filter, int64_t base,
+                                             uint32_t mask, uint32_t key, float value) {
     const uint64_t word = (static_cast<uint64_t>(__float_as_uint(value)) << 32) | key;
-    uint32_t h = mix(key) & mask;
+    const uint32_t hash = mix(key);
+    uint32_t h = hash & mask;
+    const int64_t home = base + h;
+    atomicOr(&filter[home >> 2], 1u << (8u * static_cast<uint32_t>(home & 3) + filter_bit(hash)));
     for (;;) {
         auto *slot = reinterpret_cast<unsigned long long *>(table + base + h);
         if (atomicCAS(slot, static_cast<unsigned long long>(kEmptySlot),
                       static_cast<unsigned long long>(word)) == kEmptySlot) {
             return;
         }
-        h = (h + 1) & mask;
-    }
-}
-
-// Value stored under `key`, or false when the table has no such key.
-__device__ __forceinline__ bool table_find(const uint64_t *__restrict__ table, int64_t base,
-                                           uint32_t mask, uint32_t key, float *value) {
-    uint32_t h = mix(key) & mask;
-    for (;;) {
-        const uint64_t w = table[base + h];
-        const uint32_t k = static_cast<uint32_t>(w);
-        if (k == key) {
-            *value = __uint_as_float(static_cast<uint32_t>(w >> 32));
-            return true;
-        }
-        if (k == kEmptyKey) return false;
         h = (h + 1) & mask;
     }
 }
@@ -188,7 +178,8 @@ __global__ __launch_bounds__(kBlock) void transpose_kernel(
     const int *__restrict__ pb, int inner, const int *__restrict__ cb,
     const float *__restrict__ vb, int64_t nnz_b, const int64_t *__restrict__ col_off,
     unsigned long long *__restrict__ col_fill, const int64_t *__restrict__ tab_off,
-    int *__restrict__ csc_row, float *__restrict__ csc_val, uint64_t *__restrict__ tab_b) {
+    int *__restrict__ csc_row, float *__restrict__ csc_val, uint64_t *__restrict__ tab_b,
+    unsigned *__restrict__ filter) {
     int64_t lo, hi;
     int r_lo, r_hi;
     if (!span_rows(pb, inner, nnz_b, lo, hi, r_lo, r_hi)) return;
@@ -200,23 +191,23 @@ __global__ __launch_bounds__(kBlock) void transpose_kernel(
         csc_row[slot] = j;
         csc_val[slot] = v;
         const int64_t size = tab_off[k + 1] - tab_off[k];
-        table_insert(tab_b, tab_off[k], static_cast<uint32_t>(size - 1), static_cast<uint32_t>(j),
-                     v);
+        table_insert(tab_b, filter, tab_off[k], static_cast<uint32_t>(size - 1),
+                     static_cast<uint32_t>(j), v);
     }
 }
 
-// A's entries into the per-row tables keyed by column id.
+// A's entries into the per-row tables keyed by column id, which start at slot `first`.
 __global__ __launch_bounds__(kBlock) void rows_table_kernel(
     const int *__restrict__ pa, int rows, const int *__restrict__ ca,
     const float *__restrict__ va, int64_t nnz_a, const int64_t *__restrict__ tab_off,
-    uint64_t *__restrict__ tab_a) {
+    uint64_t *__restrict__ tab, unsigned *__restrict__ filter, int64_t first) {
     int64_t lo, hi;
     int r_lo, r_hi;
     if (!span_rows(pa, rows, nnz_a, lo, hi, r_lo, r_hi)) return;
     for (int64_t e = lo + threadIdx.x; e < hi; e += kBlock) {
         const int i = static_cast<int>(last_le(pa, r_lo, r_hi, e));
         const int64_t size = tab_off[i + 1] - tab_off[i];
-        table_insert(tab_a, tab_off[i], static_cast<uint32_t>(size - 1),
+        table_insert(tab, filter, first + tab_off[i], static_cast<uint32_t>(size - 1),
                      static_cast<uint32_t>(ca[e]), va[e]);
     }
 }
@@ -227,7 +218,7 @@ __global__ void work_kernel(const int *__restrict__ pc, int rows, const int *__r
                             int64_t nnz_c, const int *__restrict__ pa,
                             const unsigned long long *__restrict__ col_count,
                             const int64_t *__restrict__ col_off,
-                            const int64_t *__restrict__ tab_a_off,
+                            const int64_t *__restrict__ tab_a_off, int64_t first_a,
                             const int64_t *__restrict__ tab_b_off, int64_t *__restrict__ work,
                             int64_t *__restrict__ walk_base, int64_t *__restrict__ probe_base,
                             uint32_t *__restrict__ probe_mask) {
@@ -242,7 +233,7 @@ __global__ void work_kernel(const int *__restrict__ pc, int rows, const int *__r
         walk_base[e] = walk_b ? col_off[k] : static_cast<int64_t>(pa[i]);
         const int64_t t0 = walk_b ? tab_a_off[i] : tab_b_off[k];
         const int64_t t1 = walk_b ? tab_a_off[i + 1] : tab_b_off[k + 1];
-        probe_base[e] = t0;
+        probe_base[e] = walk_b ? first_a + t0 : t0;
         probe_mask[e] = static_cast<uint32_t>(t1 - t0 - 1) | (walk_b ? kWalkB : 0u);
     }
 }
@@ -258,38 +249,35 @@ __global__ void chunk_bounds_kernel(const int64_t *__restrict__ woff, int64_t nn
     }
 }
 
-// Segmented inclusive sum over a wavefront: lanes holding the same `seg` are contiguous.
-// Returns the running sums; the last lane of each segment holds the segment's total.
-__device__ __forceinline__ void wave_segmented_sum(int seg, double &v, int &h) {
-    const int l = dev::lane();
-    // every lane takes part in each shuffle (a shuffle under a lane-dependent condition
-    // would read inactive lanes)
-    const int prev = __shfl_up(seg, 1, dev::kWave);
-    int head = (l == 0 || prev != seg) ? l : 0;
-#pragma unroll
-    for (int o = 1; o < dev::kWave; o <<= 1) {
-        const int n = __shfl_up(head, o, dev::kWave);
-        if (l >= o) head = max(head, n);
-    }
-#pragma unroll
-    for (int o = 1; o < dev::kWave; o <<= 1) {
-        const double nv = __shfl_up(v, o, dev::kWave);
-        const int nh = __shfl_up(h, o, dev::kWave);
-        if (l - o >= head) {
-            v += nv;
-            h += nh;
-        }
-    }
-}
+// A chunk of at most this many mask entries (a few dozen where lists are long) keeps their
+// fields in LDS and sums them there (binary64 LDS atomics, then one global atomic per entry); a
+// chunk of more, short ones reads the fields from memory and adds each hit to the global sums.
+constexpr int kAccEntries = 256;
 
+// What a probe needs of its mask entry: the walked list's position of probe 0 of the chunk (as
+// if the list went on to it), the probed table's slots and mask | kWalkB.
+struct EntryFields {
+    int walk;
+    uint32_t mask;
+    int64_t table;
+};
+
+// Bound by the lines its random reads fetch (at C4 a 134 MB table each side, one line per 8-byte
+// probe: 58 GB in 10.5 ms) and by LDS issue.  R-MAT 2^20 masked by itself, 1.14e9 probes: sums
+// in LDS instead of a segmented sum by shuffles per 64 probes 10.5 -> 9.7 ms; the filter, whose
+// bytes mostly stay in L2 and which tells most misses, 6.9; the entries' fields in LDS and the
+// values read after the filter, four rounds at a time, 5.7 (two rounds 6.0, eight 7.0).
 __global__ __launch_bounds__(kBlock) void probe_kernel(
     const int64_t *__restrict__ woff, const int64_t *__restrict__ bounds, int64_t total,
     const int64_t *__restrict__ walk_base, const int64_t *__restrict__ probe_base,
     const uint32_t *__restrict__ probe_mask, const int *__restrict__ ca,
     const float *__restrict__ va, const int *__restrict__ csc_row,
-    const float *__restrict__ csc_val, const uint64_t *__restrict__ tab_a,
-    const uint64_t *__restrict__ tab_b, const float *__restrict__ vc,
+    const float *__restrict__ csc_val, const uint64_t *__restrict__ tab,
+    const unsigned char *__restrict__ filter, const float *__restrict__ vc,
     double *__restrict__ acc, int *__restrict__ hit) {
+    __shared__ EntryFields s_field[kAccEntries];
+    __shared__ double s_acc[kAccEntries];
+    __shared__ unsigned char s_hit[kAccEntries];
     __shared__ int s_e[kPadded];
     __shared__ int s_wave[kBlock / dev::kWave];
     // neighbouring chunks (a mask row's probes into one table) on one XCD, 64 at a time:
@@ -298,6 +286,19 @@ __global__ __launch_bounds__(kBlock) void probe_kernel(
     const int64_t c0 = chunk * kChunk;
     const int n = static_cast<int>(min(static_cast<int64_t>(kChunk), total - c0));
     const int64_t e_lo = bounds[2 * chunk], e_hi = bounds[2 * chunk + 1];
+    // a chunk of at most kAccEntries mask entries sums them here
+    const bool local = e_hi - e_lo < kAccEntries;
+    const int entries = static_cast<int>(min(e_hi - e_lo + 1, static_cast<int64_t>(kAccEntries)));
+    auto fields = [&](int64_t e) {
+        // (positions stay below 2^31: a list's own do, and the chunk's probes inside it too)
+        return EntryFields{static_cast<int>(walk_base[e] - (woff[e] - c0)), probe_mask[e],
+                           probe_base[e]};
+    };
+    for (int x = threadIdx.x; x < entries; x += kBlock) {
+        s_acc[x] = 0.0;
+        s_hit[x] = 0;
+        if (local) s_field[x] = fields(e_lo + x);
+    }
     // decode: s_e[x] = (mask entry of probe c0 + x) - e_lo
     for (int x = threadIdx.x; x < kChunk; x += kBlock) s_e[pad(x)] = 0;
     __syncthreads();
@@ -324,82 +325,87 @@ __global__ __launch_bounds__(kBlock) void probe_kernel(
     static_assert(kPer % kBatch == 0, "rounds come in whole batches");
     for (int r0 = 0; r0 < kPer; r0 += kBatch) {
         bool live[kBatch];
-        int64_t e[kBatch], wb[kBatch], tb[kBatch];
+        int ent[kBatch], wb[kBatch];  // mask entry (from e_lo), position in the walked list
+        int64_t tb[kBatch];
         uint32_t pm[kBatch];
 #pragma unroll
         for (int g = 0; g < kBatch; ++g) {
             const int x = threadIdx.x + (r0 + g) * kBlock;
             live[g] = x < n;
-            e[g] = e_lo + (live[g] ? s_e[pad(x)] : 0);
-        }
-#pragma unroll
-        for (int g = 0; g < kBatch; ++g) {
-            const int x = threadIdx.x + (r0 + g) * kBlock;
-            pm[g] = probe_mask[e[g]];
-            wb[g] = walk_base[e[g]] + (c0 + x - woff[e[g]]);
-            tb[g] = probe_base[e[g]];
+            ent[g] = live[g] ? s_e[pad(x)] : 0;
+            const EntryFields f = local ? s_field[ent[g]] : fields(e_lo + ent[g]);
+            pm[g] = f.mask;
+            wb[g] = f.walk + x;
+            tb[g] = f.table;
         }
         uint32_t key[kBatch];
-        float own[kBatch];  // the walked entry's value
 #pragma unroll
         for (int g = 0; g < kBatch; ++g) {
             key[g] = 0;
-            own[g] = 0.0f;
             if (live[g]) {
-                const bool walk_b = (pm[g] & kWalkB) != 0;
-                key[g] = static_cast<uint32_t>(walk_b ? csc_row[wb[g]] : ca[wb[g]]);
-                own[g] = walk_b ? csc_val[wb[g]] : va[wb[g]];
+                key[g] = static_cast<uint32_t>(((pm[g] & kWalkB) ? csc_row : ca)[wb[g]]);
             }
         }
-        uint32_t slot[kBatch];
-        uint64_t w[kBatch];
-#pragma unroll
-        for (int g = 0; g < kBatch; ++g) {  // first probe of every table
-            const uint32_t mask = pm[g] & ~kWalkB;
-            slot[g] = mix(key[g]) & mask;
-            w[g] = kEmptySlot;
-            if (live[g]) w[g] = ((pm[g] & kWalkB) ? tab_a : tab_b)[tb[g] + slot[g]];
-        }
-        float cv[kBatch];
-#pragma unroll
-        for (int g = 0; g < kBatch; ++g) cv[g] = live[g] ? vc[e[g]] : 0.0f;
+        // The filter first: one byte of a home slot's keys, a sixteenth of the table's
+        // footprint, tells most misses.
+        uint32_t hash[kBatch], bits[kBatch];
 #pragma unroll
         for (int g = 0; g < kBatch; ++g) {
-            double v = 0.0;
-            int h = 0;
-            if (live[g]) {
-                const uint32_t mask = pm[g] & ~kWalkB;
-                const uint64_t *tab = (pm[g] & kWalkB) ? tab_a : tab_b;
-                uint64_t ww = w[g];
-                uint32_t hh = slot[g];
-                // collisions: the next two slots per step, both loads issued together (a
-                // wavefront waits for its longest chain; the second slot is nearly always in
-                // the same line); the first of them that holds the key or is empty ends it
-                while (static_cast<uint32_t>(ww) != key[g] &&
-                       static_cast<uint32_t>(ww) != kEmptyKey) {
-                    const uint32_t h1 = (hh + 1) & mask, h2 = (hh + 2) & mask;
-                    const uint64_t w1 = tab[tb[g] + h1], w2 = tab[tb[g] + h2];
-                    const bool first = static_cast<uint32_t>(w1) == key[g] ||
-                                       static_cast<uint32_t>(w1) == kEmptyKey;
-                    ww = first ? w1 : w2;
-                    hh = first ? h1 : h2;
-                }
-                if (static_cast<uint32_t>(ww) == key[g]) {
-                    const float other = __uint_as_float(static_cast<uint32_t>(ww >> 32));
-                    // a * b with a from A and b from B, as the reference writes it
-                    const float ab = (pm[g] & kWalkB) ? other * own[g] : own[g] * other;
-                    v = static_cast<double>(ab * cv[g]);
-                    h = 1;
+            hash[g] = mix(key[g]);
+            bits[g] = live[g] ? filter[tb[g] + (hash[g] & (pm[g] & ~kWalkB))] : 0u;
+        }
+        bool maybe[kBatch];
+        uint64_t w[kBatch];
+        float cv[kBatch], own[kBatch];  // the mask's and the walked entry's values
+#pragma unroll
+        for (int g = 0; g < kBatch; ++g) {
+            maybe[g] = ((bits[g] >> filter_bit(hash[g])) & 1u) != 0;
+            w[g] = kEmptySlot;
+            cv[g] = own[g] = 0.0f;
+            if (maybe[g]) {
+                w[g] = tab[tb[g] + (hash[g] & (pm[g] & ~kWalkB))];
+                own[g] = ((pm[g] & kWalkB) ? csc_val : va)[wb[g]];
+                cv[g] = vc[e_lo + ent[g]];
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < kBatch; ++g) {
+            if (!maybe[g]) continue;
+            const uint32_t mask = pm[g] & ~kWalkB;
+            uint64_t ww = w[g];
+            uint32_t hh = hash[g] & mask;
+            // collisions: the next two slots per step, both loads issued together (a
+            // wavefront waits for its longest chain; the second slot is nearly always in
+            // the same line); the first of them that holds the key or is empty ends it
+            while (static_cast<uint32_t>(ww) != key[g] && static_cast<uint32_t>(ww) != kEmptyKey) {
+                const uint32_t h1 = (hh + 1) & mask, h2 = (hh + 2) & mask;
+                const uint64_t w1 = tab[tb[g] + h1], w2 = tab[tb[g] + h2];
+                const bool first = static_cast<uint32_t>(w1) == key[g] ||
+                                   static_cast<uint32_t>(w1) == kEmptyKey;
+                ww = first ? w1 : w2;
+                hh = first ? h1 : h2;
+            }
+            if (static_cast<uint32_t>(ww) == key[g]) {
+                const float other = __uint_as_float(static_cast<uint32_t>(ww >> 32));
+                // a * b with a from A and b from B, as the reference writes it
+                const float ab = (pm[g] & kWalkB) ? other * own[g] : own[g] * other;
+                const double v = static_cast<double>(ab * cv[g]);
+                if (local) {  // uniform
+                    atomicAdd(&s_acc[ent[g]], v);
+                    s_hit[ent[g]] = 1;
+                } else {
+                    atomicAdd(&acc[e_lo + ent[g]], v);
+                    hit[e_lo + ent[g]] = 1;
                 }
             }
-            const int seg = live[g] ? static_cast<int>(e[g] - e_lo) : -1;
-            wave_segmented_sum(seg, v, h);
-            const int l = dev::lane();
-            const int next_seg = __shfl_down(seg, 1, dev::kWave);
-            const bool tail = live[g] && (l == dev::kWave - 1 || next_seg != seg);
-            if (tail && h > 0) {
-                atomicAdd(&acc[e[g]], v);
-                hit[e[g]] = 1;
+        }
+    }
+    if (local) {
+        __syncthreads();
+        for (int x = threadIdx.x; x < entries; x += kBlock) {
+            if (s_hit[x]) {
+                atomicAdd(&acc[e_lo + x], s_acc[x]);
+                hit[e_lo + x] = 1;
             }
         }
     }
@@ -518,21 +524,26 @@ int multiply(const nacho_csr *a, const nacho_csr *b, const nacho_csr *c, nacho_c
     NACHO_TRY(call.timer_start(name));
 
     // tables and B's columns
-    uint64_t *tab_b = nullptr, *tab_a = nullptr;
+    // (one array: B's tables, then A's from slot sizes[0] on; one filter byte per slot)
+    uint64_t *tab = nullptr;
+    unsigned *filter = nullptr;
     int *csc_row = nullptr;
     float *csc_val = nullptr;
-    NACHO_TRY(call.scratch_n(static_cast<size_t>(sizes[0] + sizes[1]), &tab_b));
-    tab_a = tab_b + sizes[0];
+    const int64_t slots = sizes[0] + sizes[1];
+    const int64_t filter_words = (slots + 7) / 8;  // 64-bit
+    NACHO_TRY(call.scratch_n(static_cast<size_t>(slots), &tab));
+    NACHO_TRY(call.scratch_n(2 * static_cast<size_t>(filter_words), &filter));
     NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b), &csc_row));
     NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_b), &csc_val));
-    fill_kernel<<<grid_for(sizes[0] + sizes[1]), kBlock, 0, st>>>(tab_b, sizes[0] + sizes[1],
-                                                                  kEmptySlot);
+    fill_kernel<<<grid_for(slots), kBlock, 0, st>>>(tab, slots, kEmptySlot);
+    fill_kernel<<<grid_for(filter_words), kBlock, 0, st>>>(reinterpret_cast<uint64_t *>(filter),
+                                                           filter_words, 0ull);
     transpose_kernel<<<span_grid, kBlock, 0, st>>>(
         b->dim_j_offsets, inner, b->dim_j_indices, b->values, nnz_b, col_off,
-        reinterpret_cast<unsigned long long *>(col_fill), toff_b, csc_row, csc_val, tab_b);
+        reinterpret_cast<unsigned long long *>(col_fill), toff_b, csc_row, csc_val, tab, filter);
     rows_table_kernel<<<static_cast<unsigned>(std::max<int64_t>(1, (nnz_a + kSpan - 1) / kSpan)),
                         kBlock, 0, st>>>(a->dim_j_offsets, rows, a->dim_j_indices, a->values,
-                                         nnz_a, toff_a, tab_a);
+                                         nnz_a, toff_a, tab, filter, sizes[0]);
     NACHO_TRY_HIP(hipGetLastError());
 
     // probes per mask entry
@@ -545,7 +556,7 @@ int multiply(const nacho_csr *a, const nacho_csr *b, const nacho_csr *c, nacho_c
     NACHO_TRY(call.scratch_n(static_cast<size_t>(nnz_c), &probe_mask));
     work_kernel<<<grid_for(nnz_c), kBlock, 0, st>>>(
         c->dim_j_offsets, rows, c->dim_j_indices, nnz_c, a->dim_j_offsets,
-        reinterpret_cast<const unsigned long long *>(col_count), col_off, toff_a, toff_b, work,
+        reinterpret_cast<const unsigned long long *>(col_count), col_off, toff_a, sizes[0], toff_b, work,
         walk_base, probe_base, probe_mask);
     NACHO_TRY_HIP(hipGetLastError());
     NACHO_TRY(call.value_word(0, &word[0]));
@@ -573,7 +584,8 @@ int multiply(const nacho_csr *a, const nacho_csr *b, const nacho_csr *c, nacho_c
                                                                      bounds);
         probe_kernel<<<static_cast<unsigned>(chunks), kBlock, 0, st>>>(
             woff, bounds, total, walk_base, probe_base, probe_mask, a->dim_j_indices, a->values,
-            csc_row, csc_val, tab_a, tab_b, c->values, acc, hit);
+            csc_row, csc_val, tab, reinterpret_cast<const unsigned char *>(filter), c->values, acc,
+            hit);
         NACHO_TRY_HIP(hipGetLastError());
     }
 
