@@ -986,6 +986,17 @@ __global__ __launch_bounds__(kBlock) void emit_kernel(EmitArgs g) {
     }
 }
 
+// Binary64 sum of the kBlock values of `sh` into sh[0], in a fixed order; ends synchronised.
+__device__ __forceinline__ void block_sum_fixed(double *sh) {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int w = kBlock / 2; w > 0; w >>= 1) {
+        __syncthreads();
+        if (tid < w) sh[tid] += sh[tid + w];
+    }
+    __syncthreads();
+}
+
 // ---- small levels ----------------------------------------------------------------------
 //
 // A level of few tiles in one launch: a workgroup finds its tile's boundaries, orders it,
@@ -995,19 +1006,21 @@ __global__ __launch_bounds__(kBlock) void emit_kernel(EmitArgs g) {
 // first tile's output would wait for nothing while the memory is idle: three launches are
 // better.)
 //
-// `sync` is a block of words that only these kernels write: a ticket counter that keeps
-// counting from launch to launch (this launch's tickets start at `base`) and, per tile, the
+// `sync` is a block of words that only these kernels write: two counters that keep counting
+// from launch to launch (this launch's counts start at `base` and `done_base`) and, per tile, the
 // pairs tagged with the launch's epoch, so that it is never cleared.
 constexpr int kSyncTiles = 16;  // word of tile 0
 constexpr int kMaxPolls = 1 << 22;  // seconds
 constexpr size_t kSyncBytes = (kSyncTiles + kFusedTiles) * sizeof(unsigned long long);
 
-template <Op OP, bool VALUES, bool CHILD, bool ROWS, bool WIDE>
+template <Op OP, bool VALUES, bool CHILD, bool ROWS, bool DOT, bool WIDE>
 __global__ __launch_bounds__(kBlock) void fused_kernel(EmitArgs g, int rows, int total, int bits,
                                                        unsigned long long *__restrict__ sync,
                                                        unsigned epoch, unsigned base,
+                                                       unsigned done_base,
                                                        int64_t *__restrict__ length_out,
-                                                       long long items) {
+                                                       long long items, float *__restrict__ dot) {
+    __shared__ double s_dot[DOT ? kBlock : 1];
     __shared__ __align__(16) OrderLds sh;
     __shared__ __align__(8) unsigned short s_side[kBlock], s_dup[kBlock];
     __shared__ RowLds<ROWS> lds;
@@ -1047,6 +1060,39 @@ __global__ __launch_bounds__(kBlock) void fused_kernel(EmitArgs g, int rows, int
     const TileSplit sp{u(0), u(1), u(2), u(3), u(4), u(5)};
     unsigned side, dup;
     const unsigned own = order_tile<WIDE>(sh, sp, g.pa, g.ca, g.pb, g.cb, g.pa, bits, tid, side, dup);
+    double acc = 0.0;
+    if (DOT) {
+        // No offsets to wait for: every tile's sum goes to partial, and the workgroup that
+        // finishes last (the second counter) adds them in tile order.
+        s_side[tid] = static_cast<unsigned short>(side);
+        s_dup[tid] = static_cast<unsigned short>(dup);
+        __syncthreads();
+        emit_tile<OP, VALUES, CHILD, ROWS, DOT>(
+            g, sp, t, reinterpret_cast<const unsigned long long *>(s_side)[l],
+            reinterpret_cast<const unsigned long long *>(s_dup)[l], 0, tid, lds, acc);
+        s_dot[tid] = acc;
+        block_sum_fixed(s_dot);
+        if (g.num_tiles > 1) {  // uniform
+            if (tid == 0) {
+                __hip_atomic_store(&g.partial[t], s_dot[0], __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+                const unsigned done = __hip_atomic_fetch_add(
+                    reinterpret_cast<unsigned *>(sync + 1), 1u, __ATOMIC_ACQ_REL,
+                    __HIP_MEMORY_SCOPE_AGENT);
+                s_ticket = done - done_base == static_cast<unsigned>(g.num_tiles) - 1u;
+            }
+            __syncthreads();
+            if (!s_ticket) return;  // uniform
+            acc = 0.0;
+            for (int i = tid; i < g.num_tiles; i += kBlock) {
+                acc += __hip_atomic_load(&g.partial[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            s_dot[tid] = acc;
+            block_sum_fixed(s_dot);
+        }
+        if (tid == 0) *dot = static_cast<float>(s_dot[0]);
+        return;
+    }
     if (tid == 0 && t + 1 < g.num_tiles) {
         __hip_atomic_store(&sync[kSyncTiles + t],
                            (static_cast<unsigned long long>(epoch) << 32) | own,
@@ -1079,22 +1125,10 @@ __global__ __launch_bounds__(kBlock) void fused_kernel(EmitArgs g, int rows, int
     }
     const unsigned long long side_w = reinterpret_cast<const unsigned long long *>(s_side)[l];
     const unsigned long long dup_w = reinterpret_cast<const unsigned long long *>(s_dup)[l];
-    double acc = 0.0;
     emit_tile<OP, VALUES, CHILD, ROWS, false>(g, sp, t, side_w, dup_w, pairs, tid, lds, acc);
 }
 
 // ---- fixed-order sums ------------------------------------------------------------------
-
-// Binary64 sum of the kBlock values of `sh` into sh[0], in a fixed order; ends synchronised.
-__device__ __forceinline__ void block_sum_fixed(double *sh) {
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-        __syncthreads();
-        if (tid < w) sh[tid] += sh[tid + w];
-    }
-    __syncthreads();
-}
 
 // Workgroups of the two-level sums below: few enough that one workgroup then adds their
 // partials in a handful of loads per thread.
@@ -1184,30 +1218,43 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
                   nullptr, nullptr, num_tiles, Z.pos, Z.crd, Z.val, A.next, B.next, Z.child_a,
                   Z.child_b, A.len, B.len, Z.row, Z.crd_low, Z.low_bits, nullptr};
     SyncBlock sync{};
-    if (num_tiles <= kFusedTiles && !Z.dot) {
+    if (num_tiles <= kFusedTiles) {
         // (one tile takes no ticket)
-        NACHO_TRY(call.sync_block(kSyncBytes, num_tiles > 1 ? num_tiles : 0, &sync));
+        const unsigned tickets = num_tiles > 1 ? num_tiles : 0;
+        NACHO_TRY(call.sync_block(kSyncBytes, tickets, Z.dot ? tickets : 0, &sync));
     }
     if (sync.words) {
         void (*fused)(EmitArgs, int, int, int, unsigned long long *, unsigned, unsigned,
-                      int64_t *, long long) =
-#define NACHO_FUSED(OP, VAL, CHD, ROWS) \
-    (wide ? fused_kernel<OP, VAL, CHD, ROWS, true> : fused_kernel<OP, VAL, CHD, ROWS, false>)
-            child       ? NACHO_FUSED(Op::Union, false, true, false)
-            : intersect ? (Z.row ? NACHO_FUSED(Op::Intersect, true, false, true)
-                                 : NACHO_FUSED(Op::Intersect, true, false, false))
-            : Z.row     ? NACHO_FUSED(Op::Union, true, false, true)
-                        : NACHO_FUSED(Op::Union, true, false, false);
+                      unsigned, int64_t *, long long, float *) =
+#define NACHO_FUSED(OP, VAL, CHD, ROWS, DOT)             \
+    (wide ? fused_kernel<OP, VAL, CHD, ROWS, DOT, true> \
+          : fused_kernel<OP, VAL, CHD, ROWS, DOT, false>)
+            child       ? NACHO_FUSED(Op::Union, false, true, false, false)
+            : intersect ? (Z.dot   ? NACHO_FUSED(Op::Intersect, true, false, false, true)
+                           : Z.row ? NACHO_FUSED(Op::Intersect, true, false, true, false)
+                                   : NACHO_FUSED(Op::Intersect, true, false, false, false))
+            : Z.row     ? NACHO_FUSED(Op::Union, true, false, true, false)
+                        : NACHO_FUSED(Op::Union, true, false, false, false);
 #undef NACHO_FUSED
         int64_t *length_out = nullptr;
-        NACHO_TRY(call.length_word(&length_out));
+        if (Z.dot) {
+            NACHO_TRY(call.scratch_n(static_cast<size_t>(num_tiles), &args.partial));
+        } else {
+            NACHO_TRY(call.length_word(&length_out));
+        }
         NACHO_TRY(call.timer_start(kernel_name));
         fused<<<num_tiles, kBlock, 0, s>>>(args, rows, static_cast<int>(total), crd_bits,
-                                           sync.words, sync.epoch, sync.base, length_out, items);
+                                           sync.words, sync.epoch, sync.base, sync.done, length_out, items,
+                                           Z.dot);
         NACHO_TRY_HIP(hipGetLastError());
         call.sync_launched();
-        NACHO_TRY(call.mark_length());
+        if (!Z.dot) NACHO_TRY(call.mark_length());
         NACHO_TRY(call.timer_stop());
+        if (Z.dot) {
+            NACHO_TRY(call.collect_timer());  // (kernel timing only: waits for the stream)
+            *out_len = 0;
+            return NACHO_OK;
+        }
         if (length_pending) {
             *length_pending = true;
             return NACHO_OK;

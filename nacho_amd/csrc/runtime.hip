@@ -265,6 +265,7 @@ struct SyncEntry {
     size_t bytes;
     unsigned epoch;
     unsigned tickets;
+    unsigned finishes;
     bool busy;
 };
 using SyncKey = std::tuple<int, hipStream_t, std::thread::id>;
@@ -290,8 +291,8 @@ void free_sync_blocks_locked() {
 }
 
 // A use of the caller's block, which stays busy until give_sync_block.
-int take_sync_block(size_t bytes, unsigned tickets, hipStream_t stream, SyncKey *key,
-                    SyncBlock *out) {
+int take_sync_block(size_t bytes, unsigned tickets, unsigned finishes, hipStream_t stream,
+                    SyncKey *key, SyncBlock *out) {
     int device = 0;
     NACHO_TRY_HIP(hipGetDevice(&device));
     *key = SyncKey{device, stream, std::this_thread::get_id()};
@@ -317,14 +318,16 @@ int take_sync_block(size_t bytes, unsigned tickets, hipStream_t stream, SyncKey 
             (void)hipFree(p);
             return static_cast<int>(e);
         }
-        it = g_sync.insert({*key, SyncEntry{words, bytes, 0u, 0u, false}}).first;
+        it = g_sync.insert({*key, SyncEntry{words, bytes, 0u, 0u, 0u, false}}).first;
     }
     SyncEntry &b = it->second;
     b.busy = true;
     out->words = b.words;
     out->epoch = ++b.epoch;
     out->base = b.tickets;
+    out->done = b.finishes;
     b.tickets += tickets;
+    b.finishes += finishes;
     return NACHO_OK;
 }
 
@@ -430,11 +433,11 @@ int Call::result(size_t bytes, void **out) {
     return NACHO_OK;
 }
 
-int Call::sync_block(size_t bytes, unsigned tickets, SyncBlock *out) {
+int Call::sync_block(size_t bytes, unsigned tickets, unsigned finishes, SyncBlock *out) {
     *out = SyncBlock{};
     if (arena_ || alloc_) return NACHO_OK;
     SyncKey key;
-    const int rc = take_sync_block(bytes, tickets, stream_, &key, out);
+    const int rc = take_sync_block(bytes, tickets, finishes, stream_, &key, out);
     if (out->words) {
         sync_held_ = true;
         sync_sound_ = false;  // until the launch is made

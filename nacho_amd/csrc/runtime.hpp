@@ -36,12 +36,13 @@ namespace nacho {
 
 // A block of 64-bit device words that only one family of kernels writes, kept between calls
 // and never cleared: `epoch` (>= 1, new for every use of the block; words start as zero) tags
-// what a launch stores, and `base` is the count the block's first word, a ticket counter
-// advanced by every use, starts from.
+// what a launch stores, and `base` and `done` are the counts that the block's first two words,
+// counters that a use advances by what it says, start from.
 struct SyncBlock {
     unsigned long long *words;
     unsigned epoch;
     unsigned base;
+    unsigned done;
 };
 
 // One call's execution context: its stream and allocator, and every buffer it allocated.
@@ -75,12 +76,12 @@ class Call {
         return result(count * sizeof(T), reinterpret_cast<void **>(out));
     }
 
-    // A sync block of at least `bytes` whose counter this call's next launch advances by
-    // `tickets`; kept for this stream's later calls.  words stays null where there is none to
+    // A sync block of at least `bytes` whose counters this call's next launch advances by
+    // `tickets` and `finishes`; kept for this stream's later calls.  words stays null where there is none to
     // take (an arena call, or a caller's allocator, which the library keeps no memory of).
     // sync_launched says that the launch was made: without it the block is dropped when the
     // call ends.
-    int sync_block(size_t bytes, unsigned tickets, SyncBlock *out);
+    int sync_block(size_t bytes, unsigned tickets, unsigned finishes, SyncBlock *out);
     void sync_launched() { sync_sound_ = true; }
 
     // Release one result buffer early (e.g. an over-allocated array that turned out empty).
