@@ -253,6 +253,18 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def load_bridge():
+    """The call path between the Python classes and the library (_bridge.so, built with it);
+    raises if it has not been built."""
+    try:
+        from . import _bridge
+    except ImportError as e:
+        raise RuntimeError(f"_bridge.so does not load ({e}); "
+                           "run `python -m nacho_amd.build`") from e
+    _bridge.set_free(ctypes.cast(load().nacho_free, ctypes.c_void_p).value)
+    return _bridge
+
+
 def error_string(code: int) -> str:
     return load().nacho_error_string(code).decode()
 

@@ -7,6 +7,9 @@ in-tree so that it travels with the repository to the GPU machine.
 
     python -m nacho_amd.build          # rebuild
 
+The call path between the Python classes and the C ABI (`nacho_amd/bridge`, host C++) is built
+beside it as `nacho_amd/_bridge.so` by `build_bridge()`.
+
 The HIP code generator for the GPU target (`nacho_amd/codegen`, host C++) is built beside it
 as `nacho_amd/codegen/nacho_hipgen` by `build_codegen()`.
 """
@@ -25,6 +28,7 @@ REPO_DIR = PACKAGE_DIR.parent
 CSRC_DIR = PACKAGE_DIR / "csrc"
 BUILD_DIR = PACKAGE_DIR / "_build"
 LIBRARY = PACKAGE_DIR / "libnacho_hip.so"
+BRIDGE = PACKAGE_DIR / "_bridge.so"
 CODEGEN_DIR = PACKAGE_DIR / "codegen"
 CODEGEN_EXE = CODEGEN_DIR / "nacho_hipgen"
 
@@ -81,14 +85,17 @@ def _compile(src: Path) -> Path:
 
 
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
-    """Compile every HIP source for gfx950 and link libnacho_hip.so.  Always recompiles."""
+    """Compile every HIP source for gfx950, link libnacho_hip.so and build the call path beside
+    it.  Always recompiles."""
     BUILD_DIR.mkdir(exist_ok=True)
     srcs = sources()
     if not srcs:
         raise RuntimeError(f"no HIP sources under {CSRC_DIR}")
     jobs = jobs or min(len(srcs), max(1, (os.cpu_count() or 2)))
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        bridge = pool.submit(build_bridge, verbose)
         objs = list(pool.map(_compile, srcs))
+        bridge.result()
     tmp = LIBRARY.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
@@ -115,6 +122,33 @@ def build_codegen(verbose: bool = False) -> Path:
     if verbose:
         print(f"built {CODEGEN_EXE}", file=sys.stderr)
     return CODEGEN_EXE
+
+
+def build_bridge(verbose: bool = False) -> Path:
+    """Compile nacho_amd/_bridge.so (host C++, g++): the call path between the Python classes
+    and the C ABI, against the installed torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no host C++ compiler (g++) for the call path")
+    tmp = BRIDGE.with_name(BRIDGE.name + ".tmp")
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{p}" for p in cpp_extension.include_paths()),
+           f"-isystem{sysconfig.get_path('include')}", str(PACKAGE_DIR / "bridge" / "bridge.cpp"),
+           f"-L{Path(torch.__file__).parent / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu",
+           "-lc10", "-o", str(tmp)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"call path build failed:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, BRIDGE)
+    if verbose:
+        print(f"built {BRIDGE}", file=sys.stderr)
+    return BRIDGE
 
 
 if __name__ == "__main__":

@@ -4,20 +4,20 @@ The reference's generated wrapper (src/backend/generate_bindings.cpp:288-327) un
 operand class into the kernel's tensor struct, calls `<k>::<k>_gpu_i32_f32(operands...,
 num_blocks, threads_per_block)` and adopts the returned buffers.  These functions do the
 same through the C ABI of libnacho_hip.so: borrow operand buffers, call the entry point on
-torch's current stream, adopt the result buffers.  There is no CPU fallback: a missing
-library raises.
+torch's current stream, adopt the result buffers.  Those steps are C++ (bridge/bridge.cpp);
+what an operand may be is checked there, and named here when it is refused.  There is no CPU
+fallback: a missing library raises.
 """
 
 from __future__ import annotations
 
 import ctypes
+import operator
 
 import torch
 
 from . import _device, _lib
 from .tensors import COO3_gpu, COO_gpu, CSF3_gpu, CSR64_gpu, CSR_gpu, DCSR_gpu, Scalar_gpu
-
-_I32, _I64, _F32 = torch.int32, torch.int64, torch.float32
 
 
 def _p(t: torch.Tensor):
@@ -32,132 +32,58 @@ def _same_device(*tensors):
     return device
 
 
-# ---- descriptor conversion -----------------------------------------------------------
+# ---- operand checks ------------------------------------------------------------------
 
-def _csr_desc(t: CSR_gpu) -> _lib.CsrDesc:
-    rows, cols = t._dims
+def _buffers(t):
+    return [getattr(t, name) for name in t._attributes]
+
+
+def _check_csr(t: CSR_gpu) -> None:
+    rows = t._dims[0]
     if t.dim_j_offsets.numel() != rows + 1:
         raise ValueError(f"CSR_gpu: dim_j_offsets has {t.dim_j_offsets.numel()} entries, "
                          f"expected rows + 1 = {rows + 1}")
-    n = t.dim_j_indices.numel()
-    if t.values.numel() != n:
+    if t.values.numel() != t.dim_j_indices.numel():
         raise ValueError("CSR_gpu: dim_j_indices and values differ in length")
-    return _lib.CsrDesc(rows, cols, _p(t.dim_j_offsets), n, _p(t.dim_j_indices), _p(t.values), n)
 
 
-def _coo_desc(t: COO_gpu) -> _lib.CooDesc:
-    rows, cols = t._dims
-    n = t.values.numel()
-    if t.dim_i_indices.numel() != n or t.dim_j_indices.numel() != n:
-        raise ValueError("COO_gpu: coordinate and value arrays differ in length")
-    return _lib.CooDesc(rows, cols, n, _p(t.dim_i_indices), n, _p(t.dim_j_indices),
-                        _p(t.values), n)
+def _check_coo(t) -> None:
+    if any(x.numel() != t.values.numel() for x in _buffers(t)):
+        raise ValueError(f"{type(t).__name__}: coordinate and value arrays differ in length")
 
 
-def _coo3_desc(t: COO3_gpu) -> _lib.Coo3Desc:
-    si, sj, sk = t._dims
-    n = t.values.numel()
-    if any(x.numel() != n for x in (t.dim_i_indices, t.dim_j_indices, t.dim_k_indices)):
-        raise ValueError("COO3_gpu: coordinate and value arrays differ in length")
-    return _lib.Coo3Desc(si, sj, sk, n, _p(t.dim_i_indices), n, _p(t.dim_j_indices), n,
-                         _p(t.dim_k_indices), _p(t.values), n)
-
-
-def _dcsr_desc(t: DCSR_gpu) -> _lib.DcsrDesc:
-    rows, cols = t._dims
-    ni, nj = t.dim_i_indices.numel(), t.dim_j_indices.numel()
+def _check_dcsr(t: DCSR_gpu) -> None:
+    ni = t.dim_i_indices.numel()
     if t.dim_j_offsets.numel() != ni + 1:
         raise ValueError(f"DCSR_gpu: dim_j_offsets has {t.dim_j_offsets.numel()} entries, "
                          f"expected stored rows + 1 = {ni + 1}")
-    if t.values.numel() != nj:
+    if t.values.numel() != t.dim_j_indices.numel():
         raise ValueError("DCSR_gpu: dim_j_indices and values differ in length")
-    return _lib.DcsrDesc(rows, cols, ni, _p(t.dim_i_indices), _p(t.dim_j_offsets), nj,
-                         _p(t.dim_j_indices), _p(t.values), nj)
 
 
-def _csf3_desc(t: CSF3_gpu) -> _lib.Csf3Desc:
-    si, sj, sk = t._dims
-    ni, nj, nk = t.dim_i_indices.numel(), t.dim_j_indices.numel(), t.dim_k_indices.numel()
+def _check_csf3(t: CSF3_gpu) -> None:
+    ni, nj = t.dim_i_indices.numel(), t.dim_j_indices.numel()
     if t.dim_j_offsets.numel() != ni + 1 or t.dim_k_offsets.numel() != nj + 1:
         raise ValueError("CSF3_gpu: offsets arrays must have parent length + 1 entries")
-    if t.values.numel() != nk:
+    if t.values.numel() != t.dim_k_indices.numel():
         raise ValueError("CSF3_gpu: dim_k_indices and values differ in length")
-    return _lib.Csf3Desc(si, sj, sk, ni, _p(t.dim_i_indices), _p(t.dim_j_offsets), nj,
-                         _p(t.dim_j_indices), _p(t.dim_k_offsets), nk, _p(t.dim_k_indices),
-                         _p(t.values), nk)
 
 
-def _cached_desc(t, desc_fn):
-    """The operand's C descriptor, rebuilt only when a buffer's address or length changed
-    since it was last built for this object (its fields are read-only, but a buffer could
-    be resized in place): repeated calls on the same operands skip the size checks and the
-    ctypes construction."""
-    key = tuple((b.data_ptr(), b.numel()) for b in (getattr(t, "_" + n) for n, _ in t._fields))
-    cached = t.__dict__.get("_cdesc")
-    if cached is not None and cached[0] is desc_fn and cached[1] == key:
-        return cached[2]
-    d = desc_fn(t)
-    object.__setattr__(t, "_cdesc", (desc_fn, key, d))
-    return d
+class _Operand:
+    """How the call path takes a class: its number there (enum Kind in bridge/bridge.cpp), its
+    buffers as a tuple, and the check that names what is wrong with a refused one."""
+
+    __slots__ = ("cls", "kind", "buffers", "check")
+
+    def __init__(self, cls, kind, check=None):
+        self.cls, self.kind, self.check = cls, kind, check
+        self.buffers = operator.attrgetter(*cls._attributes)
 
 
-# ---- result adoption -----------------------------------------------------------------
-
-def _adopt_csr(z: _lib.CsrDesc, device, stream) -> CSR_gpu:
-    rows, n = z.dim_i_size, z.dim_j_length
-    return CSR_gpu._trusted((_device.adopt(z.dim_j_offsets, rows + 1, _I32, device, stream),
-                             _device.adopt(z.dim_j_indices, n, _I32, device, stream),
-                             _device.adopt(z.values, n, _F32, device, stream)),
-                            [z.dim_i_size, z.dim_j_size], device)
-
-
-def _adopt_csr64(z: _lib.Csr64Desc, device, stream) -> CSR64_gpu:
-    rows, n = z.dim_i_size, z.dim_j_length
-    return CSR64_gpu._trusted((_device.adopt(z.dim_j_offsets, rows + 1, _I64, device, stream),
-                               _device.adopt(z.dim_j_indices, n, _I32, device, stream),
-                               _device.adopt(z.values, n, _F32, device, stream)),
-                              [z.dim_i_size, z.dim_j_size], device)
-
-
-def _adopt_coo(z: _lib.CooDesc, device, stream) -> COO_gpu:
-    n = z.nnz
-    return COO_gpu._trusted((_device.adopt(z.dim_i_indices, n, _I32, device, stream),
-                             _device.adopt(z.dim_j_indices, n, _I32, device, stream),
-                             _device.adopt(z.values, n, _F32, device, stream)),
-                            [z.dim_i_size, z.dim_j_size], device)
-
-
-def _adopt_coo3(z: _lib.Coo3Desc, device, stream) -> COO3_gpu:
-    n = z.nnz
-    return COO3_gpu._trusted((_device.adopt(z.dim_i_indices, n, _I32, device, stream),
-                              _device.adopt(z.dim_j_indices, n, _I32, device, stream),
-                              _device.adopt(z.dim_k_indices, n, _I32, device, stream),
-                              _device.adopt(z.values, n, _F32, device, stream)),
-                             [z.dim_i_size, z.dim_j_size, z.dim_k_size], device)
-
-
-def _adopt_dcsr(z: _lib.DcsrDesc, device, stream) -> DCSR_gpu:
-    ni, nj = z.dim_i_length, z.dim_j_length
-    return DCSR_gpu._trusted((_device.adopt(z.dim_i_indices, ni, _I32, device, stream),
-                              _device.adopt(z.dim_j_offsets, ni + 1, _I32, device, stream),
-                              _device.adopt(z.dim_j_indices, nj, _I32, device, stream),
-                              _device.adopt(z.values, nj, _F32, device, stream)),
-                             [z.dim_i_size, z.dim_j_size], device)
-
-
-def _adopt_csf3(z: _lib.Csf3Desc, device, stream) -> CSF3_gpu:
-    ni, nj, nk = z.dim_i_length, z.dim_j_length, z.dim_k_length
-    return CSF3_gpu._trusted((_device.adopt(z.dim_i_indices, ni, _I32, device, stream),
-                              _device.adopt(z.dim_j_offsets, ni + 1, _I32, device, stream),
-                              _device.adopt(z.dim_j_indices, nj, _I32, device, stream),
-                              _device.adopt(z.dim_k_offsets, nj + 1, _I32, device, stream),
-                              _device.adopt(z.dim_k_indices, nk, _I32, device, stream),
-                              _device.adopt(z.values, nk, _F32, device, stream)),
-                             [z.dim_i_size, z.dim_j_size, z.dim_k_size], device)
-
-
-def _adopt_scalar(z: _lib.ScalarDesc, device, stream) -> Scalar_gpu:
-    return Scalar_gpu._trusted((_device.adopt(z.values, 1, _F32, device, stream),), [], device)
+_CSR, _COO = _Operand(CSR_gpu, 0, _check_csr), _Operand(COO_gpu, 1, _check_coo)
+_COO3, _DCSR = _Operand(COO3_gpu, 2, _check_coo), _Operand(DCSR_gpu, 3, _check_dcsr)
+_CSF3 = _Operand(CSF3_gpu, 4, _check_csf3)
+_CSR64, _SCALAR = _Operand(CSR64_gpu, 5), _Operand(Scalar_gpu, 6)  # results only
 
 
 # ---- input validation ----------------------------------------------------------------
@@ -179,7 +105,9 @@ def validate_csr(t: CSR_gpu) -> None:
     ValueError if it is malformed."""
     if not isinstance(t, CSR_gpu):
         raise TypeError(f"validate_csr: expected CSR_gpu, got {type(t).__name__}")
-    desc = _csr_desc(t)
+    _check_csr(t)
+    n = t.values.numel()
+    desc = _lib.CsrDesc(*t._dims, _p(t.dim_j_offsets), n, _p(t.dim_j_indices), _p(t.values), n)
     with _device.on_device(t.device):
         rc = _lib.load().nacho_validate_csr(ctypes.byref(desc),
                                             ctypes.c_void_p(_device.current_stream(t.device)))
@@ -189,131 +117,125 @@ def validate_csr(t: CSR_gpu) -> None:
     _lib.check(rc, "nacho_validate_csr")
 
 
-def _maybe_validate(*operands):
-    if _VALIDATE:
-        for t in operands:
-            if isinstance(t, CSR_gpu):
-                validate_csr(t)
+def _validate_all(*operands):
+    for t in operands:
+        if isinstance(t, CSR_gpu):
+            validate_csr(t)
 
 
 # ---- generic call --------------------------------------------------------------------
 
 _ENTRIES: dict = {}
+_bridge = None
 
 
-def _entry(name):
-    """The library's entry point `name` (looked up once)."""
-    fn = _ENTRIES.get(name)
-    if fn is None:
-        fn = getattr(_lib.load(), name, None)
+def _entry(name) -> int:
+    """Address of the library's entry point `name` (looked up once)."""
+    global _bridge
+    address = _ENTRIES.get(name)
+    if address is None:
+        lib = _lib.load()
+        if _bridge is None:
+            _bridge = _lib.load_bridge()
+        fn = getattr(lib, name, None)
         if fn is None:
             raise RuntimeError(f"{name} is not exported by {_lib.LIBRARY_PATH.name}")
-        _ENTRIES[name] = fn
-    return fn
+        address = _ENTRIES[name] = ctypes.cast(fn, ctypes.c_void_p).value
+    return address
 
 
-def _call(entry, a, b, cls, desc_fn, result_desc, adopt_fn, num_blocks, threads_per_block,
-          cls_b=None, desc_fn_b=None):
-    """One two-operand entry point: a (class `cls`) and b (class `cls_b`, default `cls`)."""
-    cls_b = cls_b or cls
-    desc_fn_b = desc_fn_b or desc_fn
-    for name, t, c in (("a", a, cls), ("b", b, cls_b)):
-        if not isinstance(t, c):
-            raise TypeError(f"{entry}: operand {name} must be {c.__name__}, "
-                            f"got {type(t).__name__}")
-    _maybe_validate(a, b)
-    device = _same_device(a, b)
-    fn = _entry(entry)
-    da, db = _cached_desc(a, desc_fn), _cached_desc(b, desc_fn_b)
-    z = result_desc()
+def _refuse(entry, operands, kinds):
+    """Raise for operands that the call path did not take, naming what is wrong."""
+    for t, kind in zip(operands, kinds):
+        kind.check(t)
+    _same_device(*(buf for t, kind in zip(operands, kinds) for buf in kind.buffers(t)))
+    raise ValueError(f"{entry}: an operand has more than 2^31 - 1 entries")
+
+
+def _call(entry, operands, kinds, result, num_blocks, threads_per_block):
+    """One entry point on `operands` (of `kinds`, in order), giving a `result`."""
+    args = []
+    for t, kind in zip(operands, kinds):
+        if not isinstance(t, kind.cls):
+            raise TypeError(f"{entry}: operand {'abc'[len(args) // 3]} must be "
+                            f"{kind.cls.__name__}, got {type(t).__name__}")
+        args += (kind.kind, kind.buffers(t), t._dims)
+    if _VALIDATE:
+        _validate_all(*operands)
+    device = _same_device(*operands)
+    address = _entry(entry)
     with _device.on_device(device):
         stream = _device.current_stream(device)
-        rc = fn(ctypes.byref(da), ctypes.byref(db), ctypes.byref(z), int(num_blocks),
-                int(threads_per_block), ctypes.c_void_p(stream), None)
-        _lib.check(rc, entry)
-        return adopt_fn(z, device, stream)
+        z = _bridge.invoke(address, result.kind, int(num_blocks), int(threads_per_block), stream,
+                           device.index, *args)
+        if type(z) is tuple:
+            return result.cls._trusted(z[0], z[1], device)
+        if z is None:
+            _refuse(entry, operands, kinds)
+        _lib.check(z, entry)
 
 
 def gpu_csr_add_f32(a: CSR_gpu, b: CSR_gpu, num_blocks: int = 256,
                     threads_per_block: int = 256) -> CSR_gpu:
     """Z = a + b (sorted union per row; explicit zeros kept).  compiler.cpp:112."""
-    return _call("nacho_gpu_csr_add_f32", a, b, CSR_gpu, _csr_desc, _lib.CsrDesc, _adopt_csr,
-                 num_blocks, threads_per_block)
-
-
-def _call3(entry, a, b, c, num_blocks, threads_per_block) -> CSR_gpu:
-    for name, t in (("a", a), ("b", b), ("c", c)):
-        if not isinstance(t, CSR_gpu):
-            raise TypeError(f"{entry}: operand {name} must be CSR_gpu, got {type(t).__name__}")
-    _maybe_validate(a, b, c)
-    device = _same_device(a, b, c)
-    fn = _entry(entry)
-    da, db, dc = (_cached_desc(t, _csr_desc) for t in (a, b, c))
-    z = _lib.CsrDesc()
-    with _device.on_device(device):
-        stream = _device.current_stream(device)
-        rc = fn(ctypes.byref(da), ctypes.byref(db), ctypes.byref(dc), ctypes.byref(z),
-                int(num_blocks), int(threads_per_block), ctypes.c_void_p(stream), None)
-        _lib.check(rc, entry)
-        return _adopt_csr(z, device, stream)
+    return _call("nacho_gpu_csr_add_f32", (a, b), (_CSR, _CSR), _CSR, num_blocks, threads_per_block)
 
 
 def gpu_csr_add_3_f32(a: CSR_gpu, b: CSR_gpu, c: CSR_gpu, num_blocks: int = 256,
                       threads_per_block: int = 256) -> CSR_gpu:
     """Z = a + b + c (sorted union of three; values (a + b) + c over the present operands).
     compiler.cpp:114."""
-    return _call3("nacho_gpu_csr_add_3_f32", a, b, c, num_blocks, threads_per_block)
+    return _call("nacho_gpu_csr_add_3_f32", (a, b, c), (_CSR, _CSR, _CSR), _CSR, num_blocks,
+                 threads_per_block)
 
 
 def gpu_sssmm_f32(a: CSR_gpu, b: CSR_gpu, c: CSR_gpu, num_blocks: int = 256,
                   threads_per_block: int = 256) -> CSR_gpu:
     """Masked SpGEMM Z_ik = sum_j a_ij b_jk c_ik over the entries of c that a product reaches.
     compiler.cpp:150-153."""
-    return _call3("nacho_gpu_sssmm_f32", a, b, c, num_blocks, threads_per_block)
+    return _call("nacho_gpu_sssmm_f32", (a, b, c), (_CSR, _CSR, _CSR), _CSR, num_blocks,
+                 threads_per_block)
 
 
 def gpu_csr_mul_f32(a: CSR_gpu, b: CSR_gpu, num_blocks: int = 256,
                     threads_per_block: int = 256) -> CSR_gpu:
     """Z = a * b elementwise (sorted intersection per row).  compiler.cpp:116."""
-    return _call("nacho_gpu_csr_mul_f32", a, b, CSR_gpu, _csr_desc, _lib.CsrDesc, _adopt_csr,
-                 num_blocks, threads_per_block)
+    return _call("nacho_gpu_csr_mul_f32", (a, b), (_CSR, _CSR), _CSR, num_blocks, threads_per_block)
 
 
 def gpu_coo_add_f32(a: COO_gpu, b: COO_gpu, num_blocks: int = 256,
                     threads_per_block: int = 256) -> COO_gpu:
     """Z = a + b over COO (union of (i, j)).  compiler.cpp:118."""
-    return _call("nacho_gpu_coo_add_f32", a, b, COO_gpu, _coo_desc, _lib.CooDesc, _adopt_coo,
-                 num_blocks, threads_per_block)
+    return _call("nacho_gpu_coo_add_f32", (a, b), (_COO, _COO), _COO, num_blocks, threads_per_block)
 
 
 def gpu_coo_mul_f32(a: COO_gpu, b: COO_gpu, num_blocks: int = 256,
                     threads_per_block: int = 256) -> COO_gpu:
     """Z = a * b over COO (intersection of (i, j)).  compiler.cpp:120."""
-    return _call("nacho_gpu_coo_mul_f32", a, b, COO_gpu, _coo_desc, _lib.CooDesc, _adopt_coo,
-                 num_blocks, threads_per_block)
+    return _call("nacho_gpu_coo_mul_f32", (a, b), (_COO, _COO), _COO, num_blocks, threads_per_block)
 
 
 def gpu_coo3d_add_f32(a: COO3_gpu, b: COO3_gpu, num_blocks: int = 256,
                       threads_per_block: int = 256) -> COO3_gpu:
     """Z = a + b over COO3 (union of (i, j, k)).  compiler.cpp:138."""
-    return _call("nacho_gpu_coo3d_add_f32", a, b, COO3_gpu, _coo3_desc, _lib.Coo3Desc,
-                 _adopt_coo3, num_blocks, threads_per_block)
+    return _call("nacho_gpu_coo3d_add_f32", (a, b), (_COO3, _COO3), _COO3, num_blocks,
+                 threads_per_block)
 
 
 def gpu_dcsr_add_f32(a: DCSR_gpu, b: DCSR_gpu, num_blocks: int = 256,
                      threads_per_block: int = 256) -> DCSR_gpu:
     """Z = a + b over DCSR (union of row ids, then of each row's columns).
     compiler.cpp:124."""
-    return _call("nacho_gpu_dcsr_add_f32", a, b, DCSR_gpu, _dcsr_desc, _lib.DcsrDesc,
-                 _adopt_dcsr, num_blocks, threads_per_block)
+    return _call("nacho_gpu_dcsr_add_f32", (a, b), (_DCSR, _DCSR), _DCSR, num_blocks,
+                 threads_per_block)
 
 
 def gpu_dcsr_mul_f32(a: DCSR_gpu, b: DCSR_gpu, num_blocks: int = 256,
                      threads_per_block: int = 256) -> DCSR_gpu:
     """Z = a * b over DCSR: rows stored in both operands, each with the intersection of its
     columns (kept when that is empty).  compiler.cpp:126."""
-    return _call("nacho_gpu_dcsr_mul_f32", a, b, DCSR_gpu, _dcsr_desc, _lib.DcsrDesc,
-                 _adopt_dcsr, num_blocks, threads_per_block)
+    return _call("nacho_gpu_dcsr_mul_f32", (a, b), (_DCSR, _DCSR), _DCSR, num_blocks,
+                 threads_per_block)
 
 
 def gpu_dcsr_mul_without_recursive_partitioning_f32(
@@ -321,53 +243,51 @@ def gpu_dcsr_mul_without_recursive_partitioning_f32(
         threads_per_block: int = 256) -> DCSR_gpu:
     """The same product as gpu_dcsr_mul_f32 (the reference variant differs only in how it
     partitions work).  compiler.cpp:128-133."""
-    return _call("nacho_gpu_dcsr_mul_without_recursive_partitioning_f32", a, b, DCSR_gpu,
-                 _dcsr_desc, _lib.DcsrDesc, _adopt_dcsr, num_blocks, threads_per_block)
+    return _call("nacho_gpu_dcsr_mul_without_recursive_partitioning_f32", (a, b),
+                 (_DCSR, _DCSR), _DCSR, num_blocks, threads_per_block)
 
 
 def gpu_csf_add_f32(a: CSF3_gpu, b: CSF3_gpu, num_blocks: int = 256,
                     threads_per_block: int = 256) -> CSF3_gpu:
     """Z = a + b over CSF3 (union at every level).  compiler.cpp:135."""
-    return _call("nacho_gpu_csf_add_f32", a, b, CSF3_gpu, _csf3_desc, _lib.Csf3Desc,
-                 _adopt_csf3, num_blocks, threads_per_block)
+    return _call("nacho_gpu_csf_add_f32", (a, b), (_CSF3, _CSF3), _CSF3, num_blocks,
+                 threads_per_block)
 
 
 def gpu_coo_csr_add_f32(a: CSR_gpu, b: COO_gpu, num_blocks: int = 256,
                         threads_per_block: int = 256) -> CSR_gpu:
     """Z = a + b for a CSR a and a COO b (sorted, no duplicates), giving CSR.
     compiler.cpp:122."""
-    return _call("nacho_gpu_coo_csr_add_f32", a, b, CSR_gpu, _csr_desc, _lib.CsrDesc,
-                 _adopt_csr, num_blocks, threads_per_block, cls_b=COO_gpu,
-                 desc_fn_b=_coo_desc)
+    return _call("nacho_gpu_coo_csr_add_f32", (a, b), (_CSR, _COO), _CSR, num_blocks,
+                 threads_per_block)
 
 
 def gpu_inner_prod_f32(a: CSF3_gpu, b: CSF3_gpu, num_blocks: int = 256,
                        threads_per_block: int = 256) -> Scalar_gpu:
     """z = sum_ijk a_ijk * b_ijk over CSF3 operands (float32 products summed in float64,
     rounded once).  compiler.cpp:141."""
-    return _call("nacho_gpu_inner_prod_f32", a, b, CSF3_gpu, _csf3_desc, _lib.ScalarDesc,
-                 _adopt_scalar, num_blocks, threads_per_block)
+    return _call("nacho_gpu_inner_prod_f32", (a, b), (_CSF3, _CSF3), _SCALAR, num_blocks,
+                 threads_per_block)
 
 
 def gpu_inner_prod_coo_f32(a: COO3_gpu, b: COO3_gpu, num_blocks: int = 256,
                            threads_per_block: int = 256) -> Scalar_gpu:
     """The same inner product over COO3 operands.  compiler.cpp:143."""
-    return _call("nacho_gpu_inner_prod_coo_f32", a, b, COO3_gpu, _coo3_desc, _lib.ScalarDesc,
-                 _adopt_scalar, num_blocks, threads_per_block)
+    return _call("nacho_gpu_inner_prod_coo_f32", (a, b), (_COO3, _COO3), _SCALAR, num_blocks,
+                 threads_per_block)
 
 
 def gpu_spgemm_f32(a: CSR_gpu, b: CSR_gpu, num_blocks: int = 256,
                    threads_per_block: int = 256) -> CSR_gpu:
     """Z_ik = sum_j a_ij b_jk (ESC SpGEMM), int32 result.  compiler.cpp:145-148."""
-    return _call("nacho_gpu_spgemm_f32", a, b, CSR_gpu, _csr_desc, _lib.CsrDesc, _adopt_csr,
-                 num_blocks, threads_per_block)
+    return _call("nacho_gpu_spgemm_f32", (a, b), (_CSR, _CSR), _CSR, num_blocks, threads_per_block)
 
 
 def gpu_spgemm64_f32(a: CSR_gpu, b: CSR_gpu, num_blocks: int = 256,
                      threads_per_block: int = 256) -> CSR64_gpu:
     """The same product with int64 result offsets, for results beyond 2^31 entries."""
-    return _call("nacho_gpu_spgemm64_f32", a, b, CSR_gpu, _csr_desc, _lib.Csr64Desc,
-                 _adopt_csr64, num_blocks, threads_per_block)
+    return _call("nacho_gpu_spgemm64_f32", (a, b), (_CSR, _CSR), _CSR64, num_blocks,
+                 threads_per_block)
 
 
 def release_cached_memory() -> None:

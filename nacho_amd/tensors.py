@@ -41,6 +41,7 @@ class _GpuTensor:
     """Common machinery: named device buffers (checked dtype/device) plus a host shape."""
 
     _fields: tuple[tuple[str, torch.dtype], ...] = ()
+    _attributes: tuple[str, ...] = ()  # where the buffers of _fields are kept
     _rank = 0
 
     def __init__(self, *buffers, shape=None):
@@ -60,14 +61,15 @@ class _GpuTensor:
         object.__setattr__(self, "_device", device)
 
     @classmethod
-    def _trusted(cls, buffers, shape_list, device):
-        """Build from buffers the library just produced (already checked): no validation."""
+    def _trusted(cls, buffers, dims, device):
+        """Build from buffers and dimensions (tuples) that the library just produced: no
+        validation."""
         obj = object.__new__(cls)
-        for (name, _), buf in zip(cls._fields, buffers):
-            object.__setattr__(obj, "_" + name, buf)
-        object.__setattr__(obj, "_shape", None)  # built on first access
-        object.__setattr__(obj, "_dims", tuple(int(x) for x in shape_list))
-        object.__setattr__(obj, "_device", device)
+        state = obj.__dict__
+        state.update(zip(cls._attributes, buffers))
+        state["_shape"] = None  # built on first access
+        state["_dims"] = dims
+        state["_device"] = device
         return obj
 
     @property
@@ -107,7 +109,8 @@ def _field(name):
 
 
 def _make(cls_name, fields, rank, doc):
-    ns = {"_fields": tuple(fields), "_rank": rank, "__doc__": doc}
+    ns = {"_fields": tuple(fields), "_rank": rank, "__doc__": doc,
+          "_attributes": tuple("_" + name for name, _ in fields)}
     for name, _ in fields:
         ns[name] = _field(name)
 
@@ -173,6 +176,7 @@ class Scalar_gpu(_GpuTensor):
     dimensions left, no shape (generate_bindings.cpp:181-183)."""
 
     _fields = (("values", _F32),)
+    _attributes = ("_values",)
     _rank = 0
     values = _field("values")
 
