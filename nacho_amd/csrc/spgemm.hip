@@ -565,6 +565,38 @@ __device__ __forceinline__ void expand_runs(const int4 *__restrict__ desc, int64
     __syncthreads();  // every lane is done with the scratch
 }
 
+// Products by windows: the runs of up to kTile products laid end to end, each window of 64
+// consecutive products a wavefront's, lane x on product x, so that a window's gathers are
+// consecutive entries of a few runs (R-MAT scale 20: 14 products per run) and a product's run
+// costs two bit counts.  Eight consecutive products per lane instead (a search or a running
+// maximum for the first, then a walk; every gather instruction on 64 cache lines) took 35.4 ms
+// in the bitmap units and 17.3 ms in the dense units at scale 20; windows 31.4 and 15.3.  s_mask has a bit per product that starts a run (every
+// run has at least one product); lane l of a wavefront keeps word l and the number of bits
+// before it, and a product's run is a count of bits.
+struct RunWindows {
+    unsigned long long word;
+    int before;
+    // Run of lane l's product in window i (uniform), counted from `before`'s first run.
+    __device__ __forceinline__ int run(int i) const {
+        const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_readlane(
+            static_cast<int>(static_cast<unsigned>(word)), i));
+        const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_readlane(
+            static_cast<int>(static_cast<unsigned>(word >> 32)), i));
+        const unsigned long long m = (static_cast<unsigned long long>(hi) << 32) | lo;
+        // the bits up to lane l's own: those below it, and its own
+        const int own = __builtin_amdgcn_inverse_ballot_w64(m) ? 1 : 0;
+        return __builtin_amdgcn_readlane(before, i) +
+               static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u))) +
+               own - 1;
+    }
+};
+
+__device__ __forceinline__ RunWindows load_windows(const unsigned *s_mask, int first) {
+    const unsigned long long word = reinterpret_cast<const unsigned long long *>(s_mask)[dev::lane()];
+    const int bits = __popcll(word);
+    return RunWindows{word, first + dev::wave_inclusive_sum(bits) - bits};
+}
+
 // ---- 4: units --------------------------------------------------------------------------
 
 // A segment is accumulated densely when it has more than kShort products, or more than
@@ -1008,6 +1040,9 @@ __device__ __forceinline__ void mark_bucket(unsigned *bm, const unsigned short *
 // live in its own product range of the unit; once every bucket is done, a scan of their
 // counts gives the output offsets and the workgroup stores the unit's entries with
 // consecutive lanes on consecutive outputs.
+// At R-MAT scale 20 (1.5 million units) 30.1 ms, LDS about half busy.  A bucket of up to 512
+// products keeps its columns, values and ranks in registers, which leaves out a quarter of the
+// LDS instructions (31.4 -> 30.4 ms); tables loaded up front 30.4 -> 30.1.
 __global__ __launch_bounds__(kBitmapBlock) void bitmap_unit_kernel(
     const int *__restrict__ bitmap_list, const int *__restrict__ unit_seg,
     const int64_t *__restrict__ unit_start, int64_t n_units, int64_t n_seg,
@@ -1020,14 +1055,15 @@ __global__ __launch_bounds__(kBitmapBlock) void bitmap_unit_kernel(
     const int64_t *__restrict__ seg_out) {
     constexpr int kWaves = kBitmapBlock / dev::kWave;
     constexpr int kPerB = kTile / kBitmapBlock;
+    constexpr int kHeld = 8;  // products per lane of a bucket held in registers
     __shared__ double s_acc[kTile];
     __shared__ unsigned short s_col[kTile];  // column offset inside its bucket's window
-    __shared__ float s_pv[kPadded];          // product values (padded positions)
-    __shared__ unsigned s_bits[kWaves][kBitmapWords];
-    __shared__ int s_pre[kWaves][kBitmapWords];
+    __shared__ float s_pv[kTile];            // product values
+    __shared__ __align__(16) unsigned s_bits[kWaves][kBitmapWords];
+    __shared__ __align__(16) int s_pre[kWaves][kBitmapWords];
     __shared__ int s_x0[kMaxBitmapSegs + 1];
     __shared__ int s_base[kMaxBitmapSegs];
-    __shared__ int s_sid[kMaxBitmapSegs];
+    __shared__ int s_row[kMaxBitmapSegs];
     __shared__ int s_out[kMaxBitmapSegs];
     __shared__ int s_wave[kWaves];
     __shared__ int s_next;  // the next bucket to claim
@@ -1036,15 +1072,25 @@ __global__ __launch_bounds__(kBitmapBlock) void bitmap_unit_kernel(
     const int64_t s1 = u + 1 < n_units ? unit_seg[u + 1] : n_seg;
     const int64_t start = unit_start[u];
     const int n = static_cast<int>(unit_start[u + 1] - start);
+    // Everything the unit reads of the tables is loaded up front, four dependent steps (list,
+    // unit, segment, row and runs) before the gathers: with two workgroups per CU each step
+    // costs its latency.
+    const int64_t s = min(s0 + static_cast<int64_t>(threadIdx.x), s1 - 1);
+    const int64_t r0 = seg_roff[s0];
+    const int R = static_cast<int>(seg_roff[s1] - r0);
+    const int64_t out = seg_out ? seg_out[s0] : start;
+    const bool here = s0 + threadIdx.x < s1 && seg_len[s] > 0;
+    const int64_t first = seg_off[s];
+    const int row = seg_row[s];
+    int4 d = desc[r0 + min(static_cast<int>(threadIdx.x), R - 1)];
+    const int64_t row_seg = seg_prefix[row], row_first = row_off[row];
     // the unit's nonempty buckets in order (at most kMaxBitmapSegs segments: one per lane)
-    const int64_t s = s0 + threadIdx.x;
-    const bool here = s < s1 && seg_len[s] > 0;
     int n_buckets = 0;
     const int ord = dev::block_exclusive_sum<kBitmapBlock>(here ? 1 : 0, s_wave, n_buckets);
     if (here) {
-        s_x0[ord] = static_cast<int>(seg_off[s] - start);
-        s_base[ord] = static_cast<int>((s - seg_prefix[seg_row[s]]) << shift);
-        s_sid[ord] = static_cast<int>(s);
+        s_x0[ord] = static_cast<int>(first - start);
+        s_base[ord] = static_cast<int>((s - row_seg) << shift);
+        s_row[ord] = first == row_first ? row : -1;  // the row that starts with the bucket
     }
     if (threadIdx.x == 0) {
         s_x0[n_buckets] = n;
@@ -1053,93 +1099,158 @@ __global__ __launch_bounds__(kBitmapBlock) void bitmap_unit_kernel(
     // the unit's products from its runs: window offsets (bucket = column >> shift, so the
     // offset is the column's low bits) and values, staged once
     const int low = (1 << shift) - 1;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / dev::kWave), l = dev::lane();
     {
-        int kk[kPerB];
-        float vv[kPerB];
-        const int64_t r0 = seg_roff[s0];
-        const int R = static_cast<int>(seg_roff[s1] - r0);
-        expand_runs<kBitmapBlock, kPerB>(desc, r0, R, n, cv_b, reinterpret_cast<int *>(s_acc),
-                    reinterpret_cast<float *>(s_acc) + kTile, reinterpret_cast<int *>(s_pv),
-                    s_wave, kk, vv);
-        const int lo = threadIdx.x * kPerB;
+        int *s_bs = reinterpret_cast<int *>(s_acc);                 // product 0's B entry
+        float *s_a = reinterpret_cast<float *>(s_acc) + kTile;      // A value
+        unsigned *s_mask = s_bits[0];
+        if (threadIdx.x < kTile / 32) s_mask[threadIdx.x] = 0u;
+        __syncthreads();
+        int products = 0;
+        for (int rb = 0; rb < R; rb += kBitmapBlock) {  // uniform
+            const int r = rb + static_cast<int>(threadIdx.x);
+            if (rb > 0) d = desc[r0 + min(r, R - 1)];
+            int total = 0;
+            const int off = products + dev::block_exclusive_sum<kBitmapBlock>(
+                                           r < R ? d.y : 0, s_wave, total);
+            if (r < R) {
+                s_bs[r] = d.x - off;
+                s_a[r] = __int_as_float(d.z);
+                if (d.y > 0) atomicOr(&s_mask[off >> 5], 1u << (off & 31));
+            }
+            products += total;
+        }
+        __syncthreads();
+        const RunWindows runs = load_windows(s_mask, 0);
+        constexpr int kGroup = 4;  // windows whose gathers are issued together
 #pragma unroll
-        for (int j = 0; j < kPerB; ++j) {
-            const int q = lo + j;
-            if (q < n) {
-                s_col[q] = static_cast<unsigned short>(kk[j] & low);
-                s_pv[pad(q)] = vv[j];
+        for (int g = 0; g < kPerB; g += kGroup) {
+            if ((g * kWaves + w) * dev::kWave >= n) break;  // uniform
+            int2 e[kGroup];
+            float av[kGroup];
+#pragma unroll
+            for (int j = 0; j < kGroup; ++j) {
+                const int i = (g + j) * kWaves + w;
+                const int r = runs.run(i);
+                e[j] = cv_b[s_bs[r] + min(i * dev::kWave + l, n - 1)];
+                av[j] = s_a[r];
+            }
+#pragma unroll
+            for (int j = 0; j < kGroup; ++j) {
+                const int q = ((g + j) * kWaves + w) * dev::kWave + l;
+                if (q < n) {
+                    s_col[q] = static_cast<unsigned short>(e[j].x & low);
+                    s_pv[q] = av[j] * __int_as_float(e[j].y);
+                }
             }
         }
     }
     __syncthreads();
-    const int w = threadIdx.x / dev::kWave, l = dev::lane();
     unsigned *bm = s_bits[w];
     int *pre = s_pre[w];
     // accumulate each bucket by rank; its distinct columns (window offsets, in order) and
     // their sums are left in its own product range, s_col / s_acc[x0 + rank]
     constexpr int kWordsPerLane = kBitmapWords / dev::kWave;
+    static_assert(kWordsPerLane == 4, "a lane's words are one 16-byte access");
+    // exclusive popcount prefix per word (lane l owns words [4 l, 4 l + 4)); the bucket's count
+    auto ranks = [&]() {
+        const uint4 m = reinterpret_cast<const uint4 *>(bm)[l];
+        const int c0 = __popc(m.x), c1 = c0 + __popc(m.y), c2 = c1 + __popc(m.z);
+        const int mine = c2 + __popc(m.w);
+        const int incl = dev::wave_inclusive_sum_dpp(mine);
+        const int run = incl - mine;
+        reinterpret_cast<int4 *>(pre)[l] = make_int4(run, run + c0, run + c1, run + c2);
+        wave_sync();
+        return incl;
+    };
+    auto rank_of = [&](int c) {
+        return pre[c >> 5] + __popc(bm[c >> 5] & ((1u << (c & 31)) - 1u));
+    };
+    int *s_ocol = reinterpret_cast<int *>(s_pv);
     // Buckets differ widely in size: a wavefront that finishes one claims the next.
     for (int o = w; o < n_buckets;) {  // uniform per wavefront
-        const int x0 = s_x0[o], x1 = s_x0[o + 1];
+        const int x0 = __builtin_amdgcn_readfirstlane(s_x0[o]);
+        const int x1 = __builtin_amdgcn_readfirstlane(s_x0[o + 1]);
         for (int x = x0 + l; x < x1; x += dev::kWave) s_acc[x] = 0.0;
-        mark_bucket(bm, s_col, x0, x1);
-        // exclusive popcount prefix per word; lane l owns words [l*4, l*4 + 4)
-        int pc[kWordsPerLane];
-        int mine = 0;
+        int distinct = 0;
+        if (x1 - x0 <= kHeld * dev::kWave) {
+            // columns, values and ranks stay in registers
+            int c[kHeld];
+            float v[kHeld];
+            reinterpret_cast<uint4 *>(bm)[l] = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
-        for (int i = 0; i < kWordsPerLane; ++i) {
-            pc[i] = __popc(bm[l * kWordsPerLane + i]);
-            mine += pc[i];
-        }
-        const int incl = dev::wave_inclusive_sum(mine);
-        int run = incl - mine;
+            for (int g = 0; g < kHeld; g += 4) {
+                if (x0 + g * dev::kWave >= x1) break;  // uniform
 #pragma unroll
-        for (int i = 0; i < kWordsPerLane; ++i) {
-            pre[l * kWordsPerLane + i] = run;
-            run += pc[i];
-        }
-        wave_sync();
-        for (int xb = x0 + l; xb < x1; xb += 4 * dev::kWave) {
-            // every read of four products first (clamped to the bucket), then the adds
-            float vv[4];
-            int r[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int x = min(xb + j * dev::kWave, x1 - 1);
-                vv[j] = s_pv[pad(x)];
-                const int c = s_col[x];
-                const int wd = c >> 5;
-                r[j] = pre[wd] + __popc(bm[wd] & ((1u << (c & 31)) - 1u));
+                for (int j = g; j < g + 4; ++j) {
+                    const int x = min(x0 + j * dev::kWave + l, x1 - 1);
+                    c[j] = s_col[x];
+                    v[j] = s_pv[x];
+                }
             }
+            wave_sync();
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (xb + j * dev::kWave < x1) atomicAdd(&s_acc[x0 + r[j]], static_cast<double>(vv[j]));
+            for (int j = 0; j < kHeld; ++j) {
+                if (x0 + j * dev::kWave + l < x1) atomicOr(&bm[c[j] >> 5], 1u << (c[j] & 31));
+            }
+            wave_sync();
+            distinct = ranks();
+#pragma unroll
+            for (int g = 0; g < kHeld; g += 4) {
+                if (x0 + g * dev::kWave >= x1) break;  // uniform
+                int r[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) r[j] = rank_of(c[g + j]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (x0 + (g + j) * dev::kWave + l < x1) {
+                        atomicAdd(&s_acc[x0 + r[j]], static_cast<double>(v[g + j]));
+                        s_ocol[x0 + r[j]] = c[g + j];
+                    }
+                }
+            }
+        } else {
+            mark_bucket(bm, s_col, x0, x1);
+            distinct = ranks();
+            for (int xb = x0 + l; xb < x1; xb += 4 * dev::kWave) {
+                // every read of four products first (clamped to the bucket), then the adds
+                float vv[4];
+                int r[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int x = min(xb + j * dev::kWave, x1 - 1);
+                    vv[j] = s_pv[x];
+                    r[j] = rank_of(s_col[x]);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (xb + j * dev::kWave < x1) {
+                        atomicAdd(&s_acc[x0 + r[j]], static_cast<double>(vv[j]));
+                    }
+                }
+            }
+            wave_sync();  // every product value of the bucket is read: its slots take the columns
+            // Each product writes its column at its rank into the bucket's own product-value
+            // slots (s_pv), so the distinct columns land there in order; products of one
+            // column write the same word.  Four products per lane per round, as above.
+            for (int xb = x0 + l; xb < x1; xb += 4 * dev::kWave) {
+                int c[4], r[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    c[j] = s_col[min(xb + j * dev::kWave, x1 - 1)];
+                    r[j] = rank_of(c[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (xb + j * dev::kWave < x1) s_ocol[x0 + r[j]] = c[j];
+                }
             }
         }
-        wave_sync();  // every product value of the bucket is read: its slots take the columns
-        // Each product writes its column at its rank into the bucket's own product-value
-        // slots (s_pv), so the distinct columns land there in order; products of one column
-        // write the same word.  Four products per lane per round, as in the adds above.
-        int *s_ocol = reinterpret_cast<int *>(s_pv);
-        for (int xb = x0 + l; xb < x1; xb += 4 * dev::kWave) {
-            int c[4], r[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int x = min(xb + j * dev::kWave, x1 - 1);
-                c[j] = s_col[x];
-                const int wd = c[j] >> 5;
-                r[j] = pre[wd] + __popc(bm[wd] & ((1u << (c[j] & 31)) - 1u));
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (xb + j * dev::kWave < x1) s_ocol[pad(x0 + r[j])] = c[j];
-            }
-        }
-        if (l == dev::kWave - 1) s_out[o] = incl;  // the bucket's distinct columns
+        if (l == dev::kWave - 1) s_out[o] = distinct;  // the bucket's distinct columns
         wave_sync();
         int claim = 0;
         if (l == 0) claim = atomicAdd(&s_next, 1);
-        o = __shfl(claim, 0, dev::kWave);
+        o = __builtin_amdgcn_readfirstlane(claim);
     }
     __syncthreads();
     // output offset of each bucket inside the unit
@@ -1151,18 +1262,16 @@ __global__ __launch_bounds__(kBitmapBlock) void bitmap_unit_kernel(
     // the unit's entries, consecutive lanes on consecutive outputs: output i belongs to the
     // last bucket whose offset is at most i (a lane's outputs only move forward)
     int o = 0;
-    const int64_t out = seg_out ? seg_out[s0] : start;
     for (int i = threadIdx.x; i < total; i += kBitmapBlock) {
         while (o + 1 < n_buckets && s_out[o + 1] <= i) ++o;
         const int x = s_x0[o] + (i - s_out[o]);
-        ukey[out + i] = s_base[o] + reinterpret_cast<const int *>(s_pv)[pad(x)];
+        ukey[out + i] = s_base[o] + reinterpret_cast<const int *>(s_pv)[x];
         uval[out + i] = static_cast<float>(s_acc[x]);
     }
     // rows starting in this unit, and the unit's count
     if (static_cast<int>(threadIdx.x) < n_buckets) {
-        const int sg = s_sid[threadIdx.x];
-        const int r = seg_row[sg];
-        if (row_off[r] == seg_off[sg]) {
+        const int r = s_row[threadIdx.x];
+        if (r >= 0) {
             row_unit[r] = static_cast<int>(u);
             row_local[r] = s_out[threadIdx.x];
         }
@@ -1176,11 +1285,12 @@ __global__ __launch_bounds__(kBitmapBlock) void bitmap_unit_kernel(
 // accumulator allows two resident workgroups per CU, so the workgroup is wide.  The
 // segment's column range [bucket << shift, (bucket + 1) << shift) is accumulated kDenseCols
 // columns at a time in an LDS float64 array (plus a bitmap of touched columns), then
-// compacted in column order, 16 columns per lane.
+// compacted in column order, 16 columns per lane.  At R-MAT scale 20 (577,000 units) 14.9 ms.
+// Twice the wavefronts (1024 threads) took 1.0 ms more, and outputs compacted in LDS and stored
+// with consecutive lanes on consecutive outputs 0.4 ms more: neither bounds it.
 constexpr int kDenseBlock = 512;
-// Products per lane per round: 8 (C4 dense units 16.2 ms; 4: 16.8, 6: 16.2, 12: 16.6,
-// 16: 18.5) keeps eight gathers in flight per lane for one run search.
-constexpr int kDensePer = 8;
+constexpr int kDenseWaves = kDenseBlock / dev::kWave;
+constexpr int kDenseGroup = 4;  // windows whose gathers are issued together
 
 __global__ __launch_bounds__(kDenseBlock) void dense_unit_kernel(
     const int *__restrict__ dense_list, const int *__restrict__ unit_seg,
@@ -1194,15 +1304,21 @@ __global__ __launch_bounds__(kDenseBlock) void dense_unit_kernel(
     __shared__ double s_acc[kDenseCols];
     __shared__ unsigned s_bits[kDenseCols / 32];
     __shared__ int s_wave[kDenseBlock / dev::kWave];
-    // a batch of up to kDenseBlock runs: first product offset, B entry of product 0, A value
-    __shared__ int s_off[kDenseBlock];
+    // a batch of up to kDenseBlock runs: B entry of the batch's product 0, A value
     __shared__ int s_bs[kDenseBlock];
     __shared__ float s_a[kDenseBlock];
+    __shared__ __align__(8) unsigned s_mask[kTile / 32];  // a round's run starts
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / dev::kWave), l = dev::lane();
     static_assert(kDenseCols / 16 == kDenseBlock, "16 bitmap bits per lane");
     const int64_t u = dense_list[dev::xcd_block<kXcdGroup>()];
     const int s = unit_seg[u];
     const int64_t start = unit_start[u];
     const int row = seg_row[s];
+    // (the unit's tables and first runs up front, as in a bitmap unit)
+    const int64_t r0 = seg_roff[s], r1 = seg_roff[s + 1];
+    const int64_t seg_first = seg_out ? seg_out[s] : start;
+    const int64_t lane_run = r0 + threadIdx.x;
+    const int4 d0 = desc[min(lane_run, r1 - 1)];
     const int64_t bucket = s - seg_prefix[row];
     const int64_t c_lo = bucket << shift;
     const int64_t c_hi = min(static_cast<int64_t>(cols), (bucket + 1) << shift);
@@ -1210,63 +1326,54 @@ __global__ __launch_bounds__(kDenseBlock) void dense_unit_kernel(
         row_unit[row] = static_cast<int>(u);
         row_local[row] = 0;
     }
-    int64_t written = seg_out ? seg_out[s] : start;
+    int64_t written = seg_first;
     const int64_t out0 = written;
     for (int64_t w0 = c_lo; w0 < c_hi; w0 += kDenseCols) {
         for (int i = threadIdx.x; i < kDenseCols; i += kDenseBlock) s_acc[i] = 0.0;
         if (threadIdx.x < kDenseCols / 32) s_bits[threadIdx.x] = 0u;
         __syncthreads();
-        // runs in batches of kDenseBlock (one per lane); the batch's products are spread over
-        // the lanes, kDensePer consecutive ones per lane per round, each lane finding the run
-        // of its first product by a search of the batch's offsets and advancing from there
-        for (int64_t rb = seg_roff[s]; rb < seg_roff[s + 1]; rb += kDenseBlock) {
-            const int nr = static_cast<int>(min(static_cast<int64_t>(kDenseBlock), seg_roff[s + 1] - rb));
-            const int4 d = static_cast<int>(threadIdx.x) < nr ? desc[rb + threadIdx.x]
-                                                              : make_int4(0, 0, 0, 0);
+        // runs in batches of kDenseBlock (one per lane); the batch's products in rounds of
+        // kTile, by windows
+        for (int64_t rb = r0; rb < r1; rb += kDenseBlock) {
+            const bool mine = rb + threadIdx.x < r1;
+            const int4 d = rb == r0 ? d0 : desc[min(rb + threadIdx.x, r1 - 1)];
             int total = 0;
-            const int off = dev::block_exclusive_sum<kDenseBlock>(d.y, s_wave, total);
-            s_off[threadIdx.x] = off;
+            const int off = dev::block_exclusive_sum<kDenseBlock>(mine ? d.y : 0, s_wave, total);
             s_bs[threadIdx.x] = d.x - off;
             s_a[threadIdx.x] = __int_as_float(d.z);
-            __syncthreads();
-            for (int x0 = threadIdx.x * kDensePer; x0 < total; x0 += kDensePer * kDenseBlock) {
-                int lo = 0, hi = nr - 1;  // last run starting at or before x0
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (s_off[mid] <= x0) {
-                        lo = mid;
-                    } else {
-                        hi = mid - 1;
+            for (int x0 = 0; x0 < total; x0 += kTile) {
+                if (threadIdx.x < kTile / 32) s_mask[threadIdx.x] = 0u;
+                __syncthreads();
+                const int at = off - x0;
+                if (mine && at >= 0 && at < kTile) atomicOr(&s_mask[at >> 5], 1u << (at & 31));
+                const int before = __syncthreads_count(mine && at < 0);
+                const RunWindows runs = load_windows(s_mask, before);
+                const int left = min(total - x0, kTile);
+#pragma unroll
+                for (int g = 0; g < kTile / kDenseBlock; g += kDenseGroup) {
+                    if ((g * kDenseWaves + w) * dev::kWave >= left) break;  // uniform
+                    int2 e[kDenseGroup];
+                    float av[kDenseGroup];
+#pragma unroll
+                    for (int j = 0; j < kDenseGroup; ++j) {
+                        const int i = (g + j) * kDenseWaves + w;
+                        const int r = runs.run(i);
+                        e[j] = cv_b[s_bs[r] + x0 + min(i * dev::kWave + l, left - 1)];
+                        av[j] = s_a[r];
+                    }
+#pragma unroll
+                    for (int j = 0; j < kDenseGroup; ++j) {
+                        const int64_t c = e[j].x - w0;
+                        if (((g + j) * kDenseWaves + w) * dev::kWave + l < left && c >= 0 &&
+                            c < kDenseCols) {
+                            atomicAdd(&s_acc[c],
+                                      static_cast<double>(av[j] * __int_as_float(e[j].y)));
+                            atomicOr(&s_bits[c >> 5], 1u << (c & 31));
+                        }
                     }
                 }
-                int r = lo;
-                int qv[kDensePer];
-                float av[kDensePer];
-#pragma unroll
-                for (int q = 0; q < kDensePer; ++q) {
-                    const int x = min(x0 + q, total - 1);
-                    while (r + 1 < nr && s_off[r + 1] <= x) ++r;
-                    qv[q] = s_bs[r] + x;
-                    av[q] = s_a[r];
-                }
-                int kk[kDensePer];
-                float vv[kDensePer];
-#pragma unroll
-                for (int q = 0; q < kDensePer; ++q) {
-                    const int2 e = cv_b[qv[q]];
-                    kk[q] = e.x;
-                    vv[q] = __int_as_float(e.y);
-                }
-#pragma unroll
-                for (int q = 0; q < kDensePer; ++q) {
-                    const int64_t c = kk[q] - w0;
-                    if (x0 + q < total && c >= 0 && c < kDenseCols) {
-                        atomicAdd(&s_acc[c], static_cast<double>(av[q] * vv[q]));
-                        atomicOr(&s_bits[c >> 5], 1u << (c & 31));
-                    }
-                }
+                __syncthreads();  // the round's tables are read before the next one's
             }
-            __syncthreads();  // the batch's tables are read before the next batch
         }
         const unsigned half = (s_bits[threadIdx.x >> 1] >> ((threadIdx.x & 1) * 16)) & 0xffffu;
         int total = 0;
