@@ -100,7 +100,6 @@ static_assert(kTile == kBlock * kPer, "a unit's products are kPer per lane");
 constexpr int kPadded = kTile + kTile / 16;
 __device__ __forceinline__ int pad(int i) { return i + (i >> 4); }
 
-using dev::block_exclusive_max;
 using dev::last_le;
 
 // ---- 1-2: sizes and segments -----------------------------------------------------------
@@ -491,86 +490,13 @@ __global__ void short_runs_kernel(const int *__restrict__ pos_a, const int *__re
     }
 }
 
-// A unit's products, expanded from its runs desc[r0, r0 + R) (in segment order): run r
-// contributes (cv_b[q].x, a_r * cv_b[q].y) for q in [first_r, first_r + length_r) (cv_b: B's
-// columns and value bits interleaved, so a lane's consecutive products are one contiguous
-// span of 8-byte pairs), and the unit's
-// products [0, n) are the runs' products concatenated.  Lane t of the BLOCK-thread workgroup
-// receives positions [t * PER, (t + 1) * PER) in kk / vv (positions >= n repeat position
-// n - 1), BLOCK * PER == kTile.  Every run has at least one product, so R <= n <= kTile.
-// s_bs and s_a (R entries) and s_mark (kPadded entries) are scratch; ends synchronised, with
-// the scratch free.  The product is one float32 multiply a * b, as the reference's
-// a_ij * b_jk.
-template <int BLOCK, int PER>
-__device__ __forceinline__ void expand_runs(const int4 *__restrict__ desc, int64_t r0, int R,
-                                            int n, const int2 *__restrict__ cv_b, int *s_bs,
-                                            float *s_a, int *s_mark, int *s_wave,
-                                            int (&kk)[PER], float (&vv)[PER]) {
-    static_assert(BLOCK * PER == kTile, "a unit's products are PER per lane");
-    constexpr int kPer = PER;
-    const int base = threadIdx.x * kPer;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) s_mark[pad(base + j)] = 0;
-    int4 d[kPer];
-    int mine = 0;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int r = base + j;
-        d[j] = r < R ? desc[r0 + r] : make_int4(0, 0, 0, 0);
-        mine += d[j].y;
-    }
-    int total = 0;
-    // (its barriers also order the clears above before the marks below)
-    int off = dev::block_exclusive_sum<BLOCK>(mine, s_wave, total);
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int r = base + j;
-        if (r < R) {
-            s_bs[r] = d[j].x - off;  // product x of run r is B entry s_bs[r] + x
-            s_a[r] = __int_as_float(d[j].z);
-            if (d[j].y > 0) s_mark[pad(off)] = r + 1;
-            off += d[j].y;
-        }
-    }
-    __syncthreads();
-    int m = 0;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) m = max(m, s_mark[pad(base + j)]);
-    int cur = block_exclusive_max(m, s_wave);
-    int qv[kPer];
-    float av[kPer];
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        cur = max(cur, s_mark[pad(base + j)]);
-        const int r = max(cur - 1, 0);
-        qv[j] = s_bs[r] + min(base + j, n - 1);  // past n: the last run's last product
-        av[j] = s_a[r];
-    }
-    if (n > 0) {
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            const int2 e = cv_b[qv[j]];
-            kk[j] = e.x;
-            vv[j] = __int_as_float(e.y);
-        }
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) vv[j] = av[j] * vv[j];
-    } else {
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            kk[j] = 0;
-            vv[j] = 0.0f;
-        }
-    }
-    __syncthreads();  // every lane is done with the scratch
-}
-
 // Products by windows: the runs of up to kTile products laid end to end, each window of 64
 // consecutive products a wavefront's, lane x on product x, so that a window's gathers are
 // consecutive entries of a few runs (R-MAT scale 20: 14 products per run) and a product's run
 // costs two bit counts.  Eight consecutive products per lane instead (a search or a running
 // maximum for the first, then a walk; every gather instruction on 64 cache lines) took 35.4 ms
-// in the bitmap units and 17.3 ms in the dense units at scale 20; windows 31.4 and 15.3.  s_mask has a bit per product that starts a run (every
+// in the bitmap units, 17.3 ms in the dense units and 13.4 ms in the sort units at scale 20;
+// windows 31.4, 15.3 and 12.7.  s_mask has a bit per product that starts a run (every
 // run has at least one product); lane l of a wavefront keeps word l and the number of bits
 // before it, and a product's run is a count of bits.
 struct RunWindows {
@@ -882,6 +808,7 @@ __global__ __launch_bounds__(kBlock) void sort_unit_kernel(
     __shared__ K s_key[kPadded];
     __shared__ float s_val[kPadded];
     __shared__ int s_mark[kPadded];
+    __shared__ __align__(8) unsigned s_mask[kTile / 32];  // products that start a run
     __shared__ int s_wave[kBlock / dev::kWave];
     __shared__ double s_sum[kBlock / dev::kWave];
     __shared__ int s_flag[kBlock / dev::kWave];
@@ -890,22 +817,55 @@ __global__ __launch_bounds__(kBlock) void sort_unit_kernel(
     const int64_t start = unit_start[u];
     const int n = static_cast<int>(unit_start[u + 1] - start);
     const int64_t s_end = u + 1 < n_units ? unit_seg[u + 1] : n_seg;
+    const int64_t r0 = seg_roff[s0];
+    const int R = static_cast<int>(seg_roff[s_end] - r0);
+    int4 d = desc[r0 + min(static_cast<int>(threadIdx.x), R - 1)];
+    if (threadIdx.x < kTile / 32) s_mask[threadIdx.x] = 0u;
+    __syncthreads();
     {
-        // the unit's products from its runs, then staged in LDS (blocked positions)
-        int kk[kPer];
-        float vv[kPer];
-        const int64_t r0 = seg_roff[s0];
-        const int R = static_cast<int>(seg_roff[s_end] - r0);
-        expand_runs<kBlock, kPer>(desc, r0, R, n, cv_b, reinterpret_cast<int *>(s_key),
-                                  s_val, s_mark, s_wave, kk, vv);
-        const int lo = threadIdx.x * kPer;
+        // the unit's products from its runs, by windows, held in registers until every lane is
+        // done with the runs' tables, then staged in LDS
+        constexpr int kWaves = kBlock / dev::kWave;
+        const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / dev::kWave), l = dev::lane();
+        int *s_bs = reinterpret_cast<int *>(s_key);  // product 0's B entry
+        float *s_a = s_val;                          // A value
+        int products = 0;
+        for (int rb = 0; rb < R; rb += kBlock) {  // uniform
+            const int r = rb + static_cast<int>(threadIdx.x);
+            if (rb > 0) d = desc[r0 + min(r, R - 1)];
+            int total = 0;
+            const int off =
+                products + dev::block_exclusive_sum<kBlock>(r < R ? d.y : 0, s_wave, total);
+            if (r < R) {
+                s_bs[r] = d.x - off;
+                s_a[r] = __int_as_float(d.z);
+                if (d.y > 0) atomicOr(&s_mask[off >> 5], 1u << (off & 31));
+            }
+            products += total;
+        }
+        __syncthreads();
+        const RunWindows runs = load_windows(s_mask, 0);
+        int2 e[kPer];
+        float av[kPer];
+#pragma unroll
+        for (int g = 0; g < kPer; g += 4) {
+            if ((g * kWaves + w) * dev::kWave >= n) break;  // uniform
+#pragma unroll
+            for (int j = g; j < g + 4; ++j) {
+                const int i = j * kWaves + w;
+                const int r = runs.run(i);
+                e[j] = cv_b[s_bs[r] + min(i * dev::kWave + l, n - 1)];
+                av[j] = s_a[r];
+            }
+        }
+        __syncthreads();
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
-            const int q = lo + j;
+            const int q = (j * kWaves + w) * dev::kWave + l;
             s_mark[pad(q)] = 0;
             if (q < n) {
-                s_key[pad(q)] = static_cast<K>(static_cast<uint32_t>(kk[j]));
-                s_val[pad(q)] = vv[j];
+                s_key[pad(q)] = static_cast<K>(static_cast<uint32_t>(e[j].x));
+                s_val[pad(q)] = av[j] * __int_as_float(e[j].y);
             }
         }
     }
