@@ -69,50 +69,47 @@ PEAK_HBM_GBS = 8000.0
 ROTATE = 4  # independent operand copies cycled through by the timed steps
 
 WORKLOADS = {
-    "c2": dict(op="add", kernel="csr_partition_kernel (with the row pass) + "
-                              "csr_pair_count_kernel (pair search) + csr_write_kernel<Union> "
+    "c2": dict(op="add", kernel="split_sparse_kernel + order_kernel + emit_kernel<Union> "
                               "(one call's device pipeline)",
                desc="C2 csr_add f32 2^20x2^20, Zipf(1.6) rows rescaled to mean 16 "
                     "(16.7M nnz each), seeds 1/2"),
-    "c3": dict(op="mul", kernel="csr_partition_kernel + csr_write_kernel<Intersect> (spread) "
-                              "+ csr_compact_kernel (one call's device pipeline)",
+    "c3": dict(op="mul", kernel="csr_partition_kernel + order_kernel + "
+                              "emit_kernel<Intersect> (one call's device pipeline)",
                desc="C3 csr_mul f32 2^20x2^20, A as C2, B = 50% of A + fresh columns "
                     "(seed 3)"),
-    "c5": dict(op="csf_add", kernel="three chained level merges (csr_partition_kernel + "
-                                   "csr_pair_count_kernel + csr_write_kernel per level)",
+    "c5": dict(op="csf_add", kernel="three chained level merges (fused_kernel, or "
+                                   "csr_partition_kernel + order_kernel + emit_kernel)",
                desc="C5 csf_add f32, two CSF3 tensors of shape (200000, 100000, 1000), 20M "
                     "draws each (mode 0 Zipf(1.3), modes 1-2 uniform), deduplicated, seeds 1/2"),
     "c5coo": dict(op="coo3d_add", kernel="coo3_keys_kernel (row offsets, (j, k) keys) + "
-                                         "csr_partition_kernel + csr_pair_count_kernel + "
-                                         "csr_write_kernel<Union> (rows out, keys split)",
+                                         "csr_partition_kernel + order_kernel + "
+                                         "emit_kernel<Union> (rows out, keys split)",
                   desc="C5 as COO3: coo3d_add f32 of the same (i, j, k) tuples"),
     "c3coo": dict(op="coo_mul", kernel="coo_row_offsets_kernel + csr_partition_kernel + "
-                                      "csr_write_kernel<Intersect> (spread, rows out) + "
-                                      "csr_compact_kernel",
+                                      "order_kernel + emit_kernel<Intersect> (rows out)",
                   desc="C3 as COO: coo_mul f32 of the C3 operands' (i, j) tuples"),
-    "c2coo": dict(op="coo_add", kernel="coo_row_offsets_kernel + csr_partition_kernel + "
-                                      "csr_pair_count_kernel + csr_write_kernel<Union> (rows out)",
+    "c2coo": dict(op="coo_add", kernel="coo_row_offsets_kernel + split_sparse_kernel + "
+                                      "order_kernel + emit_kernel<Union> (rows out)",
                   desc="C2 as COO: coo_add f32 of the C2 operands' (i, j) tuples"),
     "c2add3": dict(op="add3", kernel="fused three-way merge (csr3_partition_kernel + "
                                     "csr3_count_kernel + csr3_write_kernel)",
                    desc="csr_add_3 f32: three C2 operands (Zipf(1.6) rows, 16.7M nnz each, "
                         "seeds 1, 2, 4)"),
-    "c2dcsr": dict(op="dcsr_add", kernel="two chained level merges (csr_partition_kernel + "
-                                        "csr_pair_count_kernel + csr_write_kernel per level)",
+    "c2dcsr": dict(op="dcsr_add", kernel="two chained level merges (partition, order_kernel + "
+                                        "emit_kernel per level)",
                    desc="C2 as DCSR: dcsr_add f32 of the C2 operands with empty rows "
                         "dropped"),
     "c5inner": dict(op="inner_prod", kernel="csf_row_offsets_kernel + csf_keys_kernel + "
-                                          "csr_partition_kernel + csr_write_kernel<Intersect> "
-                                          "(spread) + dot_tiles_kernel + dot_final_kernel",
+                                          "csr_partition_kernel + order_kernel + "
+                                          "emit_kernel<Intersect> (products) + dot_final_kernel",
                     desc="inner_prod f32 of the C5 CSF3 operands: sum of a*b over the "
                          "(i, j, k) both hold"),
     "c5innercoo": dict(op="inner_prod_coo", kernel="coo3_keys_kernel + csr_partition_kernel + "
-                                                   "csr_write_kernel<Intersect> (spread) + "
-                                                   "dot_tiles_kernel + dot_final_kernel",
+                                                   "order_kernel + emit_kernel<Intersect> "
+                                                   "(products) + dot_final_kernel",
                        desc="inner_prod_coo f32 of the C5 operands as COO3"),
-    "c2coocsr": dict(op="coo_csr_add", kernel="coo_row_offsets_kernel + csr_partition_kernel "
-                                             "(with the row pass) + csr_pair_count_kernel + "
-                                             "csr_write_kernel<Union>",
+    "c2coocsr": dict(op="coo_csr_add", kernel="coo_row_offsets_kernel + split_sparse_kernel + "
+                                             "order_kernel + emit_kernel<Union>",
                      desc="coo_csr_add f32: the C2 operands, A as CSR and B as COO"),
     "c3dcsr": dict(op="dcsr_mul", kernel="two chained level merges + row compaction",
                    desc="C3 as DCSR: dcsr_mul f32 of the C3 operands with empty rows "

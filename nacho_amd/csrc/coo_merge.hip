@@ -11,7 +11,7 @@
 // Coordinates are non-negative int32 below their extents, so key order is tuple order.
 // The work is the merged sequence of both key lists (nnzA + nnzB items), cut into tiles.  A
 // partition kernel finds every tile's merge-path split (equal keys never split, as the
-// reference's balancing step, partition.cpp:964-983).  As for CSR (csr_merge.hip), each
+// reference's balancing step, partition.cpp:964-983).  Each
 // workgroup then owns a fixed chunk of tiles: a count kernel stores each chunk's output count
 // and a write kernel starts from the preceding chunks' total.  Inside a tile the keys and
 // values are staged in LDS from registers loaded one tile ahead, lanes split the tile by a
@@ -580,9 +580,8 @@ int coo_binary(int arity, const int32_t extents[3], Coords ca, const float *va, 
 //
 // A 2-D COO operand sorted by (i, j) is a CSR matrix without its offsets.  When the rows are
 // not far more than the entries, coo_add / coo_mul build both operands' row offsets (one
-// pass over i), run the CSR level merge (csr_merge.hip: pair-count union or spread
-// intersection), and take each output's row from the write kernel, which knows it: the
-// result is the same sequence of (i, j, value) as the merged-coordinate path.
+// pass over i), run the level merge (level_merge.hip), and take each output's row from its
+// emit kernel: the result is the same sequence of (i, j, value) as the merged-coordinate path.
 
 // pos[r] = the first entry whose row is >= r, r in [0, rows].  Entry p writes the rows after
 // the previous entry's row up to its own, and the position nnz closes the last rows (row
@@ -696,8 +695,8 @@ int coo2_rows(const nacho_coo *a, const nacho_coo *b, nacho_coo *z, void *stream
 // lexicographic order.  When the j and k extents fit 31 bits together and the largest key
 // stays below INT_MAX, the column key j << kbits | k (kbits = bits of the k extent) orders
 // entries as (j, k) does, so coo3d_add
-// builds both operands' row offsets and keys in one pass, runs the CSR level union on them,
-// and the write kernel stores each output key split back into j and k, with its row as i.
+// builds both operands' row offsets and keys in one pass, runs the level union on them, and
+// the emit kernel stores each output key split back into j and k, with its row as i.
 
 struct KeysJob {
     const int *ci, *cj, *ck;

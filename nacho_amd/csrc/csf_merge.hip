@@ -4,7 +4,7 @@
 // three nested levels with runtime exclusion (partition.cpp:286-461, 551-584) and emit the
 // i, j and k levels with one count/scan/readback per level (stitch_and_generate_gpu.cpp:
 // 641-715).  The union of two trees is computed here as three chained level merges, each
-// the CSR merge of csr_merge.hip:
+// a row-by-row merge of level_merge.hip:
 //   i level: one "row" holding both operands' i coordinates; every output i records the
 //            positions reached in A and B, which index their j offsets (child pointers);
 //   j level: rows are the output i fibres, each row's A/B ranges given by those child

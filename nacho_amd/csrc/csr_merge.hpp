@@ -42,8 +42,11 @@ struct LevelResult {
 };
 
 // Headroom merge_level keeps below INT_MAX for its item count (entries of both operands plus
-// rows): it refuses larger levels with NACHO_ERR_INDEX_OVERFLOW.
+// rows): it refuses larger levels with NACHO_ERR_INDEX_OVERFLOW.  Callers that choose between
+// it and another path keep 2 * kLevelTileSlack.
+constexpr long long kLevelItemSlack = 7680;
 constexpr long long kLevelTileSlack = 4096;
+static_assert(kLevelItemSlack <= 2 * kLevelTileSlack, "what callers route here is taken");
 
 // Merge A and B row by row: union (or intersection) of each row's coordinates, with values
 // (a+b / a*b / copies) when `values`, or with child pointers when `child` (unions only).

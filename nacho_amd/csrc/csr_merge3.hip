@@ -6,7 +6,7 @@
 // (compute.cpp:1297-1337, lattice points with absent operands removed); its benchmark
 // compares that fused kernel with two chained csr_add calls (benchmarks/csr_add_3.py:21-29).
 //
-// Structure (the two-operand csr_merge.hip pipeline, widened to three operands):
+// Structure (a count walk and a write walk over tiles of three merged operands):
 //  * Items are every row's A, B and C entries plus one row-end item; T = nnzA + nnzB + nnzC
 //    + rows items are cut into tiles of kTile.
 //  * csr3_partition_kernel: one thread per tile boundary.  The row comes from a binary search

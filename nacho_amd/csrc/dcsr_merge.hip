@@ -5,7 +5,7 @@
 // (compiler.cpp:124-133).  Their generated kernels partition the two compressed levels
 // (partition.cpp:286-461; dcsr_mul re-partitions at the inner intersection) and emit the i
 // and j levels with one count/scan/readback per level (stitch_and_generate_gpu.cpp:641-715).
-// Both levels are CSR level merges here (csr_merge.hip):
+// Both levels are level merges here (level_merge.hip):
 //   add: i level = one "row" holding both operands' row coordinates; each output row records
 //        the operands' j offsets reached (child pointers), which are the j level's row
 //        offsets; the j level is a CSR add over those rows.

@@ -56,7 +56,7 @@ constexpr int kSlots = kBlock * kPer;   // merged entries of a tile, padded
 // stays between a tile's A and B slots.
 constexpr int kTile = kSlots - dev::kWave - 1;
 constexpr int kWords = kSlots / 64;     // 64-slot order words per tile
-static_assert(kLevelTileSlack >= kTile, "callers' item-count headroom covers merge_level's");
+static_assert(kLevelItemSlack >= kTile, "an item count rounded up to tiles fits 32 bits");
 static_assert(kWords == dev::kWave, "one order word per lane");
 // Tiles per pair total: a wavefront of the emit kernel sums the chunks before its tile's and
 // the tiles before it in its own chunk (at most 2^31 / kTile / kChunk + kChunk loads).
@@ -1182,7 +1182,7 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
                 long long *out_len, const char *kernel_name, bool *length_pending) {
     if (length_pending) *length_pending = false;
     const long long total = static_cast<long long>(A.len) + B.len + rows;
-    if (total > static_cast<long long>(INT_MAX) - 2 * kLevelTileSlack) {
+    if (total > static_cast<long long>(INT_MAX) - kLevelItemSlack) {
         return NACHO_ERR_INDEX_OVERFLOW;
     }
     // the kinds of level this merge knows
