@@ -1,0 +1,65 @@
+"""The products' size rules at their limits: scans of up to four chunks of 4096 in one launch and
+longer ones in two, SpGEMM with and without long rows and past the run count that is bounded
+instead of counted (2^22 products), sssmm chunks of more mask entries than keep their fields and
+sums in LDS (256)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle import oracle
+from tests.helpers import csr_from_rows, random_csr
+from tests.test_gpu_spgemm import run_and_check
+from tests.test_gpu_sssmm import check as check_sssmm
+from tests.test_gpu_sssmm import run as run_sssmm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows", [4095, 4096, 4097, 16383, 16384, 16385, 20481])
+def test_scans_at_chunk_limits(gpu, rows):
+    rng = np.random.default_rng(rows)
+    a = random_csr(rng, rows, 64, 0.02)
+    b = random_csr(rng, 64, 500, 0.05)
+    run_and_check(gpu, rows, 64, 500, a, b, f"{rows} rows")
+
+
+@pytest.mark.parametrize("long_rows", [0, 1, 3])
+def test_with_and_without_long_rows(gpu, long_rows):
+    """Rows of at most 20 products, and `long_rows` rows of 2500 among them."""
+    rng = np.random.default_rng(long_rows)
+    n = 600
+    rows_a = [[int(r) % n, (int(r) * 7 + 1) % n] for r in range(n)]
+    rows_a = [sorted(set(r)) for r in rows_a]
+    for i in range(long_rows):
+        rows_a[100 * i + 50] = list(range(0, n, 2))
+    nnz_a = sum(len(r) for r in rows_a)
+    a = csr_from_rows(n, n, rows_a, rng.uniform(0.5, 1.5, nnz_a).astype(np.float32))
+    b = random_csr(rng, n, 40000, 9 / 40000)
+    run_and_check(gpu, n, n, 40000, a, b, f"{long_rows} long rows")
+
+
+@pytest.mark.parametrize("length", [2047, 2049])
+def test_runs_bounded_and_counted(gpu, length):
+    """2048 rows of `length` products: either side of 2^22 products."""
+    rng = np.random.default_rng(length)
+    n = 2048
+    a = csr_from_rows(n, n, [[i] for i in range(n)], rng.uniform(0.5, 1.5, n).astype(np.float32))
+    rows_b = [np.sort(rng.choice(8192, size=length, replace=False)).tolist() for _ in range(n)]
+    b = csr_from_rows(n, 8192, rows_b, rng.uniform(-1, 1, n * length).astype(np.float32))
+    run_and_check(gpu, n, n, 8192, a, b, f"rows of {length}")
+
+
+@pytest.mark.parametrize("probes", [1, 15, 16, 17, 300])
+def test_sssmm_entries_per_chunk(gpu, probes):
+    """Mask entries of `probes` probes each: 4096, 273, 256, 241 and 14 entries per chunk of
+    4096 probes."""
+    rng = np.random.default_rng(probes)
+    n, inner = 120, 400
+    rows_a = [np.sort(rng.choice(inner, size=probes, replace=False)).tolist() for _ in range(n)]
+    a = csr_from_rows(n, inner, rows_a, rng.uniform(0.5, 1.5, n * probes).astype(np.float32))
+    b = random_csr(rng, inner, 100, 0.9)  # columns longer than the rows of A
+    c = random_csr(rng, n, 100, 0.8)
+    check_sssmm(run_sssmm(a, b, c, ((n, inner), (inner, 100), (n, 100)), gpu),
+                oracle.port_sssmm(n, 100, a, b, c), f"{probes} probes")
