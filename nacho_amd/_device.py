@@ -1,7 +1,8 @@
 """Device plumbing between torch and the C ABI: streams, and adopting result buffers.
 
 Result buffers come back from libnacho_hip.so as raw device pointers owned by the caller
-(allocated by the library's caching allocator over hipMalloc).  `adopt` wraps one in a torch
+(allocated by the library's caching allocator over hipMalloc).  The `gpu_` entry points wrap
+theirs in C++ (bridge/bridge.cpp); for callers of the C ABI, `adopt` wraps one in a torch
 tensor without copying; when the last tensor referencing it is collected the buffer is
 released with `nacho_free` on the stream it was produced on.  Work on another stream that
 reads a result must be announced with `record_stream` (torch's own `Tensor.record_stream`

@@ -5,8 +5,8 @@
 // reference's generated nanobind wrapper does (src/backend/generate_bindings.cpp:288-327,
 // runtime/nacho_nb.h:37-58).
 //
-// The same steps through ctypes and __cuda_array_interface__ cost about 11 us per call, more
-// than the kernels of a small merge; this takes about 2.
+// The same steps through ctypes and __cuda_array_interface__ cost about 11 us more per call, as
+// much as the kernels of a small merge: csr_add of 200 rows 25.2 -> 14.5 us.
 //
 // An operand that does not pass the checks here (lengths, devices) makes invoke() return None:
 // the caller (ops.py) then raises the exception that names what is wrong.
