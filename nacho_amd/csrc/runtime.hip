@@ -377,6 +377,7 @@ Call::Call(void *stream, void *arena, size_t arena_bytes)
 
 Call::~Call() {
     if (arena_) return;  // nothing was allocated
+    if (words_unread_ != 0) (void)hipStreamSynchronize(stream_);  // a queued store may be late
     if (sync_held_) {
         int device = 0;
         (void)hipGetDevice(&device);
@@ -497,6 +498,7 @@ int Call::length_word(int64_t **dev) {
     }
     NACHO_TRY(ensure_len_words());
     *t_len_host = -1;  // a kernel that did not store would show as an impossible length
+    words_unread_ |= 1u;
     *dev = t_len_dev;
     return NACHO_OK;
 }
@@ -509,6 +511,7 @@ int Call::side_word(int64_t **dev) {
     }
     NACHO_TRY(ensure_len_words());
     t_len_host[1] = -1;
+    words_unread_ |= 2u;
     *dev = t_len_dev + 1;
     return NACHO_OK;
 }
@@ -558,6 +561,7 @@ int Call::side_value(int64_t *v) {
         // that stores the length; it is waited for in the same way.
         if (!len_marked_) return NACHO_ERR_INTERNAL;
         NACHO_TRY(spin_for_word(t_len_host + 1, stream_, v));
+        words_unread_ &= ~2u;
     }
     return *v < 0 ? NACHO_ERR_INTERNAL : NACHO_OK;
 }
@@ -566,13 +570,16 @@ int Call::value_word(int i, int64_t **dev) {
     if (arena_ || i < 0 || i >= kValueWords) return NACHO_ERR_INVALID_ARGUMENT;
     NACHO_TRY(ensure_len_words());
     t_len_host[2 + i] = -1;
+    words_unread_ |= 4u << i;
     *dev = t_len_dev + 2 + i;
     return NACHO_OK;
 }
 
 int Call::value(int i, int64_t *v) {
     if (arena_ || i < 0 || i >= kValueWords) return NACHO_ERR_INVALID_ARGUMENT;
-    return spin_for_word(t_len_host + 2 + i, stream_, v);
+    NACHO_TRY(spin_for_word(t_len_host + 2 + i, stream_, v));
+    words_unread_ &= ~(4u << i);
+    return NACHO_OK;
 }
 
 int Call::mark_length() {
@@ -591,6 +598,7 @@ int Call::wait_length(int64_t *len) {
     }
     if (!len_marked_) return NACHO_ERR_INTERNAL;
     NACHO_TRY(spin_for_word(t_len_host, stream_, len));
+    words_unread_ &= ~1u;
     return collect_timer();
 }
 

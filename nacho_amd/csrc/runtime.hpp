@@ -114,6 +114,11 @@ class Call {
     // kernel stores a value >= 0 to it (system scope), and value(i) waits for it as
     // wait_length does.  A blocking copy of a count took about 15 us, this wait about 3.  Not
     // for arena calls.
+    //
+    // The words are the host thread's, and its next call sets them anew from the host, out of
+    // stream order.  A call that ends with a word (length, side or value) handed out and not
+    // read, as when an allocation fails after the kernel that stores it was queued, therefore
+    // waits for its stream first: the late store would be taken for the next call's count.
     static constexpr int kValueWords = 6;
     int value_word(int i, int64_t **dev);
     int value(int i, int64_t *v);
@@ -144,6 +149,7 @@ class Call {
     int64_t *arena_side_ = nullptr;
     bool timed_ = false;
     bool sync_held_ = false, sync_sound_ = true;
+    unsigned words_unread_ = 0;  // pinned words handed out and not read: bit per word
     bool len_marked_ = false;  // mark_length: this call launched the kernel storing its length
     float timed_ms_ = 0.0f;  // sum of this call's bracketed intervals
 };

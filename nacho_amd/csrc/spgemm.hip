@@ -1969,7 +1969,7 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
         // count.
         int64_t n_runs = P, nnz_sym = 0;
         const bool count_runs = P > kBoundRuns;
-        NACHO_TRY(words(1));
+        if (count_runs) NACHO_TRY(words(1));
         const scan::Job seg_jobs[2] = {{seg_len, n_seg, seg_off},
                                        {seg_runs, n_seg, seg_roff, count_runs ? word[0] : nullptr}};
         NACHO_TRY(scan::exclusive_scans(call, seg_jobs, 2));
