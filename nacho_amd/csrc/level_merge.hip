@@ -1223,7 +1223,21 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
         const unsigned tickets = num_tiles > 1 ? num_tiles : 0;
         NACHO_TRY(call.sync_block(kSyncBytes, tickets, Z.dot ? tickets : 0, &sync));
     }
-    if (sync.words) {
+    // A small inner product, which the host never waits for, may be recorded: each replay clears
+    // the words first.  They come with the partial sums, so that a recorded call allocates what
+    // the calls that warmed the cache up did.  (A level whose length the host waits for fails
+    // under capture.)
+    const bool recorded = Z.dot && sync.recorded;
+    if (sync.words || recorded) {
+        if (Z.dot) {
+            NACHO_TRY(call.scratch(static_cast<size_t>(num_tiles) * sizeof(double) + kSyncBytes,
+                                   reinterpret_cast<void **>(&args.partial)));
+        }
+        if (recorded) {
+            sync.words = reinterpret_cast<unsigned long long *>(args.partial + num_tiles);
+            sync.epoch = 1;
+            NACHO_TRY(clear_words(s, sync.words, kSyncBytes / sizeof(unsigned long long)));
+        }
         void (*fused)(EmitArgs, int, int, int, unsigned long long *, unsigned, unsigned,
                       unsigned, int64_t *, long long, float *) =
 #define NACHO_FUSED(OP, VAL, CHD, ROWS, DOT)             \
@@ -1237,11 +1251,7 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
                         : NACHO_FUSED(Op::Union, true, false, false, false);
 #undef NACHO_FUSED
         int64_t *length_out = nullptr;
-        if (Z.dot) {
-            NACHO_TRY(call.scratch_n(static_cast<size_t>(num_tiles), &args.partial));
-        } else {
-            NACHO_TRY(call.length_word(&length_out));
-        }
+        if (!Z.dot) NACHO_TRY(call.length_word(&length_out));
         NACHO_TRY(call.timer_start(kernel_name));
         fused<<<num_tiles, kBlock, 0, s>>>(args, rows, static_cast<int>(total), crd_bits,
                                            sync.words, sync.epoch, sync.base, sync.done, length_out, items,

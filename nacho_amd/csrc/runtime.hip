@@ -312,11 +312,10 @@ int take_sync_block(size_t bytes, unsigned tickets, unsigned finishes, hipStream
             return NACHO_OK;  // none to take
         }
         unsigned long long *words = static_cast<unsigned long long *>(p);
-        clear_words_kernel<<<1, 256, 0, stream>>>(words, bytes / sizeof(unsigned long long));
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) {
+        const int rc = clear_words(stream, words, bytes / sizeof(unsigned long long));
+        if (rc != NACHO_OK) {
             (void)hipFree(p);
-            return static_cast<int>(e);
+            return rc;
         }
         it = g_sync.insert({*key, SyncEntry{words, bytes, 0u, 0u, 0u, false}}).first;
     }
@@ -362,6 +361,12 @@ thread_local volatile int64_t *t_len_host = nullptr;
 thread_local int64_t *t_len_dev = nullptr;
 
 }  // namespace
+
+int clear_words(hipStream_t stream, unsigned long long *words, size_t n) {
+    clear_words_kernel<<<1, 256, 0, stream>>>(words, n);
+    NACHO_TRY_HIP(hipGetLastError());
+    return NACHO_OK;
+}
 
 Call::Call(void *stream, const nacho_allocator *alloc)
     : stream_(static_cast<hipStream_t>(stream)),
@@ -437,6 +442,15 @@ int Call::result(size_t bytes, void **out) {
 int Call::sync_block(size_t bytes, unsigned tickets, unsigned finishes, SyncBlock *out) {
     *out = SyncBlock{};
     if (arena_ || alloc_) return NACHO_OK;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream_, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return NACHO_OK;
+    }
+    if (capture != hipStreamCaptureStatusNone) {
+        out->recorded = true;
+        return NACHO_OK;
+    }
     SyncKey key;
     const int rc = take_sync_block(bytes, tickets, finishes, stream_, &key, out);
     if (out->words) {

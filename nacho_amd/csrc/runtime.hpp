@@ -43,7 +43,14 @@ struct SyncBlock {
     unsigned epoch;
     unsigned base;
     unsigned done;
+    // The stream is being captured, so no block was taken: what a recorded launch does to the
+    // counts at each replay is not known here.  A caller that can be recorded brings words of
+    // its own, cleared in the same capture (clear_words).
+    bool recorded;
 };
+
+// Zeroes n words by a small kernel on the stream (which, unlike a memset, may be recorded).
+int clear_words(hipStream_t stream, unsigned long long *words, size_t n);
 
 // One call's execution context: its stream and allocator, and every buffer it allocated.
 // Scratch buffers are released when the call ends; result buffers are released only if the
@@ -77,8 +84,9 @@ class Call {
     }
 
     // A sync block of at least `bytes` whose counters this call's next launch advances by
-    // `tickets` and `finishes`; kept for this stream's later calls.  words stays null where there is none to
-    // take (an arena call, or a caller's allocator, which the library keeps no memory of).
+    // `tickets` and `finishes`; kept for this stream's later calls.  words stays null where there
+    // is none to take (an arena call, a caller's allocator, which the library keeps no memory of,
+    // or a stream that is being captured).
     // sync_launched says that the launch was made: without it the block is dropped when the
     // call ends.
     int sync_block(size_t bytes, unsigned tickets, unsigned finishes, SyncBlock *out);

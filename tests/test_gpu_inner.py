@@ -273,3 +273,39 @@ def test_wide_keys_coo_through_a_caller_allocator(gpu, with_release):
         assert sorted(released) == sorted(p for p in handed if p != z.values)
     else:
         assert not released
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n", [500, 6000, 300_000, 1_200_000])
+def test_recorded_in_a_graph(gpu, kind, n):
+    """An inner product (whose host waits for nothing) recorded after calls that warmed the
+    stream's buffers up, and replayed with other values in its operands: one tile, a few, many,
+    and more than one launch takes.  Every replay equals the eager call on the same values, with
+    eager calls and synchronisations between."""
+    import nacho_amd
+
+    rng = np.random.default_rng(n)
+    shape = (300, 250, 64)
+    ac, av = random_coords(rng, shape, n)
+    bc = ac[rng.random(len(ac)) < 0.6]
+    to = nacho_amd.to_csf3 if kind == "csf" else nacho_amd.to_coo3
+    fn = nacho_amd.gpu_inner_prod_f32 if kind == "csf" else nacho_amd.gpu_inner_prod_coo_f32
+    a, b = to(ac, av, shape, gpu), to(bc, rng.uniform(-1, 1, len(bc)).astype(np.float32), shape, gpu)
+    torch.cuda.synchronize()
+    print(f"[gpu] inner_prod {kind} recorded nnz=({len(ac)},{len(bc)})", flush=True)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        for _ in range(3):
+            fn(a, b)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        z = fn(a, b)
+    for step in range(6):
+        a.values.copy_(torch.from_numpy(rng.uniform(-1, 1, len(ac)).astype(np.float32)))
+        want = fn(a, b).values.clone()  # (on the default stream)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z.values, want), (step, z.values.item(), want.item())
