@@ -416,6 +416,12 @@ const char *nacho_version(void);
 void nacho_set_kernel_timing(int enable);
 float nacho_last_kernel_ms(void);
 
+/* For tests of failure handling: how often this host thread's later calls let a workgroup look
+ * for the counts of the tiles before its own (0: the default, seconds) before it gives up, as
+ * small levels in one launch do.  A call in which a workgroup gave up returns
+ * NACHO_ERR_INTERNAL. */
+void nacho_set_wait_limit(unsigned polls);
+
 /* Name of the kernel nacho_last_kernel_ms() timed in the last call on this thread. */
 const char *nacho_last_kernel_name(void);
 

@@ -239,6 +239,8 @@ def load() -> ctypes.CDLL:
                                       ctypes.c_void_p]
     lib.nacho_version.restype = ctypes.c_char_p
     lib.nacho_version.argtypes = []
+    lib.nacho_set_wait_limit.restype = None
+    lib.nacho_set_wait_limit.argtypes = [ctypes.c_uint]
     lib.nacho_set_kernel_timing.restype = None
     lib.nacho_set_kernel_timing.argtypes = [ctypes.c_int]
     lib.nacho_last_kernel_ms.restype = ctypes.c_float

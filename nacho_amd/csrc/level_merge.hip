@@ -1009,15 +1009,21 @@ __device__ __forceinline__ void block_sum_fixed(double *sh) {
 // `sync` is a block of words that only these kernels write: two counters that keep counting
 // from launch to launch (this launch's counts start at `base` and `done_base`) and, per tile, the
 // pairs tagged with the launch's epoch, so that it is never cleared.
+//
+// Every wait is bounded, for a block whose counts are not what the host believes, and a level
+// whose length was stored is whole: the length is the last tile's to store, and it withholds it
+// where it gives up itself or sees that another tile did.  A tile that gives up says so first
+// and then waits once more, for seconds: had the last tile missed the word, every count would
+// have been published by then.
+constexpr int kSyncGaveUp = 2;  // word that holds the epoch of a launch in which a tile gave up
 constexpr int kSyncTiles = 16;  // word of tile 0
-constexpr int kMaxPolls = 1 << 22;  // seconds
 constexpr size_t kSyncBytes = (kSyncTiles + kFusedTiles) * sizeof(unsigned long long);
 
 template <Op OP, bool VALUES, bool CHILD, bool ROWS, bool DOT, bool WIDE>
 __global__ __launch_bounds__(kBlock) void fused_kernel(EmitArgs g, int rows, int total, int bits,
                                                        unsigned long long *__restrict__ sync,
                                                        unsigned epoch, unsigned base,
-                                                       unsigned done_base,
+                                                       unsigned done_base, unsigned max_polls,
                                                        int64_t *__restrict__ length_out,
                                                        long long items, float *__restrict__ dot) {
     __shared__ double s_dot[DOT ? kBlock : 1];
@@ -1034,7 +1040,10 @@ __global__ __launch_bounds__(kBlock) void fused_kernel(EmitArgs g, int rows, int
         if (tid == 0) s_ticket = static_cast<int>(atomicAdd(reinterpret_cast<unsigned *>(sync), 1u) - base);
         __syncthreads();
         t = __builtin_amdgcn_readfirstlane(s_ticket);
-        if (t < 0 || t >= g.num_tiles) return;  // (as above)
+        if (t < 0 || t >= g.num_tiles) {  // no tile: the block's counts are others
+            if (DOT && tid == 0) *dot = __builtin_nanf("");
+            return;
+        }
     }
     if (w < 2) {  // boundary t + w
         const int b = t + w;
@@ -1101,19 +1110,32 @@ __global__ __launch_bounds__(kBlock) void fused_kernel(EmitArgs g, int rows, int
     s_side[tid] = static_cast<unsigned short>(side);
     s_dup[tid] = static_cast<unsigned short>(dup);
     // (The waits end: the workgroups of the tiles before have started and wait for earlier
-    // ones only.  The bound is for a block whose counts are not what the host believes: the
-    // length is then never stored, which the host reports.)
+    // ones only.)
+    static_assert(kFusedTiles <= kBlock, "a lane waits for one tile");
+    const bool last = t == g.num_tiles - 1;
     int before = 0;
     bool found = true;
-    for (int i = tid; i < t && found; i += kBlock) {
+    if (tid < t) {
         unsigned long long v = 0;
-        int polls = 0;
-        do {
-            v = __hip_atomic_load(&sync[kSyncTiles + i], __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT);
-        } while ((v >> 32) != epoch && ++polls < kMaxPolls);
-        found = (v >> 32) == epoch;
-        if (found) before += static_cast<int>(v & 0xffffffffull);
+        auto published = [&](unsigned polls) {
+            for (unsigned i = 0; i < polls; ++i) {
+                v = __hip_atomic_load(&sync[kSyncTiles + tid], __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+                const unsigned long long gave_up =  // (issued with the load above)
+                    last ? __hip_atomic_load(&sync[kSyncGaveUp], __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT)
+                         : 0ull;
+                if ((v >> 32) == epoch) return gave_up != epoch;
+            }
+            return false;
+        };
+        found = published(max_polls);
+        if (!found && !last) {
+            __hip_atomic_store(&sync[kSyncGaveUp], static_cast<unsigned long long>(epoch),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            found = published(SyncBlock::kMaxPolls);
+        }
+        before = static_cast<int>(v & 0xffffffffull);
     }
     int pairs = 0;
     (void)dev::block_exclusive_sum<kBlock>(before, s_wave, pairs);
@@ -1239,7 +1261,7 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
             NACHO_TRY(clear_words(s, sync.words, kSyncBytes / sizeof(unsigned long long)));
         }
         void (*fused)(EmitArgs, int, int, int, unsigned long long *, unsigned, unsigned,
-                      unsigned, int64_t *, long long, float *) =
+                      unsigned, unsigned, int64_t *, long long, float *) =
 #define NACHO_FUSED(OP, VAL, CHD, ROWS, DOT)             \
     (wide ? fused_kernel<OP, VAL, CHD, ROWS, DOT, true> \
           : fused_kernel<OP, VAL, CHD, ROWS, DOT, false>)
@@ -1254,8 +1276,8 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
         if (!Z.dot) NACHO_TRY(call.length_word(&length_out));
         NACHO_TRY(call.timer_start(kernel_name));
         fused<<<num_tiles, kBlock, 0, s>>>(args, rows, static_cast<int>(total), crd_bits,
-                                           sync.words, sync.epoch, sync.base, sync.done, length_out, items,
-                                           Z.dot);
+                                           sync.words, sync.epoch, sync.base, sync.done,
+                                           sync.polls, length_out, items, Z.dot);
         NACHO_TRY_HIP(hipGetLastError());
         call.sync_launched();
         if (!Z.dot) NACHO_TRY(call.mark_length());

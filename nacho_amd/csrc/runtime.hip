@@ -272,6 +272,8 @@ using SyncKey = std::tuple<int, hipStream_t, std::thread::id>;
 constexpr size_t kMaxSyncBlocks = 64;
 std::map<SyncKey, SyncEntry> g_sync;
 
+thread_local unsigned t_sync_polls = SyncBlock::kMaxPolls;  // nacho_set_wait_limit
+
 __global__ void clear_words_kernel(unsigned long long *words, size_t n) {
     for (size_t i = threadIdx.x; i < n; i += blockDim.x) words[i] = 0ull;
 }
@@ -325,6 +327,7 @@ int take_sync_block(size_t bytes, unsigned tickets, unsigned finishes, hipStream
     out->epoch = ++b.epoch;
     out->base = b.tickets;
     out->done = b.finishes;
+    out->polls = t_sync_polls;
     b.tickets += tickets;
     b.finishes += finishes;
     return NACHO_OK;
@@ -718,6 +721,10 @@ const char *nacho_version(void) { return "nacho-mi355x 0.1 (gfx950)"; }
 
 void nacho_set_kernel_timing(int enable) {
     nacho::g_timing_enabled.store(enable ? 1 : 0, std::memory_order_relaxed);
+}
+
+void nacho_set_wait_limit(unsigned polls) {
+    nacho::t_sync_polls = polls != 0 ? polls : nacho::SyncBlock::kMaxPolls;
 }
 
 float nacho_last_kernel_ms(void) { return nacho::t_last_ms; }

@@ -43,6 +43,8 @@ struct SyncBlock {
     unsigned epoch;
     unsigned base;
     unsigned done;
+    unsigned polls;  // bound of a wait inside the launch
+    static constexpr unsigned kMaxPolls = 1u << 22;  // seconds
     // The stream is being captured, so no block was taken: what a recorded launch does to the
     // counts at each replay is not known here.  A caller that can be recorded brings words of
     // its own, cleared in the same capture (clear_words).

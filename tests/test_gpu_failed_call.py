@@ -141,3 +141,43 @@ def test_call_after_a_failed_allocation(gpu, product):
             assert_dcsr_equal(run_dcsr("mul", (70, 50), da, db, gpu),
                               want_dcsr("mul", da, db), f"after {fail_at}")
     del keep
+
+
+@pytest.mark.parametrize("polls", [1, 2, 20])
+def test_a_tile_that_gives_up(gpu, polls):
+    """One-launch levels whose workgroups look only a few times for the counts before theirs: a
+    call fails or its result is whole, and the calls after it are correct."""
+    import nacho_amd
+    from nacho_amd import _lib
+    from tests.helpers import assert_csr_equal
+    from tests.test_gpu_csr import from_gpu, to_gpu
+
+    rng = np.random.default_rng(polls)
+    rows = cols = 20_000
+    t = []
+    for _ in range(2):
+        keys = np.unique(rng.integers(0, rows * cols, size=8 * rows))
+        pos = np.concatenate([[0], np.cumsum(np.bincount(keys // cols, minlength=rows))])
+        t.append((pos.astype(np.int32), (keys % cols).astype(np.int32),
+                  rng.uniform(-1, 1, len(keys)).astype(np.float32)))
+    want = oracle.closed_csr_binary("add", rows, cols, *t[0], *t[1])
+    a, b = (to_gpu(x, rows, cols, gpu) for x in t)
+    lib = _lib.load()
+    failed = 0
+    try:
+        lib.nacho_set_wait_limit(polls)
+        for call in range(30):
+            print(f"[gpu] at most {polls} polls, call {call}", flush=True)
+            try:
+                z = nacho_amd.gpu_csr_add_f32(a, b)
+            except RuntimeError as e:
+                assert "internal" in str(e)
+                failed += 1
+                continue
+            assert_csr_equal(from_gpu(z), want, f"call {call}")
+    finally:
+        lib.nacho_set_wait_limit(0)
+    if polls == 1:
+        assert failed, "no wait ended early"
+    for call in range(3):
+        assert_csr_equal(from_gpu(nacho_amd.gpu_csr_add_f32(a, b)), want, f"after, call {call}")
