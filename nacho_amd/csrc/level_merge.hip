@@ -1279,8 +1279,11 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
                                            sync.words, sync.epoch, sync.base, sync.done,
                                            sync.polls, length_out, items, Z.dot);
         NACHO_TRY_HIP(hipGetLastError());
-        call.sync_launched();
-        if (!Z.dot) NACHO_TRY(call.mark_length());
+        if (Z.dot) {
+            call.sync_launched();
+        } else {
+            NACHO_TRY(call.mark_length());
+        }
         NACHO_TRY(call.timer_stop());
         if (Z.dot) {
             NACHO_TRY(call.collect_timer());  // (kernel timing only: waits for the stream)

@@ -333,7 +333,7 @@ int take_sync_block(size_t bytes, unsigned tickets, unsigned finishes, hipStream
     return NACHO_OK;
 }
 
-// The call that took the block ends; `sound`: every launch it was taken for was made (the
+// The call that took the block ends; `sound`: every launch it was taken for ran or will (the
 // block's counts are otherwise unknown, so it is dropped).
 void give_sync_block(const SyncKey &key, bool sound) {
     std::lock_guard<std::mutex> lock(g_cache_mutex);
@@ -458,7 +458,7 @@ int Call::sync_block(size_t bytes, unsigned tickets, unsigned finishes, SyncBloc
     const int rc = take_sync_block(bytes, tickets, finishes, stream_, &key, out);
     if (out->words) {
         sync_held_ = true;
-        sync_sound_ = false;  // until the launch is made
+        sync_sound_ = false;  // until the launch is known to count
     }
     return rc;
 }
@@ -616,6 +616,7 @@ int Call::wait_length(int64_t *len) {
     if (!len_marked_) return NACHO_ERR_INTERNAL;
     NACHO_TRY(spin_for_word(t_len_host, stream_, len));
     words_unread_ &= ~1u;
+    sync_sound_ = true;  // (the kernel that stored it ran)
     return collect_timer();
 }
 

@@ -89,8 +89,9 @@ class Call {
     // `tickets` and `finishes`; kept for this stream's later calls.  words stays null where there
     // is none to take (an arena call, a caller's allocator, which the library keeps no memory of,
     // or a stream that is being captured).
-    // sync_launched says that the launch was made: without it the block is dropped when the
-    // call ends.
+    // The block is dropped when the call ends unless its last use is known to have counted: the
+    // launch's length was read (wait_length), or, where the host waits for none, sync_launched
+    // said that the launch was made.
     int sync_block(size_t bytes, unsigned tickets, unsigned finishes, SyncBlock *out);
     void sync_launched() { sync_sound_ = true; }
 

@@ -281,7 +281,7 @@ def test_recorded_in_a_graph(gpu, kind, n):
     """An inner product (whose host waits for nothing) recorded after calls that warmed the
     stream's buffers up, and replayed with other values in its operands: one tile, a few, many,
     and more than one launch takes.  Every replay equals the eager call on the same values, with
-    eager calls and synchronisations between."""
+    eager calls and synchronisations between; small levels on the recording stream stay correct."""
     import nacho_amd
 
     rng = np.random.default_rng(n)
@@ -301,7 +301,13 @@ def test_recorded_in_a_graph(gpu, kind, n):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=stream):
         z = fn(a, b)
+    add = nacho_amd.gpu_csf_add_f32 if kind == "csf" else nacho_amd.gpu_coo3d_add_f32
+    both = add(a, b).values.clone()
+    torch.cuda.synchronize()
     for step in range(6):
+        with torch.cuda.stream(stream):
+            for _ in range(2):
+                assert torch.equal(add(a, b).values, both), step
         a.values.copy_(torch.from_numpy(rng.uniform(-1, 1, len(ac)).astype(np.float32)))
         want = fn(a, b).values.clone()  # (on the default stream)
         torch.cuda.synchronize()
@@ -309,3 +315,5 @@ def test_recorded_in_a_graph(gpu, kind, n):
             graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(z.values, want), (step, z.values.item(), want.item())
+        both = add(a, b).values.clone()
+        torch.cuda.synchronize()
