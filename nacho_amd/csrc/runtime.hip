@@ -7,7 +7,9 @@
 #include <climits>
 #include <cstdint>
 #include <cstring>
+#include <iterator>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <tuple>
@@ -256,10 +258,17 @@ int record_stream(void *ptr, hipStream_t stream) {
 }
 
 // ---- sync blocks -----------------------------------------------------------------------
-// One block per (device, stream, host thread): a thread's launches on one stream run in the
-// order it made them, which is the order of the epochs and tickets it took.  A block in use by
-// a call is not freed; the others (a few KB each) go back to the driver with the cache
-// (nacho_release_cached_memory) and when they outnumber kMaxSyncBlocks.
+// Blocks by (device, stream): a call takes an idle one of its stream's, keeps it to itself until
+// it ends, and the next call that takes it queues its launches on the same stream after those, so
+// launches run in the order of the epochs and tickets they were given.  A stream has as many
+// blocks as calls were made on it at once, however many threads make them.  The handle
+// hipStreamPerThread names another stream in each thread, so there the thread belongs to the key.
+//
+// Idle blocks (a few KB each) go back to the driver with the cache (nacho_release_cached_memory)
+// and when there are kMaxSyncBlocks: their launches may still run, so that waits for the device,
+// once for every kMaxSyncBlocks blocks that were new.
+}  // namespace
+
 struct SyncEntry {
     unsigned long long *words;
     size_t bytes;
@@ -268,9 +277,13 @@ struct SyncEntry {
     unsigned finishes;
     bool busy;
 };
+
+namespace {
+
 using SyncKey = std::tuple<int, hipStream_t, std::thread::id>;
-constexpr size_t kMaxSyncBlocks = 64;
-std::map<SyncKey, SyncEntry> g_sync;
+constexpr size_t kMaxSyncBlocks = 1024;
+std::map<SyncKey, std::vector<std::unique_ptr<SyncEntry>>> g_sync;
+size_t g_sync_blocks = 0;  // in g_sync
 
 thread_local unsigned t_sync_polls = SyncBlock::kMaxPolls;  // nacho_set_wait_limit
 
@@ -278,72 +291,76 @@ __global__ void clear_words_kernel(unsigned long long *words, size_t n) {
     for (size_t i = threadIdx.x; i < n; i += blockDim.x) words[i] = 0ull;
 }
 
-// Frees every block that no call holds (their launches may still run: the device is
-// synchronised first).  Caller holds g_cache_mutex.
+// Frees every block that no call holds.  Caller holds g_cache_mutex.
 void free_sync_blocks_locked() {
     (void)hipDeviceSynchronize();
     for (auto it = g_sync.begin(); it != g_sync.end();) {
-        if (it->second.busy) {
-            ++it;
-        } else {
-            (void)hipFree(it->second.words);
-            it = g_sync.erase(it);
+        auto &blocks = it->second;
+        for (size_t i = blocks.size(); i-- > 0;) {
+            if (blocks[i]->busy) continue;
+            (void)hipFree(blocks[i]->words);
+            blocks.erase(blocks.begin() + static_cast<std::ptrdiff_t>(i));
+            --g_sync_blocks;
         }
+        it = blocks.empty() ? g_sync.erase(it) : std::next(it);
     }
 }
 
-// A use of the caller's block, which stays busy until give_sync_block.
-int take_sync_block(size_t bytes, unsigned tickets, unsigned finishes, hipStream_t stream,
-                    SyncKey *key, SyncBlock *out) {
+// An idle block of the stream's, or a new one, busy until give_sync_block; null where the driver
+// has no memory for one.
+int take_sync_block(size_t bytes, hipStream_t stream, SyncEntry **out) {
+    *out = nullptr;
     int device = 0;
     NACHO_TRY_HIP(hipGetDevice(&device));
-    *key = SyncKey{device, stream, std::this_thread::get_id()};
+    const SyncKey key{device, stream,
+                      stream == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id{}};
     std::lock_guard<std::mutex> lock(g_cache_mutex);
-    auto it = g_sync.find(*key);
-    if (it != g_sync.end() && (it->second.bytes < bytes || it->second.epoch == UINT_MAX)) {
-        (void)hipDeviceSynchronize();
-        (void)hipFree(it->second.words);
-        g_sync.erase(it);
-        it = g_sync.end();
-    }
-    if (it == g_sync.end()) {
-        if (g_sync.size() >= kMaxSyncBlocks) free_sync_blocks_locked();
-        void *p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return NACHO_OK;  // none to take
+    if (auto it = g_sync.find(key); it != g_sync.end()) {
+        for (auto &b : it->second) {
+            // (a call makes a handful of launches: the epoch does not run out in one)
+            if (!b->busy && b->bytes >= bytes && b->epoch < UINT_MAX / 2) {
+                b->busy = true;
+                *out = b.get();
+                return NACHO_OK;
+            }
         }
-        unsigned long long *words = static_cast<unsigned long long *>(p);
-        const int rc = clear_words(stream, words, bytes / sizeof(unsigned long long));
-        if (rc != NACHO_OK) {
-            (void)hipFree(p);
-            return rc;
-        }
-        it = g_sync.insert({*key, SyncEntry{words, bytes, 0u, 0u, 0u, false}}).first;
     }
-    SyncEntry &b = it->second;
-    b.busy = true;
-    out->words = b.words;
-    out->epoch = ++b.epoch;
-    out->base = b.tickets;
-    out->done = b.finishes;
-    out->polls = t_sync_polls;
-    b.tickets += tickets;
-    b.finishes += finishes;
+    if (g_sync_blocks >= kMaxSyncBlocks) free_sync_blocks_locked();
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return NACHO_OK;
+    }
+    unsigned long long *words = static_cast<unsigned long long *>(p);
+    const int rc = clear_words(stream, words, bytes / sizeof(unsigned long long));
+    if (rc != NACHO_OK) {
+        (void)hipFree(p);
+        return rc;
+    }
+    auto &blocks = g_sync[key];
+    blocks.push_back(std::make_unique<SyncEntry>(SyncEntry{words, bytes, 0u, 0u, 0u, true}));
+    ++g_sync_blocks;
+    *out = blocks.back().get();
     return NACHO_OK;
 }
 
 // The call that took the block ends; `sound`: every launch it was taken for ran or will (the
 // block's counts are otherwise unknown, so it is dropped).
-void give_sync_block(const SyncKey &key, bool sound) {
+void give_sync_block(SyncEntry *entry, bool sound) {
     std::lock_guard<std::mutex> lock(g_cache_mutex);
-    auto it = g_sync.find(key);
-    if (it == g_sync.end()) return;
-    it->second.busy = false;
-    if (!sound) {
-        (void)hipDeviceSynchronize();
-        (void)hipFree(it->second.words);
-        g_sync.erase(it);
+    entry->busy = false;
+    if (sound) return;
+    (void)hipDeviceSynchronize();
+    for (auto it = g_sync.begin(); it != g_sync.end(); ++it) {
+        auto &blocks = it->second;
+        for (size_t i = 0; i < blocks.size(); ++i) {
+            if (blocks[i].get() != entry) continue;
+            (void)hipFree(entry->words);
+            blocks.erase(blocks.begin() + static_cast<std::ptrdiff_t>(i));
+            --g_sync_blocks;
+            if (blocks.empty()) g_sync.erase(it);
+            return;
+        }
     }
 }
 
@@ -386,11 +403,7 @@ Call::Call(void *stream, void *arena, size_t arena_bytes)
 Call::~Call() {
     if (arena_) return;  // nothing was allocated
     if (words_unread_ != 0) (void)hipStreamSynchronize(stream_);  // a queued store may be late
-    if (sync_held_) {
-        int device = 0;
-        (void)hipGetDevice(&device);
-        give_sync_block(SyncKey{device, stream_, std::this_thread::get_id()}, sync_sound_);
-    }
+    if (sync_) give_sync_block(sync_, sync_sound_);
     if (timed_) t_last_ms = timed_ms_;
     if (!committed_) scratch_.insert(scratch_.end(), results_.begin(), results_.end());
     if (alloc_) {
@@ -454,13 +467,18 @@ int Call::sync_block(size_t bytes, unsigned tickets, unsigned finishes, SyncBloc
         out->recorded = true;
         return NACHO_OK;
     }
-    SyncKey key;
-    const int rc = take_sync_block(bytes, tickets, finishes, stream_, &key, out);
-    if (out->words) {
-        sync_held_ = true;
-        sync_sound_ = false;  // until the launch is known to count
-    }
-    return rc;
+    if (!sync_) NACHO_TRY(take_sync_block(bytes, stream_, &sync_));
+    if (!sync_ || sync_->bytes < bytes) return NACHO_OK;
+    sync_sound_ = false;  // until the launch is known to count
+    // (the block is this call's alone while it is busy)
+    out->words = sync_->words;
+    out->epoch = ++sync_->epoch;
+    out->base = sync_->tickets;
+    out->done = sync_->finishes;
+    out->polls = t_sync_polls;
+    sync_->tickets += tickets;
+    sync_->finishes += finishes;
+    return NACHO_OK;
 }
 
 void Call::drop_result(void *ptr) {

@@ -51,6 +51,8 @@ struct SyncBlock {
     bool recorded;
 };
 
+struct SyncEntry;  // a kept block (runtime.hip)
+
 // Zeroes n words by a small kernel on the stream (which, unlike a memset, may be recorded).
 int clear_words(hipStream_t stream, unsigned long long *words, size_t n);
 
@@ -159,7 +161,8 @@ class Call {
     int64_t *arena_len_ = nullptr;
     int64_t *arena_side_ = nullptr;
     bool timed_ = false;
-    bool sync_held_ = false, sync_sound_ = true;
+    SyncEntry *sync_ = nullptr;  // the block this call took, and whether its counts are known
+    bool sync_sound_ = true;
     unsigned words_unread_ = 0;  // pinned words handed out and not read: bit per word
     bool len_marked_ = false;  // mark_length: this call launched the kernel storing its length
     float timed_ms_ = 0.0f;  // sum of this call's bracketed intervals

@@ -174,3 +174,65 @@ def test_one_launch_threads_and_streams(gpu):
     for th in threads:
         th.join()
     assert not failures, failures[0]
+
+
+def test_one_launch_many_threads(gpu):
+    """100 live threads, one call each on one stream: none of them waits for the device (a side
+    stream is still busy at the end)."""
+    import threading
+
+    import nacho_amd
+
+    rng = np.random.default_rng(5)
+    rows, cols = 2000, 3000
+    t = [csr_from_rows(rows, cols, [np.unique(rng.integers(0, cols, 8)) for _ in range(rows)])
+         for _ in range(2)]
+    shape = torch.tensor([rows, cols], dtype=torch.int32)
+    ops = [nacho_amd.CSR_gpu(*(torch.from_numpy(x).to(gpu) for x in o), shape) for o in t]
+    want = oracle.closed_csr_binary("add", rows, cols, *t[0], *t[1])
+    main, side = torch.cuda.Stream(), torch.cuda.Stream()
+    begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(1_000_000)
+        begin.record()
+        torch.cuda._sleep(1_000_000)
+        end.record()
+    with torch.cuda.stream(main):
+        for _ in range(3):  # (warms the buffers up)
+            nacho_amd.gpu_csr_add_f32(*ops)
+    torch.cuda.synchronize()
+    cycles = int(1_000_000 * 2000 / begin.elapsed_time(end))  # about two seconds
+    gates = [threading.Event() for _ in range(101)]
+    hold, failures = threading.Event(), []
+
+    def work(i):
+        gates[i].wait()
+        try:
+            with torch.cuda.stream(main):
+                nacho_amd.gpu_csr_add_f32(*ops)
+        except BaseException as e:  # noqa: BLE001
+            failures.append(e)
+        gates[i + 1].set()
+        hold.wait()  # (a thread that ended would give its id to the next)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(100)]
+    for th in threads:
+        th.start()
+    busy = torch.cuda.Event()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(cycles)
+        busy.record()
+    gates[0].set()
+    gates[100].wait()
+    waited = busy.query()
+    hold.set()
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    assert not failures, failures[0]
+    assert not waited, "a call waited for the device"
+    with torch.cuda.stream(main):
+        z = nacho_amd.gpu_csr_add_f32(*ops)
+    torch.cuda.synchronize()
+    assert_csr_equal(tuple(x.cpu().numpy() for x in (z.dim_j_offsets, z.dim_j_indices, z.values)),
+                     want, "after")
