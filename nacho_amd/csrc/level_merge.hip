@@ -1211,6 +1211,11 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
     if (values ? child : !child || intersect) return NACHO_ERR_INVALID_ARGUMENT;
     if (Z.crd_low && (!Z.row || intersect)) return NACHO_ERR_INVALID_ARGUMENT;
     if (Z.dot && !intersect) return NACHO_ERR_INVALID_ARGUMENT;
+    if (!intersect) {  // unions take int32 arrays at multiples of 4 bytes only
+        for (const int *p : {A.pos, A.crd, B.pos, B.crd}) {
+            if (reinterpret_cast<uintptr_t>(p) & 3u) return NACHO_ERR_INVALID_ARGUMENT;
+        }
+    }
     const int num_tiles = total > 0 ? static_cast<int>((total + kTile - 1) / kTile) : 1;
 
     void (*emit)(EmitArgs) =

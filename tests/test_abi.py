@@ -288,6 +288,26 @@ def test_allocator_failure_releases_everything(lib, entry, fail_at):
     assert z.nnz == 0 and z.dim_j_length == 0
 
 
+@pytest.mark.parametrize("field", ["dim_j_offsets", "dim_j_indices"])
+@pytest.mark.parametrize("operand", [0, 1])
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_union_refuses_misaligned_arrays(lib, field, operand, shift):
+    """csr_add refuses offsets or coordinates that are not 4-byte aligned, before any HIP call,
+    and releases what it had allocated."""
+    from nacho_amd import _lib
+
+    alloc = _CountingAllocator(100)
+    ops = [_lib.CsrDesc(8, 8, ctypes.c_void_p(0x1000), 5, ctypes.c_void_p(0x2000),
+                        ctypes.c_void_p(0x3000), 5) for _ in range(2)]
+    setattr(ops[operand], field, getattr(ops[operand], field) + shift)
+    z = _lib.CsrDesc()
+    rc = lib.nacho_gpu_csr_add_f32(*(ctypes.byref(t) for t in ops), ctypes.byref(z), 256, 256,
+                                   None, ctypes.byref(alloc.struct))
+    assert rc == -1, _lib.error_string(rc)
+    assert sorted(alloc.handed) == sorted(alloc.released)
+    assert z.dim_j_offsets is None and z.nnz == 0
+
+
 def test_validate_csr_rejects_host_visible_faults(lib):
     """nacho_validate_csr refuses null pointers, negative sizes and nnz != dim_j_length
     before touching the device."""
