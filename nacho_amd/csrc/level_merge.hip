@@ -299,8 +299,13 @@ __global__ __launch_bounds__(kBlock) void split_sparse_kernel(
 // does the same 12 minima and maxima per key, all independent within a stage, where a merge
 // walk is a serial chain of LDS reads per lane with its wavefront's lanes on both branches.
 //
-// Keys are 32-bit where row, coordinate and side fit (decided per tile), else binary64
-// numbers whose order is that of the key.
+// Keys are 32-bit where row, coordinate and side fit (decided per tile, for coordinates of the
+// declared extent), else binary64 numbers whose order is that of the key.  A tile with a
+// coordinate that its keys do not hold (past the extent, or negative) is walked afterwards
+// instead (walk_tile), so coordinates are ordered as the int32 numbers they are.  (Key widths
+// chosen by each tile's largest coordinate made the keys wait for one more reduction: 1 to 2%
+// per call; one kernel for both widths took 47 us more at C5's k level, where the 32-bit one's
+// 7 wavefronts per SIMD are worth it.)
 //
 // Bound by LDS and VALU issue together (about 60% and 55% busy at C3: 560 VALU and 73 LDS
 // instructions per lane and tile): 61 us for C3's 33M entries, 96 us for the 40M of the C5 k
@@ -526,6 +531,59 @@ __device__ __forceinline__ unsigned load_at(const int *base, int bytes) {
                                                static_cast<unsigned>(bytes));
 }
 
+// The merge order of a tile whose keys do not hold its coordinates, as order_tile gives it: a lane
+// finds its first slot by searches in the operands and takes 16 entries one by one (ties: A
+// first).  Unsorted rows keep the searches and the walk inside the tile's ranges as well.
+__device__ __forceinline__ void walk_tile(const TileSplit &sp, const int *__restrict__ pa,
+                                          const int *__restrict__ ca, const int *__restrict__ pb,
+                                          const int *__restrict__ cb, int tid, unsigned &side,
+                                          unsigned &dup) {
+    const int na = sp.a1 - sp.a0, nb = sp.b1 - sp.b0, nr = sp.r1 - sp.r0 + 1;
+    const int first = kPer * tid, count = min(max(na + nb - first, 0), kPer);
+    side = dup = 0;
+    if (count == 0) return;
+    auto begin_a = [&](int k) { return k == 0 ? 0 : k >= nr ? na : min(max(pa[sp.r0 + k] - sp.a0, 0), na); };
+    auto begin_b = [&](int k) { return k == 0 ? 0 : k >= nr ? nb : min(max(pb[sp.r0 + k] - sp.b0, 0), nb); };
+    int k = 0;  // the last row that begins at or before the slot
+    for (int hi = nr - 1; k < hi;) {
+        const int mid = (k + hi + 1) >> 1;
+        if (begin_a(mid) + begin_b(mid) <= first) {
+            k = mid;
+        } else {
+            hi = mid - 1;
+        }
+    }
+    int a = begin_a(k), b = begin_b(k), ae = begin_a(k + 1), be = begin_b(k + 1);
+    const int d = first - a - b;
+    int lo = max(0, d - (be - b)), hi = min(d, ae - a);  // A entries among the row's first d
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (ca[sp.a0 + a + mid] <= cb[sp.b0 + b + d - 1 - mid]) {
+            lo = mid + 1;
+        } else {
+            hi = mid;
+        }
+    }
+    int as = a;  // the row's first A entry
+    a += lo;
+    b += d - lo;
+    for (int i = 0; i < count; ++i) {
+        while (a >= ae && b >= be && k + 1 < nr) {
+            ++k;
+            as = a;
+            ae = begin_a(k + 1);
+            be = begin_b(k + 1);
+        }
+        if (a < ae && (b >= be || ca[sp.a0 + a] <= cb[sp.b0 + b])) {
+            ++a;
+        } else if (b < be) {
+            side |= 1u << i;
+            dup |= a > as && ca[sp.a0 + a - 1] == cb[sp.b0 + b] ? 1u << i : 0u;
+            ++b;
+        }
+    }
+}
+
 // The merge order of the tile `sp`: lane tid's 16 slots as bit masks `side` and `dup`, and the
 // tile's pairs, the same in every lane.  `some`: any readable word.  Ends without a barrier.
 template <bool WIDE>
@@ -541,15 +599,16 @@ __device__ __forceinline__ unsigned order_tile(OrderLds &sh, const TileSplit &sp
 
     // Slot tid + 256 j is A's entry of that index, or B's entry kSlots - 1 - slot.  The
     // padding is at least a wavefront wide, so a wavefront's 64 slots hold entries of one
-    // side only: a scalar base and one clamped lane offset.  What padding slots load (some
-    // valid word) is never used.
+    // side only: a scalar base and one clamped lane offset.  Padding slots load a coordinate of
+    // the tile, so that every coordinate loaded counts for whether the keys hold it.
+    const int *pad = na > 0 ? ca + sp.a0 : nb > 0 ? cb + sp.b0 : some;
     unsigned x[kPer];
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
         const int first = kBlock * j + dev::kWave * w;  // the wavefront's slots
         const int base = kSlots - kBlock * (j + 1);     // B's entry of tid == kBlock - 1
         const bool in_a = first < na, in_b = first + dev::kWave > kSlots - nb;
-        const int *from = in_a ? ca + sp.a0 + kBlock * j : in_b ? cb + sp.b0 + base  : some;
+        const int *from = in_a ? ca + sp.a0 + kBlock * j : in_b ? cb + sp.b0 + base : pad;
         const int last = in_a ? na - 1 - kBlock * j : in_b ? nb - 1 - base : 0;
         x[j] = load_at(from, min(in_a ? 4 * tid : 4 * (kBlock - 1 - tid), 4 * last));
     }
@@ -614,35 +673,54 @@ __device__ __forceinline__ unsigned order_tile(OrderLds &sh, const TileSplit &sp
     // (bits of nr, not of nr - 1: the padding's row, all ones, is no row of the tile)
     const int row_bits = 32 - __builtin_clz(static_cast<unsigned>(nr));
     const bool wide = WIDE && row_bits + bits + 1 > 32;
+    unsigned crds = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) crds |= x[j];
+    const bool past = __any(crds >> (wide ? 31 : bits));  // of no key's coordinate
     if (wide) {  // uniform
         sort_tile<WideKey>(sh, x, mark, na + nb, bits, tid, side, dup);
     } else {
         sort_tile<NarrowKey>(sh, x, mark, na + nb, bits, tid, side, dup);
     }
-    const int found = dev::wave_inclusive_sum_dpp(__popc(dup));
-    const int in_b = dev::wave_inclusive_sum_dpp(__popc(side));
-    if (l == dev::kWave - 1) {
-        sh.pairs[w] = static_cast<unsigned>(found);
-        sh.sides[w] = static_cast<unsigned>(in_b);
-    }
-    __syncthreads();
+    // The tile's pairs and B slots per wavefront (flag: bit 31 of the pairs).
+    auto count = [&](bool flag) {
+        const int found = dev::wave_inclusive_sum_dpp(__popc(dup));
+        const int in_b = dev::wave_inclusive_sum_dpp(__popc(side));
+        if (l == dev::kWave - 1) {
+            sh.pairs[w] = static_cast<unsigned>(found) | (flag ? 1u << 31 : 0u);
+            sh.sides[w] = static_cast<unsigned>(in_b);
+        }
+        __syncthreads();
+    };
+    count(past);
     // pairs across two wavefronts: the last slot of i - 1 and the first of i
     auto across = [&](int i) {
         return kPer * dev::kWave * i < na + nb &&
                (sh.first[2 * i] ^ sh.last[2 * i - 2]) == 1u && (sh.first[2 * i] & 1u) == 1u &&
                (!wide || sh.first[2 * i + 1] == sh.last[2 * i - 1]);
     };
-    unsigned pairs = sh.pairs[0], sides = sh.sides[0];
+    unsigned pairs = sh.pairs[0], sides = sh.sides[0], flags = pairs;
 #pragma unroll
     for (int i = 1; i < kWaves; ++i) {
         const bool p = across(i);
+        flags |= sh.pairs[i];
         pairs += sh.pairs[i] + static_cast<unsigned>(p);
         sides += sh.sides[i];
         if (p && tid == dev::kWave * i) dup |= 1u;
     }
+    if (flags >> 31) {  // uniform
+        __syncthreads();  // (the counts are read)
+        walk_tile(sp, pa, ca, pb, cb, tid, side, dup);
+        count(false);
+        pairs = sides = 0;
+        for (int i = 0; i < kWaves; ++i) {
+            pairs += sh.pairs[i];
+            sides += sh.sides[i];
+        }
+    }
     if (sides != static_cast<unsigned>(nb)) {  // uniform
-        // Only operands that break the contract (a coordinate beyond its extent sorts past
-        // the padding): any order with nb B slots keeps the emit kernel inside them.
+        // Only operands that break the contract (unsorted rows): any order with nb B slots
+        // keeps the emit kernel inside them.
         const int b_from = min(max(na - kPer * tid, 0), kPer);
         const int b_to = min(max(na + nb - kPer * tid, 0), kPer);
         side = ((1u << b_to) - 1u) & ~((1u << b_from) - 1u);
@@ -655,8 +733,8 @@ __device__ __forceinline__ unsigned order_tile(OrderLds &sh, const TileSplit &sp
 // One tile per workgroup.  side / dup: kBlock 16-bit masks per tile; tile_pairs[t] gets the
 // tile's pairs, which are also added into chunk_pairs[t / kChunk] (zeroed by the partition
 // kernel).  The last workgroup stores the result length: the pairs (intersection), or
-// `items` (the operands' entries) less the pairs.  WIDE: the level's coordinates may need
-// 64-bit keys.  SPARSE: split_sparse_kernel ran; state[t] holds the pairs of a tile that it
+// `items` (the operands' entries) less the pairs.  WIDE: the level's extent may need 64-bit
+// keys.  SPARSE: split_sparse_kernel ran; state[t] holds the pairs of a tile that it
 // wrote, or kDense.
 template <bool WIDE, bool SPARSE>
 __global__ __launch_bounds__(kBlock, WIDE ? 4 : 6) void order_kernel(

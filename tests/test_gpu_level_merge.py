@@ -236,3 +236,52 @@ def test_one_launch_many_threads(gpu):
     torch.cuda.synchronize()
     assert_csr_equal(tuple(x.cpu().numpy() for x in (z.dim_j_offsets, z.dim_j_indices, z.values)),
                      want, "after")
+
+
+@pytest.mark.parametrize("lo,hi", [(0, 40), (0, 70_000), (0, 2**31), (-50, 50), (-(2**31), 2**31)])
+@pytest.mark.parametrize("rows,mean", [(1, 3000), (40, 400), (3000, 5), (70_000, 12)])
+@pytest.mark.parametrize("op", ["add", "mul"])
+def test_coordinates_past_the_extent(gpu, op, rows, mean, lo, hi):
+    """Coordinates are ordered as the int32 numbers they are, whatever extent is declared (8)."""
+    import nacho_amd
+
+    rng = np.random.default_rng(rows + mean)
+    n = min(mean, (hi - lo) // 2)
+    keys = []
+    pool = np.unique(rng.integers(lo, hi, size=4 * n))  # (coordinates that both operands draw)
+    for _ in range(2):
+        r = np.repeat(np.arange(rows, dtype=np.int64), n)
+        keys.append(np.unique(r * 2**33 + pool[rng.integers(0, len(pool), size=len(r))] + 2**32))
+    vals = [rng.uniform(-1, 1, len(k)).astype(np.float32) for k in keys]
+
+    def csr(k):
+        pos = np.zeros(rows + 1, np.int32)
+        pos[1:] = np.cumsum(np.bincount(k >> 33, minlength=rows))
+        return pos, ((k & (2**33 - 1)) - 2**32).astype(np.int32)
+
+    both, ia, ib = np.intersect1d(*keys, assume_unique=True, return_indices=True)
+    if op == "mul":
+        want_keys, want = both, vals[0][ia] * vals[1][ib]
+    else:
+        want_keys = np.union1d(*keys)
+        at = [np.searchsorted(want_keys, k) for k in keys]
+        want = np.zeros(len(want_keys), np.float32)
+        want[at[1]] = vals[1]
+        want[at[0]] = vals[0]
+        want[at[0][ia]] = vals[0][ia] + vals[1][ib]
+    print(f"[gpu] level merge {op} rows={rows} n={n} coordinates in [{lo}, {hi})", flush=True)
+    shape = torch.tensor([rows, 8], dtype=torch.int32)
+
+    def dev(x):
+        return torch.from_numpy(np.ascontiguousarray(x)).to(gpu)
+
+    z = getattr(nacho_amd, f"gpu_csr_{op}_f32")(
+        *(nacho_amd.CSR_gpu(*(dev(x) for x in csr(k)), dev(v), shape) for k, v in zip(keys, vals)))
+    got = tuple(x.cpu().numpy() for x in (z.dim_j_offsets, z.dim_j_indices, z.values))
+    assert_csr_equal(got, (*csr(want_keys), want), op)
+    z = getattr(nacho_amd, f"gpu_coo_{op}_f32")(
+        *(nacho_amd.COO_gpu(dev((k >> 33).astype(np.int32)), dev(csr(k)[1]), dev(v), shape)
+          for k, v in zip(keys, vals)))
+    assert np.array_equal(z.dim_i_indices.cpu().numpy(), (want_keys >> 33).astype(np.int32))
+    assert np.array_equal(z.dim_j_indices.cpu().numpy(), csr(want_keys)[1])
+    assert np.array_equal(z.values.cpu().numpy().view(np.uint32), want.view(np.uint32))
