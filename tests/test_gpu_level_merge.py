@@ -190,18 +190,35 @@ def test_one_launch_many_threads(gpu):
     shape = torch.tensor([rows, cols], dtype=torch.int32)
     ops = [nacho_amd.CSR_gpu(*(torch.from_numpy(x).to(gpu) for x in o), shape) for o in t]
     want = oracle.closed_csr_binary("add", rows, cols, *t[0], *t[1])
-    main, side = torch.cuda.Stream(), torch.cuda.Stream()
-    begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-    with torch.cuda.stream(side):
+    main = torch.cuda.Stream()
+    begin, end, busy = (torch.cuda.Event(enable_timing=True) for _ in range(3))
+    with torch.cuda.stream(main):
+        for _ in range(3):  # (warms the buffers up)
+            nacho_amd.gpu_csr_add_f32(*ops)
         torch.cuda._sleep(1_000_000)
         begin.record()
         torch.cuda._sleep(1_000_000)
         end.record()
-    with torch.cuda.stream(main):
-        for _ in range(3):  # (warms the buffers up)
-            nacho_amd.gpu_csr_add_f32(*ops)
     torch.cuda.synchronize()
-    cycles = int(1_000_000 * 2000 / begin.elapsed_time(end))  # about two seconds
+    cycles = int(1_000_000 * 300 / begin.elapsed_time(end))  # about 0.3 seconds
+
+    def sleep_on(side):
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(cycles)
+            busy.record()
+
+    # Streams share the few hardware queues of a process: a side stream on another one than main.
+    for _ in range(8):
+        side = torch.cuda.Stream()
+        sleep_on(side)
+        with torch.cuda.stream(main):
+            nacho_amd.gpu_csr_add_f32(*ops)
+        if not busy.query():
+            break
+        torch.cuda.synchronize()
+    else:
+        pytest.fail("no stream runs beside the first one")
+    torch.cuda.synchronize()
     gates = [threading.Event() for _ in range(101)]
     hold, failures = threading.Event(), []
 
@@ -218,10 +235,7 @@ def test_one_launch_many_threads(gpu):
     threads = [threading.Thread(target=work, args=(i,)) for i in range(100)]
     for th in threads:
         th.start()
-    busy = torch.cuda.Event()
-    with torch.cuda.stream(side):
-        torch.cuda._sleep(cycles)
-        busy.record()
+    sleep_on(side)
     gates[0].set()
     gates[100].wait()
     waited = busy.query()
