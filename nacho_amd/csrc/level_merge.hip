@@ -285,8 +285,15 @@ __global__ __launch_bounds__(kBlock) void split_sparse_kernel(
     if (bits_below(odd) & 1) bits = ~bits;  // (the toggles are even in number: 0 past the end)
     side_out[static_cast<size_t>(t) * kWords + l] = bits;
     dup_out[static_cast<size_t>(t) * kWords + l] = dup;
-    const int pairs = dev::wave_inclusive_sum_dpp(__popcll(dup));
-    if (l == dev::kWave - 1) tile_pairs[t] = state[t] = static_cast<unsigned>(pairs);
+    // Two searches of an unsorted row may land on one slot and their toggles cancel; a tile whose
+    // B slots are not nb, or whose pairs end on another slot, is left to the order kernel.
+    const bool stray = __any((dup & ~bits) != 0);
+    const unsigned sums = static_cast<unsigned>(dev::wave_inclusive_sum_dpp(
+        __popcll(bits) << 16 | __popcll(dup)));  // (at most kSlots each)
+    if (l == dev::kWave - 1) {
+        const bool whole = !stray && sums >> 16 == static_cast<unsigned>(nb);
+        tile_pairs[t] = state[t] = whole ? sums & 0xffffu : kDense;
+    }
 }
 
 // ---- order kernel ----------------------------------------------------------------------
@@ -315,8 +322,9 @@ __global__ __launch_bounds__(kBlock) void split_sparse_kernel(
 // entry), and a running maximum over the slots gives every entry its row and side: a mark is
 // the tile row k for A, ~k for B, and kPadMark for the padding between them.
 //
-// Whatever the operands hold (unsorted or out-of-range coordinates), a tile's order has
-// exactly nb B slots among its n, so the emit kernel's indices stay inside the operands.
+// Whatever coordinates a tile's rows hold, its order (here and in split_sparse_kernel) has
+// exactly nb B slots among its n, so the emit kernel's indices stay inside the tile's ranges of
+// the operands.  (The ranges themselves come from searches that take rows for sorted.)
 
 // LDS word of slot p's key: the wavefront's lanes fall on distinct banks in all three layouts,
 // and a lane's 16 consecutive slots stay 16-byte aligned.

@@ -299,3 +299,37 @@ def test_coordinates_past_the_extent(gpu, op, rows, mean, lo, hi):
     assert np.array_equal(z.dim_i_indices.cpu().numpy(), (want_keys >> 33).astype(np.int32))
     assert np.array_equal(z.dim_j_indices.cpu().numpy(), csr(want_keys)[1])
     assert np.array_equal(z.values.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("na,nb", [(2, 7), (7, 2), (4, 5), (9, 9)])
+def test_short_unsorted_rows(gpu, na, nb):
+    """Rows whose coordinates are in no order break the contract, but every entry still comes out
+    once, in its row (more tiles than one launch takes, few searches in each)."""
+    import nacho_amd
+
+    rng = np.random.default_rng(10 * na + nb)
+    rows = 160_000
+    ca = rng.permuted(np.tile(np.arange(12), (rows, 1)), axis=1)[:, :na] * 2
+    cb = rng.permuted(np.tile(np.arange(12), (rows, 1)), axis=1)[:, :nb] * 2 + 1
+    # most rows belong to one operand, so that tiles hold few searches
+    la = np.where(np.arange(rows) % 16 == 0, na, np.where(np.arange(rows) % 2 == 0, na, 0))
+    lb = np.where(np.arange(rows) % 16 == 0, nb, np.where(np.arange(rows) % 2 == 1, nb, 0))
+    ops, want = [], []
+    for c, n in ((ca, la), (cb, lb)):
+        pos = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+        keep = np.arange(c.shape[1])[None, :] < n[:, None]
+        crd = c[keep].astype(np.int32)
+        val = rng.uniform(-1, 1, len(crd)).astype(np.float32)
+        ops.append((pos, crd, val))
+        want.append((np.repeat(np.arange(rows), n), crd, val))
+    shape = torch.tensor([rows, 24], dtype=torch.int32)
+    print(f"[gpu] unsorted rows of {na} and {nb}", flush=True)
+    z = nacho_amd.gpu_csr_add_f32(
+        *(nacho_amd.CSR_gpu(*(torch.from_numpy(x).to(gpu) for x in o), shape) for o in ops))
+    pos, crd, val = (x.cpu().numpy() for x in (z.dim_j_offsets, z.dim_j_indices, z.values))
+    assert np.array_equal(pos, ops[0][0] + ops[1][0])
+    row = np.repeat(np.arange(rows), np.diff(pos))
+    w = [np.concatenate([x[i] for x in want]) for i in range(3)]
+    got, exp = np.lexsort((crd, row)), np.lexsort((w[1], w[0]))
+    assert np.array_equal(row[got], w[0][exp]) and np.array_equal(crd[got], w[1][exp])
+    assert np.array_equal(val[got], w[2][exp])
