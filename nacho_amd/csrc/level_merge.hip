@@ -740,8 +740,8 @@ __device__ __forceinline__ unsigned order_tile(OrderLds &sh, const TileSplit &sp
 
 // One tile per workgroup.  side / dup: kBlock 16-bit masks per tile; tile_pairs[t] gets the
 // tile's pairs, which are also added into chunk_pairs[t / kChunk] (zeroed by the partition
-// kernel).  The last workgroup stores the result length: the pairs (intersection), or
-// `items` (the operands' entries) less the pairs.  WIDE: the level's extent may need 64-bit
+// kernel).  The last workgroup stores the result length: the pairs (intersection), or the
+// entries that the operands' offsets span less the pairs.  WIDE: the level's extent may need 64-bit
 // keys.  SPARSE: split_sparse_kernel ran; state[t] holds the pairs of a tile that it
 // wrote, or kDense.
 template <bool WIDE, bool SPARSE>
@@ -752,13 +752,15 @@ __global__ __launch_bounds__(kBlock, WIDE ? 4 : 6) void order_kernel(
     unsigned short *__restrict__ dup_out, const unsigned *__restrict__ state,
     unsigned *__restrict__ tile_pairs, unsigned *__restrict__ chunk_pairs,
     unsigned long long *__restrict__ done,
-    int64_t *__restrict__ length_out, int intersect, long long items) {
+    int64_t *__restrict__ length_out, int intersect) {
     __shared__ __align__(16) OrderLds sh;
     const int tid = threadIdx.x;
     const int l = tid % dev::kWave;
     const int w = __builtin_amdgcn_readfirstlane(tid / dev::kWave);
     const int t = blockIdx.x;
     const int c = t / kChunk;
+    // (of the offsets: an operand's arrays may be longer)
+    const int64_t items = static_cast<int64_t>(split_a[gridDim.x]) + split_b[gridDim.x];
     // The tile's pairs, or those of a chunk's written tiles, `tickets` of the chunk's (one
     // thread).
     auto total = [&](unsigned pairs, int tickets) {
@@ -1111,7 +1113,7 @@ __global__ __launch_bounds__(kBlock) void fused_kernel(EmitArgs g, int rows, int
                                                        unsigned epoch, unsigned base,
                                                        unsigned done_base, unsigned max_polls,
                                                        int64_t *__restrict__ length_out,
-                                                       long long items, float *__restrict__ dot) {
+                                                       float *__restrict__ dot) {
     __shared__ double s_dot[DOT ? kBlock : 1];
     __shared__ __align__(16) OrderLds sh;
     __shared__ __align__(8) unsigned short s_side[kBlock], s_dup[kBlock];
@@ -1229,7 +1231,8 @@ __global__ __launch_bounds__(kBlock) void fused_kernel(EmitArgs g, int rows, int
     if (__syncthreads_or(!found)) return;
     if (tid == 0 && t == g.num_tiles - 1) {
         const int64_t all = static_cast<int64_t>(pairs) + own;
-        dev::store_system(length_out, OP == Op::Union ? items - all : all);
+        dev::store_system(length_out,
+                          OP == Op::Union ? static_cast<int64_t>(sp.a1) + sp.b1 - all : all);
     }
     const unsigned long long side_w = reinterpret_cast<const unsigned long long *>(s_side)[l];
     const unsigned long long dup_w = reinterpret_cast<const unsigned long long *>(s_dup)[l];
@@ -1352,7 +1355,7 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
             NACHO_TRY(clear_words(s, sync.words, kSyncBytes / sizeof(unsigned long long)));
         }
         void (*fused)(EmitArgs, int, int, int, unsigned long long *, unsigned, unsigned,
-                      unsigned, unsigned, int64_t *, long long, float *) =
+                      unsigned, unsigned, int64_t *, float *) =
 #define NACHO_FUSED(OP, VAL, CHD, ROWS, DOT)             \
     (wide ? fused_kernel<OP, VAL, CHD, ROWS, DOT, true> \
           : fused_kernel<OP, VAL, CHD, ROWS, DOT, false>)
@@ -1368,7 +1371,7 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
         NACHO_TRY(call.timer_start(kernel_name));
         fused<<<num_tiles, kBlock, 0, s>>>(args, rows, static_cast<int>(total), crd_bits,
                                            sync.words, sync.epoch, sync.base, sync.done,
-                                           sync.polls, length_out, items, Z.dot);
+                                           sync.polls, length_out, Z.dot);
         NACHO_TRY_HIP(hipGetLastError());
         if (Z.dot) {
             call.sync_launched();
@@ -1438,7 +1441,7 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
                            : (wide ? order_kernel<true, false> : order_kernel<false, false>);
     order_fn<<<num_tiles, kBlock, 0, s>>>(A.pos, A.crd, B.pos, B.crd, split_r, split_a, split_b,
                                           crd_bits, side, dup, state, tile_pairs, counts, done,
-                                          length_out, intersect ? 1 : 0, items);
+                                          length_out, intersect ? 1 : 0);
     NACHO_TRY_HIP(hipGetLastError());
     if (!Z.dot) NACHO_TRY(call.mark_length());
     args.split_r = split_r;

@@ -333,3 +333,29 @@ def test_short_unsorted_rows(gpu, na, nb):
     got, exp = np.lexsort((crd, row)), np.lexsort((w[1], w[0]))
     assert np.array_equal(row[got], w[0][exp]) and np.array_equal(crd[got], w[1][exp])
     assert np.array_equal(val[got], w[2][exp])
+
+
+@pytest.mark.parametrize("rows,mean", [(50, 30), (90_000, 5), (90_000, 14)])
+@pytest.mark.parametrize("op", ["add", "mul"])
+def test_arrays_longer_than_the_entries(gpu, op, rows, mean):
+    """Coordinate and value arrays with room past the last offset: the result holds the entries
+    that the offsets span (in one launch, and in three with and without the sparse split)."""
+    import nacho_amd
+
+    rng = np.random.default_rng(mean)
+    cols, t = 200_000, []
+    for _ in range(2):
+        keys = np.unique(rng.integers(0, rows * cols, size=rows * mean))
+        pos = np.zeros(rows + 1, np.int32)
+        pos[1:] = np.cumsum(np.bincount(keys // cols, minlength=rows))
+        t.append((pos, (keys % cols).astype(np.int32),
+                  rng.uniform(-1, 1, len(keys)).astype(np.float32)))
+    want = oracle.closed_csr_binary(op, rows, cols, *t[0], *t[1])
+    room = [(pos, np.append(crd, np.full(777, 5, np.int32)),
+             np.append(val, np.full(777, 9, np.float32))) for pos, crd, val in t]
+    shape = torch.tensor([rows, cols], dtype=torch.int32)
+    print(f"[gpu] {op} rows={rows} mean={mean}, arrays with room", flush=True)
+    z = getattr(nacho_amd, f"gpu_csr_{op}_f32")(
+        *(nacho_amd.CSR_gpu(*(torch.from_numpy(x).to(gpu) for x in o), shape) for o in room))
+    got = tuple(x.cpu().numpy() for x in (z.dim_j_offsets, z.dim_j_indices, z.values))
+    assert_csr_equal(got, want, op)
