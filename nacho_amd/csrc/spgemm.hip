@@ -105,58 +105,163 @@ using dev::last_le;
 // ---- 1-2: sizes and segments -----------------------------------------------------------
 
 // Per row of A: its products, the A entries whose B row is not empty, its segments (1, or nb
-// for a long row) and, for a long row, its work blocks of kBlock A entries.  Eight lanes per
-// row; a row of more than kWave entries (a hub) is taken by its whole wavefront.
+// for a long row) and, for a long row, its work blocks of kBlock A entries.
+struct RowCounts {
+    int64_t *products;
+    int *entries;
+    int64_t *segments;
+    int64_t *blocks;
+    int nb;
+    // One entry of A, in column j.
+    static __device__ __forceinline__ void add(const int *__restrict__ pos_b, int j, int64_t &sum,
+                                               int &some) {
+        const int n = pos_b[j + 1] - pos_b[j];
+        sum += n;
+        some += n > 0 ? 1 : 0;
+    }
+    __device__ __forceinline__ void store(int64_t row, int len, int64_t sum, int some) const {
+        products[row] = sum;
+        entries[row] = some;
+        finish(row, len, sum);
+    }
+    __device__ __forceinline__ void finish(int64_t row, int len, int64_t sum) const {
+        segments[row] = sum > kShort ? nb : 1;
+        blocks[row] = sum > kShort ? (len + kBlock - 1) / kBlock : 0;
+    }
+};
+
+// LANES lanes per row.  A row of more than kWave entries is taken by its whole wavefront or, with
+// `split`, only zeroed: long_products_kernel adds it up.
 constexpr int kRowLanes = 8;
+constexpr int kOneLaneEntries = 4;  // per row on average, below which a row takes one lane
+// A's entries from which long rows are split: R-MAT graphs hold their longest rows side by side,
+// and one wavefront for each took 364 us at scale 20 (both kernels now: 176).  The launch costs
+// 3 us, a wavefront 80 us for all of fewer entries at worst.
+constexpr int64_t kSplitEntries = int64_t{1} << 15;
+
+template <int LANES>
 __global__ __launch_bounds__(kBlock) void row_products_kernel(
     const int *__restrict__ pos_a, const int *__restrict__ crd_a, int rows,
-    const int *__restrict__ pos_b, int nb, int64_t *__restrict__ products,
-    int *__restrict__ entries, int64_t *__restrict__ seg_count, int64_t *__restrict__ nblk) {
+    const int *__restrict__ pos_b, bool split, RowCounts out) {
     const int l = dev::lane();
-    const int64_t i = (blockIdx.x * static_cast<int64_t>(kBlock) + threadIdx.x) / kRowLanes;
-    const bool lead = l % kRowLanes == 0;
+    const int64_t i = (blockIdx.x * static_cast<int64_t>(kBlock) + threadIdx.x) / LANES;
+    const bool lead = l % LANES == 0;
     int s = 0, e = 0;
     if (i < rows) {
         s = pos_a[i];
         e = pos_a[i + 1];
     }
-    auto add = [&](int p, int64_t &sum, int &some) {
-        const int j = crd_a[p];
-        const int len = pos_b[j + 1] - pos_b[j];
-        sum += len;
-        some += len > 0 ? 1 : 0;
-    };
-    auto store = [&](int64_t row, int first, int last, int64_t sum, int some) {
-        products[row] = sum;
-        entries[row] = some;
-        seg_count[row] = sum > kShort ? nb : 1;
-        nblk[row] = sum > kShort ? (last - first + kBlock - 1) / kBlock : 0;
-    };
-    const bool hub = e - s > dev::kWave;
+    const bool is_long = e - s > dev::kWave;
     int64_t sum = 0;
     int some = 0;
-    if (!hub) {
+    if (!is_long) {
 #pragma unroll 4
-        for (int p = s + l % kRowLanes; p < e; p += kRowLanes) add(p, sum, some);
+        for (int p = s + l % LANES; p < e; p += LANES) out.add(pos_b, crd_a[p], sum, some);
     }
 #pragma unroll
-    for (int d = kRowLanes / 2; d > 0; d >>= 1) {
+    for (int d = LANES / 2; d > 0; d >>= 1) {
         sum += __shfl_xor(sum, d, dev::kWave);
         some += __shfl_xor(some, d, dev::kWave);
     }
-    if (lead && i < rows && !hub) store(i, s, e, sum, some);
-    unsigned long long hubs = __ballot(hub && lead);
-    while (hubs) {  // uniform
-        const int src = __ffsll(static_cast<long long>(hubs)) - 1;
-        hubs &= hubs - 1;
+    if (lead && i < rows && !is_long) out.store(i, e - s, sum, some);
+    if (split) {  // uniform
+        if (lead && is_long) {
+            out.products[i] = out.segments[i] = 0;
+            out.entries[i] = 0;
+        }
+        return;
+    }
+    unsigned long long rest = __ballot(is_long && lead);
+    while (rest) {  // uniform
+        const int src = __ffsll(static_cast<long long>(rest)) - 1;
+        rest &= rest - 1;
         const int hs = __shfl(s, src, dev::kWave), he = __shfl(e, src, dev::kWave);
-        int64_t hsum = 0;
-        int hsome = 0;
+        sum = 0;
+        some = 0;
 #pragma unroll 4
-        for (int p = hs + l; p < he; p += dev::kWave) add(p, hsum, hsome);
-        hsum = dev::wave_sum(hsum);
-        hsome = dev::wave_sum(hsome);
-        if (l == src) store(i, hs, he, hsum, hsome);
+        for (int p = hs + l; p < he; p += dev::kWave) out.add(pos_b, crd_a[p], sum, some);
+        sum = dev::wave_sum(sum);
+        some = dev::wave_sum(some);
+        if (l == src) out.store(i, e - s, sum, some);
+    }
+}
+
+// The rows of more than kWave entries: workgroup b takes A's entries [b * kLongSpan,
+// (b + 1) * kLongSpan), its wavefronts kLongPart entries of one such row among them at a time.
+// The parts of a row that reaches into several spans are added where they are counted, its
+// segments' word counts the parts, and the workgroup that adds the last one stores what follows
+// from the sum.
+constexpr int kLongSpan = 4096;
+constexpr int kLongPart = 4 * dev::kWave;
+
+__global__ __launch_bounds__(kBlock) void long_products_kernel(
+    const int *__restrict__ pos_a, const int *__restrict__ crd_a, int rows, int64_t nnz_a,
+    const int *__restrict__ pos_b, RowCounts out) {
+    constexpr int kWaves = kBlock / dev::kWave;
+    __shared__ int s_ends[2];
+    constexpr int kRows = kLongSpan / dev::kWave + 2;  // (the first and last may reach outside)
+    __shared__ int s_row[kRows];
+    __shared__ int s_rows;
+    __shared__ unsigned long long s_sum[kRows];
+    __shared__ int s_some[kRows];
+    const int lo = static_cast<int>(blockIdx.x) * kLongSpan;
+    const int hi = static_cast<int>(min(static_cast<int64_t>(lo) + kLongSpan, nnz_a));
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / dev::kWave), l = dev::lane();
+    if (w < 2) {  // the row of the first and of the last entry
+        const int at = w == 0 ? lo : hi - 1;
+        const int r = dev::group_last_true<dev::kWave>(0, rows - 1,
+                                                       [&](int x) { return pos_a[x] <= at; });
+        if (l == 0) s_ends[w] = r;
+    }
+    if (threadIdx.x == 0) s_rows = 0;
+    if (threadIdx.x < kRows) {
+        s_sum[threadIdx.x] = 0;
+        s_some[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    for (int r = s_ends[0] + static_cast<int>(threadIdx.x); r <= s_ends[1]; r += kBlock) {
+        const int e = pos_a[r + 1];
+        if (e - pos_a[r] > dev::kWave && e > lo) s_row[atomicAdd(&s_rows, 1)] = r;
+    }
+    __syncthreads();
+    for (int k = 0; k < s_rows; ++k) {
+        const int row = s_row[k];
+        const int s = max(pos_a[row], lo), e = min(pos_a[row + 1], hi);
+        // (row k's first part is wavefront k's: most rows have one)
+        for (int at = s + ((w - k) & (kWaves - 1)) * kLongPart; at < e; at += kWaves * kLongPart) {
+            int64_t sum = 0;
+            int some = 0;
+#pragma unroll
+            for (int u = 0; u < kLongPart; u += dev::kWave) {
+                if (at + u + l < e) out.add(pos_b, crd_a[at + u + l], sum, some);
+            }
+            sum = dev::wave_sum(sum);
+            some = dev::wave_sum(some);
+            if (l == 0) {
+                atomicAdd(&s_sum[k], static_cast<unsigned long long>(sum));
+                atomicAdd(&s_some[k], some);
+            }
+        }
+    }
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) >= s_rows) return;
+    const int row = s_row[threadIdx.x], some = s_some[threadIdx.x];
+    const unsigned long long sum = s_sum[threadIdx.x];
+    const int s = pos_a[row], e = pos_a[row + 1];
+    if (s >= lo && e <= hi) {
+        out.store(row, e - s, static_cast<int64_t>(sum), some);
+        return;
+    }
+    auto *products = reinterpret_cast<unsigned long long *>(&out.products[row]);
+    auto *parts = reinterpret_cast<unsigned long long *>(&out.segments[row]);
+    atomicAdd(products, sum);
+    atomicAdd(&out.entries[row], some);
+    const unsigned long long before =
+        __hip_atomic_fetch_add(parts, 1ull, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    if (before == static_cast<unsigned long long>((e - 1) / kLongSpan - s / kLongSpan)) {
+        out.finish(row, e - s,
+                   static_cast<int64_t>(__hip_atomic_load(products, __ATOMIC_RELAXED,
+                                                          __HIP_MEMORY_SCOPE_AGENT)));
     }
 }
 
@@ -1831,11 +1936,22 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
     int64_t *products = per_row, *seg_count = per_row + (rows + 1),
             *nblk = per_row + 2 * (static_cast<size_t>(rows) + 1);
     if (rows > 0) {
-        const int64_t blocks = (static_cast<int64_t>(rows) * kRowLanes + kBlock - 1) / kBlock;
-        row_products_kernel<<<static_cast<unsigned>(blocks), kBlock, 0, st>>>(
-            a->dim_j_offsets, a->dim_j_indices, rows, b->dim_j_offsets, nb, products, entries,
-            seg_count, nblk);
+        const int64_t nnz_a = a->dim_j_length;
+        const bool split = nnz_a > kSplitEntries;
+        const RowCounts counts{products, entries, seg_count, nblk, nb};
+        // (short rows: lanes of a row idle, and its counts are stored eight rows at a time)
+        const bool one = nnz_a < kOneLaneEntries * static_cast<int64_t>(rows);
+        const int64_t lanes = static_cast<int64_t>(rows) * (one ? 1 : kRowLanes);
+        auto kernel = one ? row_products_kernel<1> : row_products_kernel<kRowLanes>;
+        kernel<<<static_cast<unsigned>((lanes + kBlock - 1) / kBlock), kBlock, 0, st>>>(
+            a->dim_j_offsets, a->dim_j_indices, rows, b->dim_j_offsets, split, counts);
         NACHO_TRY_HIP(hipGetLastError());
+        if (split) {
+            long_products_kernel<<<static_cast<unsigned>((nnz_a + kLongSpan - 1) / kLongSpan), kBlock,
+                                   0, st>>>(a->dim_j_offsets, a->dim_j_indices, rows, nnz_a,
+                                            b->dim_j_offsets, counts);
+            NACHO_TRY_HIP(hipGetLastError());
+        }
     }
     int64_t *word[3] = {nullptr, nullptr, nullptr};  // counts read back on the way
     auto words = [&](int n) {

@@ -40,6 +40,28 @@ def test_with_and_without_long_rows(gpu, long_rows):
     run_and_check(gpu, n, n, 40000, a, b, f"{long_rows} long rows")
 
 
+@pytest.mark.parametrize("copies", [1, 4])
+@pytest.mark.parametrize("empty", [0, 60_000])
+def test_rows_of_a_by_length(gpu, copies, empty):
+    """A's rows on both sides of what a lane group takes (64), of the spans (4096) that long rows are
+    split into and of several of those, side by side; with and without the split (32,768 entries)
+    and, with many empty rows, one lane per row."""
+    rng = np.random.default_rng(copies + empty)
+    inner = 24_000
+    lengths = np.array([0, 1, 8, 9, 63, 64, 65, 66, 127, 500, 700, 4095, 4096, 4097, 9000] * copies
+                       + [20_000] * (copies > 1) + [0] * empty + [2] * 300)
+    if empty:
+        lengths = rng.permutation(lengths)
+    rows_a = [np.sort(rng.choice(inner, size=n, replace=False)).tolist() for n in lengths]
+    a = csr_from_rows(len(lengths), inner, rows_a,
+                      rng.uniform(0.5, 1.5, int(lengths.sum())).astype(np.float32))
+    rows_b = [np.sort(rng.choice(700, size=int(n), replace=False)).tolist()
+              for n in rng.integers(0, 4, inner)]
+    nnz_b = sum(len(r) for r in rows_b)
+    b = csr_from_rows(inner, 700, rows_b, rng.uniform(-1, 1, nnz_b).astype(np.float32))
+    run_and_check(gpu, len(lengths), inner, 700, a, b, f"{copies} copies, {empty} empty rows")
+
+
 @pytest.mark.parametrize("length", [2047, 2049])
 def test_runs_bounded_and_counted(gpu, length):
     """2048 rows of `length` products: either side of 2^22 products."""
