@@ -4,10 +4,11 @@
 // SpGEMM configuration (6.0e9 products).
 //
 // Two launches: every chunk's sum, then every chunk's scan, whose workgroup adds up the sums
-// of the chunks before its own (at most a few thousand words, read from L2) instead of waiting
-// for a launch that scans them, and whose last chunk stores the total.  Inputs of up to
-// kDirectChunks chunks need the second launch only: its workgroups add up the entries before
-// their own.  Against four launches (sums, their scan, chunks, total), or one of a single
+// of the chunks before its own (at most kSummedChunks words, read from L2) instead of waiting
+// for a launch that scans them, and whose last chunk stores the total.  Inputs of more chunks have
+// their sums scanned by a launch in between: what the workgroups read of them otherwise grows
+// with the square.  Inputs of up to kDirectChunks chunks need the last launch only: its
+// workgroups add up the entries before their own.  Against four launches (sums, their scan, chunks, total), or one of a single
 // workgroup up to 32,768 entries (10.8 us), 8 to 10 us less per scan on MI355X.
 #include <hip/hip_runtime.h>
 
@@ -23,6 +24,8 @@ constexpr int kBlock = 256;
 constexpr int kPerThread = 16;
 constexpr int kChunk = kBlock * kPerThread;
 constexpr unsigned kDirectChunks = 4;  // a launch costs about as much as reading 3 chunks
+constexpr unsigned kSummedChunks = 2048;
+constexpr int kSumsBlock = 1024;
 
 struct Jobs {
     const int64_t *in[kMaxJobs];
@@ -60,9 +63,26 @@ __global__ __launch_bounds__(kBlock) void chunk_sums_kernel(Jobs jobs,
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-// sums: the chunks' sums, or null (few chunks).
+// Workgroup j: the sums of job j's chunks become those of the chunks before each.
+__global__ __launch_bounds__(kSumsBlock) void scan_sums_kernel(Jobs jobs,
+                                                               int64_t *__restrict__ sums) {
+    __shared__ int64_t s_wave[kSumsBlock / dev::kWave];
+    const unsigned first = jobs.first[blockIdx.x], end = jobs.first[blockIdx.x + 1];
+    int64_t carry = 0;
+    for (unsigned c0 = first; c0 < end; c0 += kSumsBlock) {  // uniform
+        const unsigned c = c0 + threadIdx.x;
+        const int64_t v = c < end ? sums[c] : 0;
+        int64_t total = 0;
+        const int64_t before = dev::block_exclusive_sum<kSumsBlock>(v, s_wave, total);
+        if (c < end) sums[c] = carry + before;
+        carry += total;
+    }
+}
+
+// sums: the chunks' sums, those of the chunks before (`scanned`), or null (few chunks).
 __global__ __launch_bounds__(kBlock) void scan_chunks_kernel(Jobs jobs,
-                                                             const int64_t *__restrict__ sums) {
+                                                             const int64_t *__restrict__ sums,
+                                                             bool scanned) {
     __shared__ int64_t s_wave[kBlock / dev::kWave];
     unsigned chunk;
     const int job = job_of(jobs, blockIdx.x, chunk);
@@ -80,7 +100,9 @@ __global__ __launch_bounds__(kBlock) void scan_chunks_kernel(Jobs jobs,
         mine += v[j];
     }
     int64_t before = 0, carry = 0;
-    if (chunk > 0) {  // uniform
+    if (scanned) {  // uniform
+        carry = sums[blockIdx.x];
+    } else if (chunk > 0) {
         if (!sums) {
 #pragma unroll 8
             for (int64_t i = threadIdx.x; i < base; i += kBlock) before += in[i];
@@ -109,7 +131,8 @@ int exclusive_scans(Call &call, const Job *jobs, int count) {
     if (count < 1 || count > kMaxJobs) return NACHO_ERR_INVALID_ARGUMENT;
     Jobs j{};
     j.count = count;
-    bool direct = true;  // every input is a few chunks
+    bool direct = true;    // every input is a few chunks
+    bool scanned = false;  // some input is many
     int64_t chunks = 0;
     for (int k = 0; k < count; ++k) {
         j.in[k] = jobs[k].in;
@@ -119,6 +142,7 @@ int exclusive_scans(Call &call, const Job *jobs, int count) {
         j.first[k] = static_cast<unsigned>(chunks);
         const int64_t c = jobs[k].n > 0 ? (jobs[k].n + kChunk - 1) / kChunk : 1;
         direct = direct && c <= kDirectChunks;
+        scanned = scanned || c > kSummedChunks;
         chunks += c;
         if (chunks > INT32_MAX) return NACHO_ERR_INDEX_OVERFLOW;
     }
@@ -129,8 +153,12 @@ int exclusive_scans(Call &call, const Job *jobs, int count) {
         NACHO_TRY(call.scratch_n(static_cast<size_t>(chunks), &sums));
         chunk_sums_kernel<<<static_cast<unsigned>(chunks), kBlock, 0, s>>>(j, sums);
         NACHO_TRY_HIP(hipGetLastError());
+        if (scanned) {
+            scan_sums_kernel<<<static_cast<unsigned>(count), kSumsBlock, 0, s>>>(j, sums);
+            NACHO_TRY_HIP(hipGetLastError());
+        }
     }
-    scan_chunks_kernel<<<static_cast<unsigned>(chunks), kBlock, 0, s>>>(j, sums);
+    scan_chunks_kernel<<<static_cast<unsigned>(chunks), kBlock, 0, s>>>(j, sums, scanned);
     NACHO_TRY_HIP(hipGetLastError());
     return NACHO_OK;
 }

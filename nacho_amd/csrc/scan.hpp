@@ -17,7 +17,7 @@ struct Job {
     int64_t *total = nullptr;
 };
 
-// Up to kMaxJobs independent scans at once: one launch when every input is short, two
+// Up to kMaxJobs independent scans at once: one launch when every input is short, two or three
 // otherwise.  Runs on the call's stream; scratch comes from the call.
 constexpr int kMaxJobs = 4;
 int exclusive_scans(Call &call, const Job *jobs, int count);

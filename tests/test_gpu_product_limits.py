@@ -1,7 +1,7 @@
-"""The products' size rules at their limits: scans of up to four chunks of 4096 in one launch and
-longer ones in two, SpGEMM with and without long rows and past the run count that is bounded
-instead of counted (2^22 products), sssmm chunks of more mask entries than keep their fields and
-sums in LDS (256)."""
+"""The products' size rules at their limits: scans of up to four chunks of 4096 in one launch, of
+up to 2048 in two and longer ones in three, SpGEMM with and without long rows and past the run
+count that is bounded instead of counted (2^22 products), sssmm chunks of more mask entries than
+keep their fields and sums in LDS (256)."""
 
 from __future__ import annotations
 
@@ -10,7 +10,7 @@ import pytest
 
 from oracle import oracle
 from tests.helpers import csr_from_rows, random_csr
-from tests.test_gpu_spgemm import run_and_check
+from tests.test_gpu_spgemm import run_and_check, spgemm
 from tests.test_gpu_sssmm import check as check_sssmm
 from tests.test_gpu_sssmm import run as run_sssmm
 
@@ -23,6 +23,29 @@ def test_scans_at_chunk_limits(gpu, rows):
     a = random_csr(rng, rows, 64, 0.02)
     b = random_csr(rng, 64, 500, 0.05)
     run_and_check(gpu, rows, 64, 500, a, b, f"{rows} rows")
+
+
+@pytest.mark.parametrize("chunks,more", [(2048, 0), (2048, 1), (2049, 4095), (3100, 7)])
+def test_scans_of_many_chunks(gpu, chunks, more):
+    """Either side of the 2048 chunks whose sums a chunk adds up itself: rows of A with one entry
+    or none, B rows of 0 to 2 entries."""
+    rng = np.random.default_rng(chunks + more)
+    rows, inner = chunks * 4096 + more, 1000
+    pos = np.zeros(rows + 1, np.int64)
+    np.cumsum(rng.random(rows) < 0.25, out=pos[1:])
+    crd = rng.integers(0, inner, pos[-1]).astype(np.int32)
+    a = (pos.astype(np.int32), crd, rng.uniform(0.5, 1.5, len(crd)).astype(np.float32))
+    len_b = rng.integers(0, 3, inner)
+    pos_b = np.concatenate([[0], np.cumsum(len_b)]).astype(np.int32)
+    crd_b = np.concatenate([np.sort(rng.choice(50, n, replace=False)) for n in len_b])
+    b = (pos_b, crd_b.astype(np.int32), rng.uniform(-1, 1, len(crd_b)).astype(np.float32))
+    got = spgemm(a, b, rows, inner, 50, gpu)
+    n = len_b[crd]  # a row's result is its one B row, scaled
+    want_pos = np.concatenate([[0], np.cumsum(n)])[pos]
+    assert np.array_equal(got[0], want_pos)
+    at = np.repeat(pos_b[crd] - np.concatenate([[0], np.cumsum(n)[:-1]]), n) + np.arange(n.sum())
+    assert np.array_equal(got[1], b[1][at])
+    assert np.array_equal(got[2], np.repeat(a[2], n) * b[2][at])
 
 
 @pytest.mark.parametrize("long_rows", [0, 1, 3])
