@@ -108,3 +108,21 @@ def test_sssmm_entries_per_chunk(gpu, probes):
     c = random_csr(rng, n, 100, 0.8)
     check_sssmm(run_sssmm(a, b, c, ((n, inner), (inner, 100), (n, 100)), gpu),
                 oracle.port_sssmm(n, 100, a, b, c), f"{probes} probes")
+
+
+@pytest.mark.parametrize("half", [0, 1, 2, 7, 8, 12, 40])
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_sssmm_bands(gpu, half, shuffled):
+    """Bands: lists of 2 half + 1 entries, nearly every probe hits, several lanes of a wavefront on
+    one mask entry; and the same with every third mask entry elsewhere (misses among the hits)."""
+    rng = np.random.default_rng(half)
+    n = 3000
+    rows = [list(range(max(0, i - half), min(n, i + half + 1))) for i in range(n)]
+    a, b = (csr_from_rows(n, n, rows, rng.uniform(-1, 1, sum(map(len, rows))).astype(np.float32))
+            for _ in range(2))
+    mask = rows
+    if shuffled:
+        mask = [sorted({k if (i + k) % 3 else (k * 7919) % n for k in r}) for i, r in enumerate(rows)]
+    c = csr_from_rows(n, n, mask, rng.uniform(0.5, 1.5, sum(map(len, mask))).astype(np.float32))
+    check_sssmm(run_sssmm(a, b, c, ((n, n),) * 3, gpu), oracle.port_sssmm(n, n, a, b, c),
+                f"band {half}")
