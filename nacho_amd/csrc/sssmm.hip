@@ -72,13 +72,11 @@ __device__ __forceinline__ uint32_t mix(uint32_t x) {
 // The filter's bit of a key in its home slot's byte.
 __device__ __forceinline__ uint32_t filter_bit(uint32_t hash) { return hash >> 29; }
 
-__device__ __forceinline__ void table_insert(uint64_t *table, unsigned *filter, int64_t base,
-                                             uint32_t mask, uint32_t key, float value) {
+// Inserts the key into its table; the caller has set its bit in the filter (hash: mix(key)).
+__device__ __forceinline__ void table_insert(uint64_t *table, int64_t base, uint32_t mask,
+                                             uint32_t key, uint32_t hash, float value) {
     const uint64_t word = (static_cast<uint64_t>(__float_as_uint(value)) << 32) | key;
-    const uint32_t hash = mix(key);
     uint32_t h = hash & mask;
-    const int64_t home = base + h;
-    atomicOr(&filter[home >> 2], 1u << (8u * static_cast<uint32_t>(home & 3) + filter_bit(hash)));
     for (;;) {
         auto *slot = reinterpret_cast<unsigned long long *>(table + base + h);
         if (atomicCAS(slot, static_cast<unsigned long long>(kEmptySlot),
@@ -87,6 +85,11 @@ __device__ __forceinline__ void table_insert(uint64_t *table, unsigned *filter, 
         }
         h = (h + 1) & mask;
     }
+}
+
+// A key's bit in the filter's word (of four slots) of its home slot.
+__device__ __forceinline__ unsigned filter_word_bit(int64_t home, uint32_t hash) {
+    return 1u << (8u * static_cast<uint32_t>(home & 3) + filter_bit(hash));
 }
 
 __global__ void fill_kernel(uint64_t *__restrict__ p, int64_t n, uint64_t v) {
@@ -197,25 +200,63 @@ __global__ __launch_bounds__(kBlock) void transpose_kernel(
         const int64_t slot = col_off[k] + static_cast<int64_t>(atomicAdd(&col_fill[k], 1ull));
         csc_row[slot] = j;
         csc_val[slot] = v;
-        const int64_t size = tab_off[k + 1] - tab_off[k];
-        table_insert(tab_b, filter, tab_off[k], static_cast<uint32_t>(size - 1),
-                     static_cast<uint32_t>(j), v);
+        const int64_t base = tab_off[k];
+        const uint32_t mask = static_cast<uint32_t>(tab_off[k + 1] - base - 1);
+        const uint32_t hash = mix(static_cast<uint32_t>(j));
+        const int64_t home = base + (hash & mask);
+        atomicOr(&filter[home >> 2], filter_word_bit(home, hash));
+        table_insert(tab_b, base, mask, static_cast<uint32_t>(j), hash, v);
     }
 }
 
-// A's entries into the per-row tables keyed by column id, which start at slot `first`.
+// A's entries into the per-row tables keyed by column id, which start at slot `first`.  The filter
+// of the rows that lie inside the workgroup's span, whose tables are neighbours, is built in LDS
+// and stored; that of a row which reaches out of it by global atomics.  (All by global atomics,
+// where the entries of a short row meet in a few words: 310 us for the 3.9M entries of a band of
+// 15 a row, 182 so, 195 without a filter.)
 __global__ __launch_bounds__(kBlock) void rows_table_kernel(
     const int *__restrict__ pa, int rows, const int *__restrict__ ca,
     const float *__restrict__ va, int64_t nnz_a, int span, const int64_t *__restrict__ tab_off,
     uint64_t *__restrict__ tab, unsigned *__restrict__ filter, int64_t first) {
+    // (a list's table is smaller than four times its length, and starts anywhere in a word)
+    constexpr int kWords = kSpan + 1;
+    __shared__ unsigned s_filter[kWords];
     int64_t lo, hi;
     int r_lo, r_hi;
     if (!span_rows(pa, rows, nnz_a, span, lo, hi, r_lo, r_hi)) return;
+    const int i0 = pa[r_lo] >= lo ? r_lo : r_lo + 1;       // rows [i0, i1) lie inside
+    const int i1 = pa[r_hi + 1] <= hi ? r_hi + 1 : r_hi;
+    const int64_t s0 = i0 < i1 ? first + tab_off[i0] : 0;  // their slots
+    const int64_t s1 = i0 < i1 ? first + tab_off[i1] : 0;
+    const int64_t w0 = s0 >> 2;
+    const int words = static_cast<int>((s1 + 3) / 4 - w0);
+    for (int x = threadIdx.x; x < words; x += kBlock) s_filter[x] = 0u;
+    __syncthreads();
     for (int64_t e = lo + threadIdx.x; e < hi; e += kBlock) {
         const int i = static_cast<int>(last_le(pa, r_lo, r_hi, e));
-        const int64_t size = tab_off[i + 1] - tab_off[i];
-        table_insert(tab, filter, first + tab_off[i], static_cast<uint32_t>(size - 1),
-                     static_cast<uint32_t>(ca[e]), va[e]);
+        const int64_t base = first + tab_off[i];
+        const uint32_t mask = static_cast<uint32_t>(first + tab_off[i + 1] - base - 1);
+        const uint32_t key = static_cast<uint32_t>(ca[e]);
+        const uint32_t hash = mix(key);
+        const int64_t home = base + (hash & mask);
+        const unsigned bit = filter_word_bit(home, hash);
+        if (i >= i0 && i < i1) {
+            atomicOr(&s_filter[static_cast<int>((home >> 2) - w0)], bit);
+        } else {
+            atomicOr(&filter[home >> 2], bit);
+        }
+        table_insert(tab, base, mask, key, hash, va[e]);
+    }
+    __syncthreads();
+    for (int x = threadIdx.x; x < words; x += kBlock) {
+        const unsigned v = s_filter[x];
+        if (v == 0) continue;
+        const int64_t at = 4 * (w0 + x);
+        if (at >= s0 && at + 4 <= s1) {
+            filter[w0 + x] = v;  // (zeroed before)
+        } else {
+            atomicOr(&filter[w0 + x], v);  // shared with a neighbour's table
+        }
     }
 }
 
@@ -260,7 +301,8 @@ __global__ void chunk_bounds_kernel(const int64_t *__restrict__ woff, int64_t nn
 // fields in LDS and sums them there (binary64 LDS atomics, then one global atomic per entry); a
 // chunk of more, short ones reads the fields from memory, and each wavefront sums an entry's hits
 // in LDS before one global atomic for its 64 probes.  (With a global atomic for every hit, the
-// probes of a band of 15 entries a row, where most hit, took 2088 us instead of 439.)
+// probes of a band of 15 entries a row, where most hit, took 2088 us instead of 439.  A band of 17,
+// 241 mask entries a chunk: 1368 us a call in LDS, 1505 the other way.)
 constexpr int kAccEntries = 256;
 static_assert(kAccEntries == kBlock, "or one slot per lane");
 
