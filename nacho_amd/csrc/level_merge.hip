@@ -90,11 +90,15 @@ __device__ __forceinline__ int bits_below(unsigned long long m) {
 // dependent loads, so what counts is how many tiles are in flight.  C2: 24 us with the split,
 // and 11 us for the order kernel on the tiles left (2%), against 8.5 us for the split and 65
 // for ordering every tile.  Where rows hold few entries (or, in tensors, thousands of both
-// operands) most tiles are dense and the look would be lost: 5 us of 106 for 8 entries a row.
+// operands) most tiles are dense and the look is lost.
 constexpr int kMaxSearches = 256;  // entries to search
 constexpr int kMaxSearchRows = 512;
 constexpr int kSearchWays = 8;     // of a lower bound: probes per round + 1
-// Entries of both operands per row from which a union looks for sparse tiles.
+// Entries of both operands per row from which a union looks for sparse tiles.  How even the rows
+// are, which decides what the look brings, is not known here.  csr_add of 700,000 rows, looking /
+// not: Zipf rows of 5, 6, 8, 10, 16, 32 entries per operand 48.3 / 48.4, 53.5 / 54.5, 59.1 /
+// 64.1, 67.7 / 78.2, 103.5 / 117.3, 183.5 / 216.1 us, even rows 51.8 / 47.2, 58.4 / 53.3, 69.2 /
+// 62.3, 83.1 / 80.3, 134.7 / 129.3, 240.6 / 231.1; below 4 per operand neither gains by it.
 constexpr int kSparseEntriesPerRow = 8;
 constexpr unsigned kDense = UINT_MAX;  // tile_pairs of a tile left to the order kernel
 
