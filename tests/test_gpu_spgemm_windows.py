@@ -41,17 +41,23 @@ def test_dense_units(gpu, monkeypatch, runs, length, mode):
 @pytest.mark.parametrize("buckets", [3, 9])
 def test_bitmap_units(gpu, per_bucket, buckets):
     """A long row with `per_bucket` products in each of its column buckets but the last, which
-    makes the row long."""
+    makes the row long; two products on every column."""
     rng = np.random.default_rng(per_bucket + buckets)
     cols = 8192 * (buckets + 1)
     m = 33
     rows_b = [[] for _ in range(m)]
     for bucket in range(buckets):
-        for p in range(per_bucket):  # uneven runs, one column repeated over the rows
-            rows_b[(p * p + bucket) % m].append(bucket * 8192 + (p * 37) % 8192)
+        for p in range(per_bucket):  # uneven runs, columns in pairs on two rows
+            q = p // 2
+            rows_b[(q * q + bucket + 3 * (p % 2)) % m].append(bucket * 8192 + (q * 37) % 8192)
     rows_b[0] += list(range(buckets * 8192, buckets * 8192 + 2200))
-    rows_b = [sorted(set(r)) for r in rows_b]
+    rows_b[1] += list(range(buckets * 8192 + 1000, buckets * 8192 + 1500))
+    rows_b = [sorted(r) for r in rows_b]
+    assert all(len(set(r)) == len(r) for r in rows_b)
     nnz = sum(len(r) for r in rows_b)
+    distinct = len(set().union(*rows_b))
+    assert nnz == buckets * per_bucket + 2700
+    assert distinct == buckets * ((per_bucket + 1) // 2) + 2200
     a = csr_from_rows(2, m, [list(range(m)), list(range(0, m, 3))],
                       rng.uniform(0.5, 1.5, m + (m + 2) // 3).astype(np.float32))
     b = csr_from_rows(m, cols, rows_b, rng.uniform(-1, 1, nnz).astype(np.float32))
