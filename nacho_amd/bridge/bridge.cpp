@@ -17,6 +17,8 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
+#include <exception>
+#include <string>
 
 #include "../../include/nacho_hip.h"
 
@@ -240,17 +242,27 @@ PyObject *invoke(PyObject *, PyObject *const *args, Py_ssize_t n) {
             }
         }
         int rc = 0;
+        std::string failure;  // an exception must not pass the point where the lock is taken again
         Py_BEGIN_ALLOW_THREADS
-        if (operands == 2) {
-            using Fn = int (*)(const void *, const void *, void *, int32_t, int32_t, void *,
-                               const nacho_allocator *);
-            rc = reinterpret_cast<Fn>(entry)(&d[0], &d[1], &z, nb, tpb, stream, nullptr);
-        } else {
-            using Fn = int (*)(const void *, const void *, const void *, void *, int32_t, int32_t,
-                               void *, const nacho_allocator *);
-            rc = reinterpret_cast<Fn>(entry)(&d[0], &d[1], &d[2], &z, nb, tpb, stream, nullptr);
+        try {
+            if (operands == 2) {
+                using Fn = int (*)(const void *, const void *, void *, int32_t, int32_t, void *,
+                                   const nacho_allocator *);
+                rc = reinterpret_cast<Fn>(entry)(&d[0], &d[1], &z, nb, tpb, stream, nullptr);
+            } else {
+                using Fn = int (*)(const void *, const void *, const void *, void *, int32_t,
+                                   int32_t, void *, const nacho_allocator *);
+                rc = reinterpret_cast<Fn>(entry)(&d[0], &d[1], &d[2], &z, nb, tpb, stream,
+                                                 nullptr);
+            }
+        } catch (const std::exception &e) {
+            failure = std::string("the entry point threw: ") + e.what();
         }
         Py_END_ALLOW_THREADS
+        if (!failure.empty()) {
+            PyErr_SetString(PyExc_RuntimeError, failure.c_str());
+            return nullptr;
+        }
         if (rc != 0) return PyLong_FromLong(rc);
         return adopt(static_cast<int>(kind), z, device, stream);
     } catch (const std::exception &e) {

@@ -99,3 +99,25 @@ def test_buffer_returns_to_the_allocator_with_its_last_view(gpu):
     assert view.tolist() == expect
     del view
     assert na.cached_bytes() >= idle
+
+
+def test_exception_of_an_entry_point(gpu, tmp_path):
+    """A C++ exception out of the library (no host memory, say) arrives as a Python one, and the
+    interpreter goes on."""
+    import ctypes
+    import subprocess
+
+    from nacho_amd import _lib, ops
+
+    src = tmp_path / "throws.cpp"
+    src.write_text('#include <new>\nextern "C" int throws() { throw std::bad_alloc(); }\n')
+    lib = tmp_path / "throws.so"
+    subprocess.run(["g++", "-shared", "-fPIC", str(src), "-o", str(lib)], check=True)
+    address = ctypes.cast(ctypes.CDLL(str(lib)).throws, ctypes.c_void_p).value
+    a, b = _operands("csr", gpu, 8)
+    bridge = _lib.load_bridge()
+    args = [x for t in (a, b) for x in (ops._CSR.kind, ops._CSR.buffers(t), t._dims)]
+    for _ in range(3):
+        with pytest.raises(RuntimeError, match="bad_alloc"):
+            bridge.invoke(address, ops._CSR.kind, 256, 256, 0, 0, *args)
+    assert na.gpu_csr_add_f32(a, b).values.tolist() == (2 * a.values).tolist()
