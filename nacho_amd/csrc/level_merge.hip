@@ -98,7 +98,7 @@ constexpr int kSearchWays = 8;     // of a lower bound: probes per round + 1
 // are, which decides what the look brings, is not known here.  csr_add of 700,000 rows, looking /
 // not: Zipf rows of 5, 6, 8, 10, 16, 32 entries per operand 48.3 / 48.4, 53.5 / 54.5, 59.1 /
 // 64.1, 67.7 / 78.2, 103.5 / 117.3, 183.5 / 216.1 us, even rows 51.8 / 47.2, 58.4 / 53.3, 69.2 /
-// 62.3, 83.1 / 80.3, 134.7 / 129.3, 240.6 / 231.1; below 4 per operand neither gains by it.
+// 62.3, 83.1 / 80.3, 134.7 / 129.3, 240.6 / 231.1.
 constexpr int kSparseEntriesPerRow = 8;
 constexpr unsigned kDense = UINT_MAX;  // tile_pairs of a tile left to the order kernel
 
