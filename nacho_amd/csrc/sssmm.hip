@@ -14,8 +14,8 @@
 // A B (R-MAT scale 20 squared and masked by itself: 1.1e9 probes against 6.0e9 products).
 //
 //   count_cols_kernel, scan          column counts of B, column offsets
-//   table_sizes_kernel (x2), scans   hash table sizes (power of two >= 2 * length) and bases
-//   fill_kernel                      empty tables
+//   table_sizes_kernel, scans        hash table sizes (power of two >= 2 * length) and bases
+//   fill_kernel                      empty tables, zeroed filter
 //   transpose_kernel                 B's entries into columns (row ids + values), and into
 //                                    the per-column tables keyed by row id
 //   rows_table_kernel                A's entries into the per-row tables keyed by column id
@@ -26,13 +26,14 @@
 //                                    to mask entries (max-scan of entry start marks in LDS),
 //                                    walk, filter, probe, (a * b) * c per hit in float32 as
 //                                    written, summed per entry in float64 in LDS, one atomic
-//                                    add per entry and chunk
+//                                    add per entry and chunk (of few mask entries) or per
+//                                    entry and wavefront
 //   keep_kernel, scan, output_kernel the entries that some product reached, in C's order
 //
 // Values: each term is rounded as the reference writes it, ((a * b) * c) in float32, and the
 // terms of an entry are summed in float64 and rounded once.  The order of the float64 sums
-// follows atomic arrival, so values are reproducible within
-// one float32 rounding; the structure is exact.
+// follows atomic arrival, so values are reproducible within one float32 rounding; the structure
+// is exact.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -314,11 +315,12 @@ struct EntryFields {
     int64_t table;
 };
 
-// Bound by the lines its random reads fetch (at C4 a 134 MB table each side, one line per 8-byte
-// probe: 58 GB in 10.5 ms) and by LDS issue.  R-MAT 2^20 masked by itself, 1.14e9 probes: sums
-// in LDS instead of a segmented sum by shuffles per 64 probes 10.5 -> 9.7 ms; the filter, whose
-// bytes mostly stay in L2 and which tells most misses, 6.9; the entries' fields in LDS and the
-// values read after the filter, four rounds at a time, 5.7 (two rounds 6.0, eight 7.0).
+// Bound by the lines that its random reads fetch: R-MAT 2^20 masked by itself, 1.14e9 probes into
+// 134 MB of slots each side, 23 GB in 5.7 ms.  Without the filter, whose bytes mostly stay in L2
+// and which tells most misses, one line per probe: 58 GB in 10.5 ms.  On the way: sums in LDS
+// instead of a segmented sum by shuffles per 64 probes 10.5 -> 9.7 ms; the filter 6.9; the entries'
+// fields in LDS and the values read after the filter, four rounds at a time, 5.7 (two rounds 6.0,
+// eight 7.0).
 __global__ __launch_bounds__(kBlock) void probe_kernel(
     const int64_t *__restrict__ woff, const int64_t *__restrict__ bounds, int64_t total,
     const int64_t *__restrict__ walk_base, const int64_t *__restrict__ probe_base,
