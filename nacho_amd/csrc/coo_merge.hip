@@ -1066,7 +1066,7 @@ int nacho_gpu_coo3d_add_f32(const nacho_coo3 *a, const nacho_coo3 *b, nacho_coo3
     }
     NACHO_TRY(nacho::check_launch_hints(num_blocks, threads_per_block));
     const long long entries = static_cast<long long>(a->nnz) + b->nnz;
-    // the row path's column keys stay below INT_MAX, the merge's exhausted-row sentinel
+    // (extents whose largest column key is INT_MAX take the packed path)
     const int kbits = bits_for_extent(a->dim_k_size);
     const bool keys_fit = a->dim_j_size >= 1 && a->dim_k_size >= 1 &&
                           bits_for_extent(a->dim_j_size) + kbits <= 31 &&

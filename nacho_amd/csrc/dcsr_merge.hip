@@ -191,8 +191,8 @@ int dcsr_binary(bool intersect, const nacho_dcsr *a, const nacho_dcsr *b, nacho_
     long long ni = nu;
     if (intersect) {
         // The kept rows are compacted into arrays sized for all nu rows, so nothing waits for
-        // their count; it and the j level's length are read once the j level's write pass has
-        // ended, while its compaction and this one may still run (stream-ordered).
+        // their count; it and the j level's length are read once the j level's order pass has
+        // ended, while its write pass and this one may still run (stream-ordered).
         NACHO_TRY(call.collect_timer());  // (kernel timing only) the j level's interval
         NACHO_TRY(call.result_n(static_cast<size_t>(nu), &crd_i));
         NACHO_TRY(call.result_n(static_cast<size_t>(nu) + 1, &pos_j));
