@@ -33,9 +33,10 @@
  * Input contract (the reference's, made explicit): pos[0] == 0, pos non-decreasing,
  * pos[rows] == length of the coordinate array, coordinates strictly increasing within
  * each fibre (sorted, no duplicates) and in [0, extent) of their dimension, COO/COO3
- * coordinates sorted lexicographically and distinct.  As in the reference, the entry points do not check it on the device: host-side
- * shape and pointer checks return NACHO_ERR_INVALID_ARGUMENT, operand contents are trusted,
- * and nacho_validate_csr() checks a CSR operand on request.
+ * coordinates sorted lexicographically and distinct.  As in the reference, the entry points
+ * do not check it on the device: host-side shape and pointer checks return
+ * NACHO_ERR_INVALID_ARGUMENT, operand contents are trusted, and nacho_validate_csr() checks a
+ * CSR operand on request.
  */
 #ifndef NACHO_HIP_H
 #define NACHO_HIP_H

@@ -51,9 +51,9 @@ static_assert(kLevelItemSlack <= 2 * kLevelTileSlack, "what callers route here i
 // Merge A and B row by row: union (or intersection) of each row's coordinates, with values
 // (a+b / a*b / copies) when `values`, or with child pointers when `child` (unions only).
 // Coordinates are ordered as int32 numbers; those of the extent lie in [0, 2^crd_bits),
-// crd_bits <= 31, and others (walked, slowly) are merged as well.  Writes Z.pos for every row and returns
-// the result length in *out_len.  The call's kernel timer (if enabled) brackets all of the
-// level's kernels under `kernel_name`.
+// crd_bits <= 31, and others are merged as well, by a slow walk.  Writes Z.pos for every row and
+// returns the result length in *out_len.  The call's kernel timer (if enabled) brackets all of
+// the level's kernels under `kernel_name`.
 //
 // With `length_pending`, the host does not wait for the length: *length_pending is set,
 // *out_len is left alone, and the caller, having queued what it has to on the stream, reads

@@ -554,8 +554,12 @@ __device__ __forceinline__ void walk_tile(const TileSplit &sp, const int *__rest
     const int first = kPer * tid, count = min(max(na + nb - first, 0), kPer);
     side = dup = 0;
     if (count == 0) return;
-    auto begin_a = [&](int k) { return k == 0 ? 0 : k >= nr ? na : min(max(pa[sp.r0 + k] - sp.a0, 0), na); };
-    auto begin_b = [&](int k) { return k == 0 ? 0 : k >= nr ? nb : min(max(pb[sp.r0 + k] - sp.b0, 0), nb); };
+    auto begin_a = [&](int k) {
+        return k == 0 ? 0 : k >= nr ? na : min(max(pa[sp.r0 + k] - sp.a0, 0), na);
+    };
+    auto begin_b = [&](int k) {
+        return k == 0 ? 0 : k >= nr ? nb : min(max(pb[sp.r0 + k] - sp.b0, 0), nb);
+    };
     int k = 0;  // the last row that begins at or before the slot
     for (int hi = nr - 1; k < hi;) {
         const int mid = (k + hi + 1) >> 1;

@@ -8,8 +8,9 @@
 // for a launch that scans them, and whose last chunk stores the total.  Inputs of more chunks have
 // their sums scanned by a launch in between: what the workgroups read of them otherwise grows
 // with the square.  Inputs of up to kDirectChunks chunks need the last launch only: its
-// workgroups add up the entries before their own.  Against four launches (sums, their scan, chunks, total), or one of a single
-// workgroup up to 32,768 entries (10.8 us), 8 to 10 us less per scan on MI355X.
+// workgroups add up the entries before their own.  Against four launches (sums, their scan,
+// chunks, total), or one of a single workgroup up to 32,768 entries (10.8 us), 8 to 10 us less
+// per scan on MI355X; above kSummedChunks, a product of 128M rows 24.2 -> 20.5 ms a call.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

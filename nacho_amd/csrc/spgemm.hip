@@ -1947,9 +1947,9 @@ int multiply(Call &call, const nacho_csr *a, const nacho_csr *b, Product *z) {
             a->dim_j_offsets, a->dim_j_indices, rows, b->dim_j_offsets, split, counts);
         NACHO_TRY_HIP(hipGetLastError());
         if (split) {
-            long_products_kernel<<<static_cast<unsigned>((nnz_a + kLongSpan - 1) / kLongSpan), kBlock,
-                                   0, st>>>(a->dim_j_offsets, a->dim_j_indices, rows, nnz_a,
-                                            b->dim_j_offsets, counts);
+            const int64_t spans = (nnz_a + kLongSpan - 1) / kLongSpan;
+            long_products_kernel<<<static_cast<unsigned>(spans), kBlock, 0, st>>>(
+                a->dim_j_offsets, a->dim_j_indices, rows, nnz_a, b->dim_j_offsets, counts);
             NACHO_TRY_HIP(hipGetLastError());
         }
     }

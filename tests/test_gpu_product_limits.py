@@ -122,7 +122,8 @@ def test_sssmm_bands(gpu, half, shuffled):
             for _ in range(2))
     mask = rows
     if shuffled:
-        mask = [sorted({k if (i + k) % 3 else (k * 7919) % n for k in r}) for i, r in enumerate(rows)]
+        mask = [sorted({k if (i + k) % 3 else (k * 7919) % n for k in r})
+                for i, r in enumerate(rows)]
     c = csr_from_rows(n, n, mask, rng.uniform(0.5, 1.5, sum(map(len, mask))).astype(np.float32))
     check_sssmm(run_sssmm(a, b, c, ((n, n),) * 3, gpu), oracle.port_sssmm(n, n, a, b, c),
                 f"band {half}")
