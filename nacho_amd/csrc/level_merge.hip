@@ -767,15 +767,16 @@ __global__ __launch_bounds__(kBlock, WIDE ? 4 : 6) void order_kernel(
     const int w = __builtin_amdgcn_readfirstlane(tid / dev::kWave);
     const int t = blockIdx.x;
     const int c = t / kChunk;
-    // (of the offsets: an operand's arrays may be longer)
-    const int64_t items = static_cast<int64_t>(split_a[gridDim.x]) + split_b[gridDim.x];
     // The tile's pairs, or those of a chunk's written tiles, `tickets` of the chunk's (one
     // thread).
     auto total = [&](unsigned pairs, int tickets) {
         if (pairs) atomicAdd(&chunk_pairs[c * kChunkStride], pairs);
         const int64_t all = SPARSE ? ticket_total(pairs, tickets, c, gridDim.x, done)
                                    : dev::two_level_total(pairs, done);
-        if (all >= 0) dev::store_system(length_out, intersect ? all : items - all);
+        if (all >= 0) {  // (the last one; an operand's arrays may be longer than its offsets say)
+            const int64_t items = static_cast<int64_t>(split_a[gridDim.x]) + split_b[gridDim.x];
+            dev::store_system(length_out, intersect ? all : items - all);
+        }
     };
     if (SPARSE) {
         if (t % kChunk == 0) {  // uniform: the chunk's tiles whose order is written
@@ -1345,7 +1346,7 @@ int merge_level(Call &call, bool intersect, bool values, bool child, int rows, i
     if (num_tiles <= kFusedTiles) {
         // (one tile takes no ticket)
         const unsigned tickets = num_tiles > 1 ? num_tiles : 0;
-        NACHO_TRY(call.sync_block(kSyncBytes, tickets, Z.dot ? tickets : 0, &sync));
+        NACHO_TRY(call.sync_block(kSyncBytes, tickets, Z.dot ? tickets : 0, Z.dot != nullptr, &sync));
     }
     // A small inner product, which the host never waits for, may be recorded: each replay clears
     // the words first.  They come with the partial sums, so that a recorded call allocates what

@@ -455,17 +455,20 @@ int Call::result(size_t bytes, void **out) {
     return NACHO_OK;
 }
 
-int Call::sync_block(size_t bytes, unsigned tickets, unsigned finishes, SyncBlock *out) {
+int Call::sync_block(size_t bytes, unsigned tickets, unsigned finishes, bool recordable,
+                     SyncBlock *out) {
     *out = SyncBlock{};
     if (arena_ || alloc_) return NACHO_OK;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream_, &capture) != hipSuccess) {
-        (void)hipGetLastError();
-        return NACHO_OK;
-    }
-    if (capture != hipStreamCaptureStatusNone) {
-        out->recorded = true;
-        return NACHO_OK;
+    if (recordable) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream_, &capture) != hipSuccess) {
+            (void)hipGetLastError();
+            return NACHO_OK;
+        }
+        if (capture != hipStreamCaptureStatusNone) {
+            out->recorded = true;
+            return NACHO_OK;
+        }
     }
     if (!sync_) NACHO_TRY(take_sync_block(bytes, stream_, &sync_));
     if (!sync_ || sync_->bytes < bytes) return NACHO_OK;

@@ -90,11 +90,13 @@ class Call {
     // A sync block of at least `bytes` whose counters this call's next launch advances by
     // `tickets` and `finishes`; kept for this stream's later calls.  words stays null where there
     // is none to take (an arena call, a caller's allocator, which the library keeps no memory of,
-    // or a stream that is being captured).
+    // or, for a `recordable` call, one whose host waits for no length, a stream that is being
+    // captured: other calls fail there, and their block with them).
     // The block is dropped when the call ends unless its last use is known to have counted: the
     // launch's length was read (wait_length), or, where the host waits for none, sync_launched
     // said that the launch was made.
-    int sync_block(size_t bytes, unsigned tickets, unsigned finishes, SyncBlock *out);
+    int sync_block(size_t bytes, unsigned tickets, unsigned finishes, bool recordable,
+                   SyncBlock *out);
     void sync_launched() { sync_sound_ = true; }
 
     // Release one result buffer early (e.g. an over-allocated array that turned out empty).
