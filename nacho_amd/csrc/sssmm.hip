@@ -459,8 +459,8 @@ __global__ __launch_bounds__(kBlock) void probe_kernel(
             const unsigned long long hits = __ballot(found);
             if (hits == 0) continue;  // uniform in the wavefront
             // the lanes of one entry are neighbours: its sum forms in its first lane's slot
-            const unsigned long long first = __ballot(
-                l == 0 || ent[g] != __shfl_up(ent[g], 1, dev::kWave));
+            const int prev = __shfl_up(ent[g], 1, dev::kWave);  // (every lane takes part)
+            const unsigned long long first = __ballot(l == 0 || ent[g] != prev);
             const unsigned long long upto = first & (~0ull >> (63 - l));
             const int lead = 63 - __clzll(static_cast<long long>(upto));
             double *sum = s_acc + (threadIdx.x - l);  // the wavefront's slots

@@ -110,14 +110,16 @@ def test_sssmm_entries_per_chunk(gpu, probes):
                 oracle.port_sssmm(n, 100, a, b, c), f"{probes} probes")
 
 
-@pytest.mark.parametrize("half", [0, 1, 2, 7, 8, 12, 40])
+@pytest.mark.parametrize("half", [0, 1, 2, 7, 8, 12, 40, "ragged"])
 @pytest.mark.parametrize("shuffled", [False, True])
 def test_sssmm_bands(gpu, half, shuffled):
-    """Bands: lists of 2 half + 1 entries, nearly every probe hits, several lanes of a wavefront on
-    one mask entry; and the same with every third mask entry elsewhere (misses among the hits)."""
-    rng = np.random.default_rng(half)
+    """Bands: lists of 2 half + 1 entries (ragged: 1 to 15), nearly every probe hits, several lanes
+    of a wavefront on one mask entry, whose entries change at any lane; and the same with every
+    third mask entry elsewhere (misses among the hits)."""
+    rng = np.random.default_rng(7 if half == "ragged" else half)
     n = 3000
-    rows = [list(range(max(0, i - half), min(n, i + half + 1))) for i in range(n)]
+    halves = rng.integers(0, 8, n) if half == "ragged" else [half] * n
+    rows = [list(range(max(0, i - h), min(n, i + h + 1))) for i, h in enumerate(halves)]
     a, b = (csr_from_rows(n, n, rows, rng.uniform(-1, 1, sum(map(len, rows))).astype(np.float32))
             for _ in range(2))
     mask = rows
